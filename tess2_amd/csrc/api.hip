@@ -15,6 +15,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 using namespace t2;
@@ -61,7 +62,9 @@ struct DevBlock {
     int *v2t = nullptr;
     float4 *cc = nullptr;
     int *order = nullptr;                    // cells in Morton order
-    std::vector<int> tet_new;                // caller's tet id -> device tet id
+    bool laid = false;                       // cells and tets in Morton order (launch_layout)
+    int *tet_new = nullptr;                  // caller's tet id -> device tet id, when laid
+    StageBox box{};                          // bounding box of the particles
     float *vol = nullptr;
     bool vol_valid = false;                  // the last run wrote vol
     int *status = nullptr, *npts = nullptr;
@@ -155,6 +158,12 @@ struct tess2_ctx {
     unsigned long long ggen = 0;     // generation the graph was captured at
     bool in_capture = false;
     BlockStats *d_stats = nullptr, *h_stats = nullptr;   // per-block counters, device / pinned
+    int h_stats_cap = 0;
+    StageInfo *d_info = nullptr, *h_info = nullptr;      // one block's staging checks
+    // device buffers given back by earlier stagings, for the next one to use
+    std::unordered_map<void *, size_t> live;             // bytes of every buffer in use
+    std::vector<std::pair<void *, size_t>> spare;        // oldest first
+    size_t spare_bytes = 0;
     double *d_gpart = nullptr;                           // partial grid sums, 1024 per block
     // exact assignment over several blocks: every particle's home key
     // (rank << 23 | cell), and the per-rank npts / deposit-status tables
@@ -193,34 +202,6 @@ static void drop_graph(tess2_ctx *c)
     c->ggen = 0;
 }
 
-static void free_multi(tess2_ctx *c)
-{
-    void *ps[] = {c->d_ins, c->d_gps, c->d_outs, c->d_router, c->d_chunks, c->d_queue,
-                  c->d_stats, c->d_gpart, c->d_npts_tab, c->d_stex_tab, c->d_rmap, c->d_rcand,
-                  c->d_items};
-    c->d_items = nullptr;
-    c->nitems = 0;
-    c->d_rmap = nullptr;
-    c->d_rcand = nullptr;
-    c->rmap_cap = c->rcand_cap = 0;
-    c->d_npts_tab = nullptr;
-    c->d_stex_tab = nullptr;
-    c->homes_ok = false;
-    for (void *p : ps)
-        if (p) (void)hipFree(p);
-    if (c->h_stats) (void)hipHostFree(c->h_stats);
-    c->d_stats = nullptr;
-    c->h_stats = nullptr;
-    c->d_gpart = nullptr;
-    c->d_ins = nullptr;
-    c->d_gps = nullptr;
-    c->d_outs = nullptr;
-    c->d_router = nullptr;
-    c->d_chunks = nullptr;
-    c->d_queue = nullptr;
-    c->nchunks = 0;
-}
-
 static int fail(tess2_ctx *c, int code, const char *fmt, ...)
 {
     char buf[512];
@@ -239,34 +220,133 @@ static int fail(tess2_ctx *c, int code, const char *fmt, ...)
             return fail((c), TESS2_E_HIP, "%s failed: %s", #x, hipGetErrorString(e_)); \
     } while (0)
 
+// Buffers that a staging gives back stay with the context for its next calls,
+// up to SPARE_BYTES (the oldest are freed first): a one-call entry point on a
+// block of some thousand particles would otherwise spend its time in about 30
+// hipMalloc / hipFree pairs (10k particles, ghost test: 2.8 ms a call with
+// them).  A buffer is only used again by work of the context's own
+// stream, or after a wait for it, so that earlier kernels are done with it.
+static constexpr size_t SPARE_BYTES = 256ull << 20;
+
+static void drop_spare(tess2_ctx *c)
+{
+    for (auto &q : c->spare) (void)hipFree(q.first);
+    c->spare.clear();
+    c->spare_bytes = 0;
+}
+
+template <class T>
+static void dfree(tess2_ctx *c, T *&p)
+{
+    if (!p) return;
+    void *q = p;
+    p = nullptr;
+    const auto it = c->live.find(q);
+    const size_t bytes = it == c->live.end() ? SPARE_BYTES + 1 : it->second;
+    if (it != c->live.end()) c->live.erase(it);
+    if (bytes > SPARE_BYTES) {
+        (void)hipFree(q);
+        return;
+    }
+    c->spare.emplace_back(q, bytes);
+    c->spare_bytes += bytes;
+    size_t k = 0;
+    while (c->spare_bytes > SPARE_BYTES) {
+        (void)hipFree(c->spare[k].first);
+        c->spare_bytes -= c->spare[k++].second;
+    }
+    c->spare.erase(c->spare.begin(), c->spare.begin() + (long)k);
+}
+
 template <class T>
 static int dalloc(tess2_ctx *c, T **p, size_t n)
 {
-    if (*p) {
-        (void)hipFree(*p);
-        *p = nullptr;
-    }
+    dfree(c, *p);
     if (n == 0) n = 1;
-    if (c) c->gen++;   // any captured graph refers to the old buffers
-    hipError_t e = hipMalloc((void **)p, n * sizeof(T));
+    c->gen++;   // any captured graph refers to the old buffers
+    // sizes in steps of an eighth of their power of two, so that calls of
+    // similar size find each other's buffers
+    size_t bytes = std::max<size_t>(n * sizeof(T), 256), step = 32;
+    while (step * 16 <= bytes) step *= 2;
+    bytes = (bytes + step - 1) / step * step;
+    size_t best = c->spare.size();
+    for (size_t k = 0; k < c->spare.size(); ++k)
+        if (c->spare[k].second >= bytes && c->spare[k].second <= 2 * bytes &&
+            (best == c->spare.size() || c->spare[k].second < c->spare[best].second))
+            best = k;
+    if (best < c->spare.size()) {
+        *p = static_cast<T *>(c->spare[best].first);
+        c->live[*p] = c->spare[best].second;
+        c->spare_bytes -= c->spare[best].second;
+        c->spare.erase(c->spare.begin() + (long)best);
+        return 0;
+    }
+    hipError_t e = hipMalloc((void **)p, bytes);
+    if (e != hipSuccess && !c->spare.empty()) {
+        (void)hipGetLastError();
+        drop_spare(c);
+        e = hipMalloc((void **)p, bytes);
+    }
     if (e != hipSuccess) {
         *p = nullptr;
-        return fail(c, TESS2_E_NOMEM, "hipMalloc(%zu bytes): %s", n * sizeof(T),
-                    hipGetErrorString(e));
+        (void)hipGetLastError();
+        return fail(c, TESS2_E_NOMEM, "hipMalloc(%zu bytes): %s", bytes, hipGetErrorString(e));
     }
+    c->live[*p] = bytes;
     return 0;
 }
 
-static void free_block(DevBlock &b)
+static void free_block(tess2_ctx *c, DevBlock &b)
 {
-    void *ps[] = {b.order,  b.pts,    b.tets,   b.v2t,   b.cc,   b.vol,  b.status,    b.npts,
-                  b.density, b.count, b.first, b.second, b.head, b.ovf,  b.slow,
-                  b.owner, b.status_ex, b.exflags, b.hstart, b.hfill,
-                  b.hsums,  b.hbk,    b.hsorted, b.hkey, b.defq, b.seg, b.fold[0], b.fold[1],
-                  b.fold[2]};
-    for (void *p : ps)
-        if (p) (void)hipFree(p);
+    dfree(c, b.pts);
+    dfree(c, b.tets);
+    dfree(c, b.v2t);
+    dfree(c, b.cc);
+    dfree(c, b.order);
+    dfree(c, b.tet_new);
+    dfree(c, b.vol);
+    dfree(c, b.status);
+    dfree(c, b.npts);
+    dfree(c, b.density);
+    dfree(c, b.count);
+    dfree(c, b.first);
+    dfree(c, b.second);
+    dfree(c, b.head);
+    dfree(c, b.ovf);
+    dfree(c, b.seg);
+    for (int k = 0; k < 3; ++k) dfree(c, b.fold[k]);
+    dfree(c, b.slow);
+    dfree(c, b.owner);
+    dfree(c, b.status_ex);
+    dfree(c, b.exflags);
+    dfree(c, b.hstart);
+    dfree(c, b.hfill);
+    dfree(c, b.hsums);
+    dfree(c, b.hbk);
+    dfree(c, b.hsorted);
+    dfree(c, b.hkey);
+    dfree(c, b.defq);
     b = DevBlock();
+}
+
+static void free_multi(tess2_ctx *c)
+{
+    dfree(c, c->d_ins);
+    dfree(c, c->d_gps);
+    dfree(c, c->d_outs);
+    dfree(c, c->d_router);
+    dfree(c, c->d_rmap);
+    dfree(c, c->d_rcand);
+    dfree(c, c->d_chunks);
+    dfree(c, c->d_items);
+    dfree(c, c->d_queue);
+    dfree(c, c->d_stats);
+    dfree(c, c->d_gpart);
+    dfree(c, c->d_npts_tab);
+    dfree(c, c->d_stex_tab);
+    c->rmap_cap = c->rcand_cap = 0;
+    c->nchunks = c->nitems = 0;
+    c->homes_ok = false;
 }
 
 // ---------------------------------------------------------------------------
@@ -356,8 +436,12 @@ extern "C" int tess2_destroy(tess2_ctx *c)
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     drop_graph(c);
-    for (auto &b : c->blocks) free_block(b);
+    for (auto &b : c->blocks) free_block(c, b);
     free_multi(c);
+    dfree(c, c->d_info);
+    drop_spare(c);
+    if (c->h_stats) (void)hipHostFree(c->h_stats);
+    if (c->h_info) (void)hipHostFree(c->h_info);
     if (c->ev_run0) (void)hipEventDestroy(c->ev_run0);
     if (c->ev_run1) (void)hipEventDestroy(c->ev_run1);
     if (c->ev_k0) (void)hipEventDestroy(c->ev_k0);
@@ -375,80 +459,20 @@ extern "C" const char *tess2_last_error(const tess2_ctx *c)
 // ---------------------------------------------------------------------------
 // staging
 // ---------------------------------------------------------------------------
-static inline uint32_t spread3(uint32_t x)
-{
-    x &= 0x3ffu;
-    x = (x | (x << 16)) & 0x030000FFu;
-    x = (x | (x << 8)) & 0x0300F00Fu;
-    x = (x | (x << 4)) & 0x030C30C3u;
-    x = (x | (x << 2)) & 0x09249249u;
-    return x;
-}
-
-// Morton ranks of all particles, the original cells in Morton order, and the
-// tets renumbered by the smallest Morton rank among their vertices.
-static void morton_layout(const tess2_block_t &hb, std::vector<int> &rank,
-                          std::vector<int> &order, std::vector<int> &tnew,
-                          std::vector<tess2_tet_t> &tl, std::vector<int> &v2t)
-{
-    const int np = hb.num_particles, nt = hb.num_tets;
-    float lo[3] = {0, 0, 0}, hi[3] = {1, 1, 1};
-    for (int p = 0; p < np; ++p)
-        for (int i = 0; i < 3; ++i) {
-            const float x = hb.particles[3 * p + i];
-            if (p == 0 || x < lo[i]) lo[i] = x;
-            if (p == 0 || x > hi[i]) hi[i] = x;
-        }
-    std::vector<uint64_t> key(np);
-    for (int p = 0; p < np; ++p) {
-        uint32_t q[3];
-        for (int i = 0; i < 3; ++i) {
-            const double ext = (double)hi[i] - lo[i];
-            double f = ext > 0 ? ((double)hb.particles[3 * p + i] - lo[i]) / ext : 0.0;
-            q[i] = (uint32_t)std::min(1023.0, std::max(0.0, f * 1023.0));
-        }
-        const uint32_t code = spread3(q[0]) | (spread3(q[1]) << 1) | (spread3(q[2]) << 2);
-        key[p] = ((uint64_t)code << 32) | (uint32_t)p;
-    }
-    std::sort(key.begin(), key.end());
-    rank.assign(np, 0);
-    order.clear();
-    order.reserve(hb.num_orig_particles);
-    for (int k = 0; k < np; ++k) {
-        const int p = (int)(key[k] & 0xffffffffu);
-        rank[p] = k;
-        if (p < hb.num_orig_particles) order.push_back(p);
-    }
-    std::vector<uint64_t> tk(nt);
-    for (int t = 0; t < nt; ++t) {
-        int m = rank[hb.tets[t].verts[0]];
-        for (int i = 1; i < 4; ++i) m = std::min(m, rank[hb.tets[t].verts[i]]);
-        tk[t] = ((uint64_t)(uint32_t)m << 32) | (uint32_t)t;
-    }
-    std::sort(tk.begin(), tk.end());
-    tnew.assign(nt, 0);
-    for (int k = 0; k < nt; ++k) tnew[(int)(tk[k] & 0xffffffffu)] = k;
-    tl.resize(nt);
-    for (int k = 0; k < nt; ++k) {
-        const tess2_tet_t &q = hb.tets[(int)(tk[k] & 0xffffffffu)];
-        tess2_tet_t &o = tl[k];
-        for (int i = 0; i < 4; ++i) {
-            o.verts[i] = q.verts[i];
-            o.tets[i] = q.tets[i] < 0 ? q.tets[i] : tnew[q.tets[i]];
-        }
-    }
-    v2t.resize(np);
-    for (int p = 0; p < np; ++p)
-        v2t[p] = hb.vert_to_tet[p] < 0 ? hb.vert_to_tet[p] : tnew[hb.vert_to_tet[p]];
-}
-
-static int validate(tess2_ctx *c, const tess2_block_t &b)
+// the arguments that can be checked without reading the arrays
+static int validate_args(tess2_ctx *c, const tess2_block_t &b)
 {
     if (b.num_orig_particles < 0 || b.num_particles < b.num_orig_particles || b.num_tets < 0)
         return fail(c, TESS2_E_ARG, "block %d: bad counts", b.gid);
-    if ((b.num_particles && !b.particles) || (b.num_tets && !b.tets) ||
-        (b.num_particles && !b.vert_to_tet))
+    if ((b.num_particles && !b.particles) || (b.num_tets && !b.tets))
         return fail(c, TESS2_E_ARG, "block %d: null array", b.gid);
+    return 0;
+}
+
+// The index ranges on the host: names the first entry out of range, once the
+// device check (launch_stage_check) has found that there is one.
+static int validate_ranges(tess2_ctx *c, const tess2_block_t &b)
+{
     const int np = b.num_particles, nt = b.num_tets;
     for (int t = 0; t < nt; ++t) {
         const tess2_tet_t &q = b.tets[t];
@@ -461,10 +485,56 @@ static int validate(tess2_ctx *c, const tess2_block_t &b)
                             t, q.tets[i]);
         }
     }
-    for (int p = 0; p < np; ++p)
-        if (b.vert_to_tet[p] < -1 || b.vert_to_tet[p] >= nt)
-            return fail(c, TESS2_E_ARG, "block %d: vert_to_tet[%d] out of range", b.gid, p);
+    if (b.vert_to_tet)
+        for (int p = 0; p < np; ++p)
+            if (b.vert_to_tet[p] < -1 || b.vert_to_tet[p] >= nt)
+                return fail(c, TESS2_E_ARG, "block %d: vert_to_tet[%d] out of range", b.gid, p);
     return 0;
+}
+
+static float ord2f(unsigned u)
+{
+    u = (u & 0x80000000u) ? (u & 0x7fffffffu) : ~u;
+    float x;
+    memcpy(&x, &u, sizeof x);
+    return x;
+}
+
+// the block's cells and tets in Morton order: buffers in the new numbering
+// replace those in the caller's
+static int lay_out(tess2_ctx *c, DevBlock &d)
+{
+    int r = 0;
+    int4 *tets = nullptr;
+    int *v2t = nullptr;
+    unsigned *work = nullptr;
+    if ((r = dalloc(c, &tets, 2 * (size_t)d.nt)) || (r = dalloc(c, &v2t, (size_t)d.np)) ||
+        (r = dalloc(c, &work, layout_scratch_words(d.np, d.nt))) ||
+        (r = dalloc(c, &d.order, (size_t)d.norig)) ||
+        (r = dalloc(c, &d.tet_new, (size_t)d.nt))) {
+        dfree(c, tets);
+        dfree(c, v2t);
+        dfree(c, work);
+        return r;
+    }
+    launch_layout(d.pts, d.np, d.norig, d.box, d.tets, d.nt, d.v2t, work, d.order, tets, v2t,
+                  d.tet_new, c->stream);
+    dfree(c, work);
+    std::swap(d.tets, tets);
+    std::swap(d.v2t, v2t);
+    dfree(c, tets);
+    dfree(c, v2t);
+    HIPCHK(c, hipGetLastError());
+    d.laid = true;
+    return 0;
+}
+
+// host -> device on the context's stream, done when it returns: a buffer from
+// the spare list may still be read by earlier work of that stream
+static hipError_t upload(tess2_ctx *c, void *dst, const void *src, size_t bytes)
+{
+    const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream);
+    return e == hipSuccess ? hipStreamSynchronize(c->stream) : e;
 }
 
 // Work list of the batched launch: each block's cells (in its Morton order)
@@ -504,8 +574,7 @@ static int build_chunks(tess2_ctx *c)
     int r = dalloc(c, &c->d_chunks, std::max<size_t>(ch.size(), 1));
     if (r) return r;
     if (!ch.empty())
-        HIPCHK(c, hipMemcpy(c->d_chunks, ch.data(), sizeof(Chunk) * ch.size(),
-                            hipMemcpyHostToDevice));
+        HIPCHK(c, upload(c, c->d_chunks, ch.data(), sizeof(Chunk) * ch.size()));
     // the item list of the queue-free launches: two cells at a time
     std::vector<Chunk> it;
     for (int b = 0; b < (int)c->blocks.size(); ++b)
@@ -514,8 +583,7 @@ static int build_chunks(tess2_ctx *c)
     c->nitems = (int)it.size();
     if ((r = dalloc(c, &c->d_items, std::max<size_t>(it.size(), 1)))) return r;
     if (!it.empty())
-        HIPCHK(c, hipMemcpy(c->d_items, it.data(), sizeof(Chunk) * it.size(),
-                            hipMemcpyHostToDevice));
+        HIPCHK(c, upload(c, c->d_items, it.data(), sizeof(Chunk) * it.size()));
     return 0;
 }
 
@@ -561,8 +629,7 @@ static int build_home_keys(tess2_ctx *c)
         int rr = 0;
         if ((rr = dalloc(c, &d.hkey, (size_t)d.np))) return rr;
         if (d.np)
-            HIPCHK(c, hipMemcpy(d.hkey, key.data(), sizeof(int) * (size_t)d.np,
-                                hipMemcpyHostToDevice));
+            HIPCHK(c, upload(c, d.hkey, key.data(), sizeof(int) * (size_t)d.np));
     }
     std::vector<int *> tn(nb), ts(nb);
     for (int k = 0; k < nb; ++k) {
@@ -572,19 +639,121 @@ static int build_home_keys(tess2_ctx *c)
     int rr = 0;
     if ((rr = dalloc(c, &c->d_npts_tab, (size_t)nb)) || (rr = dalloc(c, &c->d_stex_tab, (size_t)nb)))
         return rr;
-    HIPCHK(c, hipMemcpy(c->d_npts_tab, tn.data(), sizeof(int *) * nb, hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemcpy(c->d_stex_tab, ts.data(), sizeof(int *) * nb, hipMemcpyHostToDevice));
+    HIPCHK(c, upload(c, c->d_npts_tab, tn.data(), sizeof(int *) * nb));
+    HIPCHK(c, upload(c, c->d_stex_tab, ts.data(), sizeof(int *) * nb));
     c->homes_ok = true;
     return 0;
 }
 
-extern "C" int tess2_stage(tess2_ctx *c, const tess2_block_t *blocks, int nblocks)
+// One block into device memory: its arrays as they are, one pass that checks
+// and packs them, then (layout) the Morton order.  Waits for the check.
+static int stage_block(tess2_ctx *c, const tess2_block_t &hb, DevBlock &d, bool layout)
+{
+    hipStream_t s = c->stream;
+    d.gid = hb.gid;
+    d.norig = hb.num_orig_particles;
+    d.np = hb.num_particles;
+    d.nt = hb.num_tets;
+    if (hb.ghost_gid && hb.ghost_cell && d.np > d.norig) {
+        d.ghost_gid.assign(hb.ghost_gid, hb.ghost_gid + (d.np - d.norig));
+        d.ghost_cell.assign(hb.ghost_cell, hb.ghost_cell + (d.np - d.norig));
+    }
+    for (int i = 0; i < 3; ++i) {
+        d.bmin[i] = hb.bounds_min[i];
+        d.bmax[i] = hb.bounds_max[i];
+    }
+    int r = 0;
+    float *xyz = nullptr;
+    if ((r = dalloc(c, &d.pts, (size_t)d.np)) || (r = dalloc(c, &d.tets, 2 * (size_t)d.nt)) ||
+        (r = dalloc(c, &d.v2t, (size_t)d.np)) || (r = dalloc(c, &d.cc, (size_t)d.nt)) ||
+        (r = dalloc(c, &d.vol, (size_t)d.norig)) || (r = dalloc(c, &d.status, (size_t)d.norig)) ||
+        (r = dalloc(c, &d.npts, (size_t)d.norig)) || (r = dalloc(c, &xyz, 3 * (size_t)d.np)))
+        return r;
+    hipError_t e = hipSuccess;
+    if (d.np) e = hipMemcpyAsync(xyz, hb.particles, 12 * (size_t)d.np, hipMemcpyHostToDevice, s);
+    if (e == hipSuccess && d.nt)
+        e = hipMemcpyAsync(d.tets, hb.tets, sizeof(tess2_tet_t) * (size_t)d.nt,
+                           hipMemcpyHostToDevice, s);
+    if (e == hipSuccess && d.np && hb.vert_to_tet)
+        e = hipMemcpyAsync(d.v2t, hb.vert_to_tet, sizeof(int) * (size_t)d.np,
+                           hipMemcpyHostToDevice, s);
+    if (e == hipSuccess) {
+        if (!hb.vert_to_tet) launch_fill_u32((unsigned *)d.v2t, (size_t)d.np, 0xffffffffu, s);
+        launch_stage_check(xyz, d.np, d.tets, d.nt, d.v2t, d.pts, c->d_info, s);
+        e = hipMemcpyAsync(c->h_info, c->d_info, sizeof(StageInfo), hipMemcpyDeviceToHost, s);
+    }
+    // the caller's arrays are read until here
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    dfree(c, xyz);
+    if (e != hipSuccess)
+        return fail(c, TESS2_E_HIP, "block %d: upload: %s", d.gid, hipGetErrorString(e));
+    if (c->h_info->err) {
+        r = validate_ranges(c, hb);
+        return r ? r : fail(c, TESS2_E_INTERNAL, "block %d: the device's range check failed", d.gid);
+    }
+    float lo[3] = {0, 0, 0}, hi[3] = {1, 1, 1};
+    if (d.np && !c->h_info->nonfinite)
+        for (int i = 0; i < 3; ++i) {
+            lo[i] = ord2f(c->h_info->lo[i]);
+            hi[i] = ord2f(c->h_info->hi[i]);
+        }
+    else   // infinities and NaN: comparisons in particle order
+        for (int p = 0; p < d.np; ++p)
+            for (int i = 0; i < 3; ++i) {
+                const float x = hb.particles[3 * p + i];
+                if (p == 0 || x < lo[i]) lo[i] = x;
+                if (p == 0 || x > hi[i]) hi[i] = x;
+            }
+    for (int i = 0; i < 3; ++i) {
+        d.box.lo[i] = lo[i];
+        d.box.hi[i] = hi[i];
+    }
+    // HBM layout: cells visited in Morton order of their sites; tets
+    // renumbered by the Morton rank of their first-ranked vertex so that
+    // the stars of cells processed together are close in memory.  The
+    // results do not depend on either order (the star traversal follows
+    // neighbour slots, not tet ids).
+    if (layout && (r = lay_out(c, d))) return r;
+    d.slow_cap = (unsigned)std::max(1024, d.norig / 32);
+    if ((r = dalloc(c, &d.slow, d.slow_cap))) return r;
+    // bucket hash over the particle bounding box, about two particles
+    // per bucket; at most 2^24 - 1024 buckets, so that the bucket scan
+    // needs at most 16384 blocks of 1024 (k_scan_sums' limit)
+    double vol = 1.0;
+    for (int i = 0; i < 3; ++i) vol *= std::max((double)hi[i] - lo[i], 1e-12);
+    double cell = std::cbrt(vol * 2.0 / std::max(d.np, 1));
+    for (;;) {
+        long long nb = 1;
+        for (int i = 0; i < 3; ++i)
+            nb *= (long long)((hi[i] - lo[i]) / cell) + 1;
+        if (nb <= (1ll << 24) - 1024) break;
+        cell *= 1.25;
+    }
+    d.hash.cell = (float)cell;
+    d.hash.inv = (float)(1.0 / cell);
+    for (int i = 0; i < 3; ++i) {
+        d.hash.lo[i] = lo[i];
+        d.hash.dims[i] = (int)((hi[i] - lo[i]) / cell) + 1;
+    }
+    const size_t nbk = (size_t)d.hash.dims[0] * d.hash.dims[1] * d.hash.dims[2];
+    if ((r = dalloc(c, &d.hstart, nbk + 1)) || (r = dalloc(c, &d.hfill, nbk + 1)) ||
+        (r = dalloc(c, &d.hsums, (nbk + 1 + 1023) / 1024)) ||
+        (r = dalloc(c, &d.hbk, (size_t)d.np)) || (r = dalloc(c, &d.hsorted, (size_t)d.np)) ||
+        (r = dalloc(c, &d.status_ex, (size_t)d.norig)) ||
+        (r = dalloc(c, &d.exflags, ((size_t)d.norig * 3 + 3) / 4)))
+        return r;
+    return 0;
+}
+
+// layout: the caller's next run reads the tets (else the order is made by the
+// first run that does, prepare_run)
+static int stage_blocks(tess2_ctx *c, const tess2_block_t *blocks, int nblocks, bool layout)
 {
     if (!c || (nblocks > 0 && !blocks) || nblocks < 0) return fail(c, TESS2_E_ARG, "bad args");
     HIPCHK(c, hipSetDevice(c->device));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     for (int i = 0; i < nblocks; ++i) {
-        int r = validate(c, blocks[i]);
+        int r = validate_args(c, blocks[i]);
         if (r) return r;
     }
     // deposit keys: cell << 1 | z bit for own cells; 1 << 31 | rank << 24 |
@@ -601,95 +770,46 @@ extern "C" int tess2_stage(tess2_ctx *c, const tess2_block_t *blocks, int nblock
                 return fail(c, TESS2_E_ARG, "blocks must be given in ascending gid order");
         }
     }
-    drop_graph(c);
-    c->gen++;
-    for (auto &b : c->blocks) free_block(b);
-    free_multi(c);
-    c->blocks.assign(nblocks, DevBlock());
-    c->have_run = false;
-    std::vector<float4> tmp;
-    for (int k = 0; k < nblocks; ++k) {
-        const tess2_block_t &hb = blocks[k];
-        DevBlock &d = c->blocks[k];
-        d.gid = hb.gid;
-        d.norig = hb.num_orig_particles;
-        d.np = hb.num_particles;
-        d.nt = hb.num_tets;
-        if (hb.ghost_gid && hb.ghost_cell && d.np > d.norig) {
-            d.ghost_gid.assign(hb.ghost_gid, hb.ghost_gid + (d.np - d.norig));
-            d.ghost_cell.assign(hb.ghost_cell, hb.ghost_cell + (d.np - d.norig));
-        }
-        for (int i = 0; i < 3; ++i) {
-            d.bmin[i] = hb.bounds_min[i];
-            d.bmax[i] = hb.bounds_max[i];
-        }
-        int r = 0;
-        if ((r = dalloc(c, &d.pts, (size_t)d.np)) || (r = dalloc(c, &d.tets, 2 * (size_t)d.nt)) ||
-            (r = dalloc(c, &d.v2t, (size_t)d.np)) || (r = dalloc(c, &d.cc, (size_t)d.nt)) ||
-            (r = dalloc(c, &d.vol, (size_t)d.norig)) || (r = dalloc(c, &d.status, (size_t)d.norig)) ||
-            (r = dalloc(c, &d.npts, (size_t)d.norig)))
-            return r;
-        tmp.resize(d.np);
-        for (int p = 0; p < d.np; ++p)
-            tmp[p] = make_float4(hb.particles[3 * p], hb.particles[3 * p + 1],
-                                 hb.particles[3 * p + 2], 0.0f);
-        HIPCHK(c, hipMemcpy(d.pts, tmp.data(), sizeof(float4) * d.np, hipMemcpyHostToDevice));
-        // HBM layout: cells visited in Morton order of their sites; tets
-        // renumbered by the Morton rank of their first-ranked vertex so that
-        // the stars of cells processed together are close in memory.  The
-        // results do not depend on either order (the star traversal follows
-        // neighbour slots, not tet ids).
-        std::vector<int> rank, order, tnew;
-        std::vector<tess2_tet_t> tl;
-        std::vector<int> v2t;
-        morton_layout(hb, rank, order, tnew, tl, v2t);
-        d.tet_new.swap(tnew);
-        if ((r = dalloc(c, &d.order, (size_t)d.norig))) return r;
-        if (d.norig)
-            HIPCHK(c, hipMemcpy(d.order, order.data(), sizeof(int) * (size_t)d.norig,
-                                hipMemcpyHostToDevice));
-        HIPCHK(c, hipMemcpy(d.tets, tl.data(), sizeof(tess2_tet_t) * (size_t)d.nt,
-                            hipMemcpyHostToDevice));
-        HIPCHK(c, hipMemcpy(d.v2t, v2t.data(), sizeof(int) * (size_t)d.np,
-                            hipMemcpyHostToDevice));
-        d.slow_cap = (unsigned)std::max(1024, d.norig / 32);
-        if ((r = dalloc(c, &d.slow, d.slow_cap))) return r;
-        // bucket hash over the particle bounding box, about two particles
-        // per bucket; at most 2^24 - 1024 buckets, so that the bucket scan
-        // needs at most 16384 blocks of 1024 (k_scan_sums' limit)
-        float lo[3] = {0, 0, 0}, hi[3] = {1, 1, 1};
-        for (int p = 0; p < d.np; ++p)
-            for (int i = 0; i < 3; ++i) {
-                const float x = hb.particles[3 * p + i];
-                if (p == 0 || x < lo[i]) lo[i] = x;
-                if (p == 0 || x > hi[i]) hi[i] = x;
+    int r = 0;
+    if (!c->d_info && (r = dalloc(c, &c->d_info, 1))) return r;
+    if (!c->h_info &&
+        hipHostMalloc((void **)&c->h_info, sizeof(StageInfo), hipHostMallocDefault) != hipSuccess)
+        return fail(c, TESS2_E_NOMEM, "pinned host buffer");
+    // the new blocks beside the old ones, which stay staged when an input is
+    // refused; without room for both, the inputs are checked on the host
+    // first and the old blocks make room
+    std::vector<DevBlock> fresh(nblocks);
+    auto stage_all = [&]() -> int {
+        for (int k = 0; k < nblocks; ++k) {
+            int rr = stage_block(c, blocks[k], fresh[k], layout);
+            if (rr) {
+                for (auto &b : fresh) free_block(c, b);
+                return rr;
             }
-        double vol = 1.0;
-        for (int i = 0; i < 3; ++i) vol *= std::max((double)hi[i] - lo[i], 1e-12);
-        double cell = std::cbrt(vol * 2.0 / std::max(d.np, 1));
-        for (;;) {
-            long long nb = 1;
-            for (int i = 0; i < 3; ++i)
-                nb *= (long long)((hi[i] - lo[i]) / cell) + 1;
-            if (nb <= (1ll << 24) - 1024) break;
-            cell *= 1.25;
         }
-        d.hash.cell = (float)cell;
-        d.hash.inv = (float)(1.0 / cell);
-        for (int i = 0; i < 3; ++i) {
-            d.hash.lo[i] = lo[i];
-            d.hash.dims[i] = (int)((hi[i] - lo[i]) / cell) + 1;
-        }
-        const size_t nbk = (size_t)d.hash.dims[0] * d.hash.dims[1] * d.hash.dims[2];
-        if ((r = dalloc(c, &d.hstart, nbk + 1)) || (r = dalloc(c, &d.hfill, nbk + 1)) ||
-            (r = dalloc(c, &d.hsums, (nbk + 1 + 1023) / 1024)) ||
-            (r = dalloc(c, &d.hbk, (size_t)d.np)) || (r = dalloc(c, &d.hsorted, (size_t)d.np)) ||
-            (r = dalloc(c, &d.status_ex, (size_t)d.norig)) ||
-            (r = dalloc(c, &d.exflags, ((size_t)d.norig * 3 + 3) / 4)))
-            return r;
+        return 0;
+    };
+    auto drop_old = [&]() {
+        drop_graph(c);
+        c->gen++;
+        for (auto &b : c->blocks) free_block(c, b);
+        c->blocks.clear();
+        free_multi(c);
+        c->have_run = false;
+    };
+    r = stage_all();
+    if (r == TESS2_E_NOMEM && !c->blocks.empty()) {
+        for (int i = 0; i < nblocks; ++i)
+            if ((r = validate_ranges(c, blocks[i]))) return r;
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        drop_old();
+        drop_spare(c);
+        r = stage_all();
     }
+    if (r) return r;
+    drop_old();
+    c->blocks.swap(fresh);
     if (nblocks > 0) {
-        int r = 0;
         if ((r = dalloc(c, &c->d_ins, (size_t)nblocks)) || (r = dalloc(c, &c->d_gps, (size_t)nblocks)) ||
             (r = dalloc(c, &c->d_outs, (size_t)nblocks)) || (r = dalloc(c, &c->d_router, 1)) ||
             (r = dalloc(c, &c->d_queue, 16)) || (r = dalloc(c, &c->d_stats, (size_t)nblocks)) ||
@@ -697,9 +817,15 @@ extern "C" int tess2_stage(tess2_ctx *c, const tess2_block_t *blocks, int nblock
             return r;
         // counters and statistics of all blocks: one device array, one pinned
         // host copy (so that the copy can sit in a captured graph)
-        if (hipHostMalloc((void **)&c->h_stats, sizeof(BlockStats) * nblocks,
-                          hipHostMallocDefault) != hipSuccess)
-            return fail(c, TESS2_E_NOMEM, "pinned host buffer");
+        if (nblocks > c->h_stats_cap) {
+            if (c->h_stats) (void)hipHostFree(c->h_stats);
+            c->h_stats = nullptr;
+            c->h_stats_cap = 0;
+            if (hipHostMalloc((void **)&c->h_stats, sizeof(BlockStats) * nblocks,
+                              hipHostMallocDefault) != hipSuccess)
+                return fail(c, TESS2_E_NOMEM, "pinned host buffer");
+            c->h_stats_cap = nblocks;
+        }
         memset(c->h_stats, 0, sizeof(BlockStats) * nblocks);
         for (int k = 0; k < nblocks; ++k) {
             DevBlock &d = c->blocks[k];
@@ -707,11 +833,19 @@ extern "C" int tess2_stage(tess2_ctx *c, const tess2_block_t *blocks, int nblock
             d.ctrs = d.st->ctrs;
             d.hm = c->h_stats + k;
         }
-        r = build_chunks(c);
-        if (r) return r;
-        if (nblocks > 1 && (r = build_home_keys(c))) return r;
+        // work lists and home keys of multi-block runs
+        if (nblocks > 1 && ((r = build_chunks(c)) || (r = build_home_keys(c)))) return r;
     }
     return 0;
+}
+
+extern "C" int tess2_stage(tess2_ctx *c, const tess2_block_t *blocks, int nblocks)
+{
+    if (c && blocks)
+        for (int i = 0; i < nblocks; ++i)
+            if (blocks[i].num_particles && !blocks[i].vert_to_tet)
+                return fail(c, TESS2_E_ARG, "block %d: null array", blocks[i].gid);
+    return stage_blocks(c, blocks, nblocks, true);
 }
 
 // shared-point list and the fold's segment storage and class lists for
@@ -871,6 +1005,12 @@ static int prepare_run(tess2_ctx *c, const RunArgs &a)
     if (a.gnum[0] < 2 || a.gnum[1] < 2 || a.gnum[2] < 2)
         return fail(c, TESS2_E_ARG, "grid needs at least 2 points per axis");
     if (c->blocks.empty()) return fail(c, TESS2_E_ARG, "no staged blocks");
+    if (a.alg == TESS2_DENSE_TESS)
+        for (DevBlock &d : c->blocks)
+            if (!d.laid) {
+                const int r = lay_out(c, d);
+                if (r) return r;
+            }
     const int nb = (int)c->blocks.size();
     const bool exact = a.alg == TESS2_DENSE_TESS && a.assignment == TESS2_ASSIGN_EXACT_VORONOI;
     if (exact && nb > 1 && !c->homes_ok)
@@ -923,8 +1063,7 @@ static int prepare_run(tess2_ctx *c, const RunArgs &a)
             d.owner_cap = n;
             // a quarter of the grid (beyond it the search runs inline); the
             // queue holds 32-bit grid indices
-            if (d.defq) (void)hipFree(d.defq);
-            d.defq = nullptr;
+            dfree(c, d.defq);
             d.defq_cap = 0;
             if (n < (1ull << 32)) {
                 const size_t cap = n / 4 + 1024;
@@ -1415,14 +1554,16 @@ extern "C" int tess2_fetch(tess2_ctx *c, int b, float *density, float *volumes,
         HIPCHK(c, hipMemcpy(volumes, d.vol, sizeof(float) * d.norig, hipMemcpyDeviceToHost));
     }
     if (circumcenters && d.nt) {
-        std::vector<float4> tmp(d.nt);
-        HIPCHK(c, hipMemcpy(tmp.data(), d.cc, sizeof(float4) * d.nt, hipMemcpyDeviceToHost));
-        for (int t = 0; t < d.nt; ++t) {
-            const float4 q = tmp[d.tet_new[t]];   // caller's numbering
-            circumcenters[3 * t] = q.x;
-            circumcenters[3 * t + 1] = q.y;
-            circumcenters[3 * t + 2] = q.z;
-        }
+        // packed on the device, in the caller's numbering
+        float *tmp = nullptr;
+        const int r = dalloc(c, &tmp, 3 * (size_t)d.nt);
+        if (r) return r;
+        launch_unpack_cc(d.cc, d.laid ? d.tet_new : nullptr, d.nt, tmp, c->stream);
+        hipError_t e = hipMemcpyAsync(circumcenters, tmp, 12 * (size_t)d.nt,
+                                      hipMemcpyDeviceToHost, c->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+        dfree(c, tmp);
+        HIPCHK(c, e);
     }
     return 0;
 }
@@ -1461,15 +1602,14 @@ extern "C" int tess2_fill_circumcenters(tess2_ctx *c, const tess2_tet_t *tets, i
 {
     if (!c || num_tets < 0 || num_particles < 0 || (num_tets && (!tets || !out)))
         return fail(c, TESS2_E_ARG, "bad arguments");
-    std::vector<int> v2t(num_particles, -1);
     tess2_block_t b{};
     b.num_orig_particles = 0;
     b.num_particles = num_particles;
     b.particles = particles;
     b.num_tets = num_tets;
     b.tets = tets;
-    b.vert_to_tet = v2t.data();
-    int r = tess2_stage(c, &b, 1);
+    b.vert_to_tet = nullptr;   // no cell: no particle needs a tet
+    int r = stage_blocks(c, &b, 1, false);   // one pass over the tets in the caller's order
     if (r) return r;
     DevBlock &d = c->blocks[0];
     launch_circumcenters(d.pts, d.tets, d.nt, d.cc, c->stream);
@@ -1595,28 +1735,35 @@ extern "C" int tess2_ghost_sends(tess2_ctx *c, const tess2_block_t *block, int n
     if (!c || !block || num_neighbors < 0 || num_neighbors > 64 || first_neighbor < 0 ||
         (num_neighbors > 0 && !neighbor_boxes) || (block->num_orig_particles > 0 && !sends))
         return fail(c, TESS2_E_ARG, "bad arguments (at most 64 neighbours)");
-    int r = tess2_stage(c, block, 1);
+    if (block->num_particles && !block->vert_to_tet)
+        return fail(c, TESS2_E_ARG, "block %d: null array", block->gid);
+    int r = stage_blocks(c, block, 1, false);   // one pass over the tets in the caller's order
     if (r) return r;
     DevBlock &d = c->blocks[0];
     if (d.norig == 0) return 0;
     float *dbox = nullptr;
     unsigned long long *dsend = nullptr;
-    if ((r = dalloc(c, &dbox, (size_t)std::max(6 * num_neighbors, 1))) ||
-        (r = dalloc(c, &dsend, (size_t)d.norig)))
-        return r;
     hipStream_t s = c->stream;
-    if (num_neighbors > 0)
-        HIPCHK(c, hipMemcpyAsync(dbox, neighbor_boxes, sizeof(float) * 6 * num_neighbors,
-                                 hipMemcpyHostToDevice, s));
-    launch_fill_u32(reinterpret_cast<unsigned *>(dsend), 2 * (size_t)d.norig, 0u, s);
-    launch_ghost_sends(d.pts, d.tets, d.nt, d.norig, d.bmin, d.bmax, dbox, num_neighbors,
-                       first_neighbor, dsend, s);
-    HIPCHK(c, hipGetLastError());
-    HIPCHK(c, hipMemcpyAsync(sends, dsend, sizeof(unsigned long long) * d.norig,
-                             hipMemcpyDeviceToHost, s));
-    HIPCHK(c, hipStreamSynchronize(s));
-    (void)hipFree(dbox);
-    (void)hipFree(dsend);
+    r = dalloc(c, &dbox, (size_t)std::max(6 * num_neighbors, 1));
+    if (!r) r = dalloc(c, &dsend, (size_t)d.norig);
+    hipError_t e = hipSuccess;
+    if (!r && num_neighbors > 0)
+        e = hipMemcpyAsync(dbox, neighbor_boxes, sizeof(float) * 6 * num_neighbors,
+                           hipMemcpyHostToDevice, s);
+    if (!r && e == hipSuccess) {
+        launch_fill_u32(reinterpret_cast<unsigned *>(dsend), 2 * (size_t)d.norig, 0u, s);
+        launch_ghost_sends(d.pts, d.tets, d.nt, d.norig, d.bmin, d.bmax, dbox, num_neighbors,
+                           first_neighbor, dsend, s);
+        e = hipGetLastError();
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(sends, dsend, sizeof(unsigned long long) * d.norig,
+                               hipMemcpyDeviceToHost, s);
+    }
+    if (!r && e == hipSuccess) e = hipStreamSynchronize(s);
+    dfree(c, dbox);
+    dfree(c, dsend);
+    if (r) return r;
+    HIPCHK(c, e);
     return 0;
 }
 
@@ -1629,7 +1776,11 @@ extern "C" int tess2_dense(tess2_ctx *c, int alg, int num_given_bounds, const fl
                            tess2_stats_t *stats)
 {
     if (!c || !blocks || nblocks <= 0 || !density_out) return fail(c, TESS2_E_ARG, "bad args");
-    int r = tess2_stage(c, blocks, nblocks);
+    for (int k = 0; k < nblocks; ++k)
+        if (blocks[k].num_particles && !blocks[k].vert_to_tet)
+            return fail(c, TESS2_E_ARG, "block %d: null array", blocks[k].gid);
+    // CIC reads the particles only
+    int r = stage_blocks(c, blocks, nblocks, alg == TESS2_DENSE_TESS);
     if (r) return r;
     r = tess2_run(c, alg, num_given_bounds, given_mins, given_maxs, project, proj_plane, mass,
                   eps, glo_num_idx, assignment, precision, 0);

@@ -107,6 +107,19 @@ struct Router {
     int rbase[3], rlen[3], roff[3], rn[3];
 };
 
+// what staging checks of a block's arrays (device); lo / hi: the bounding
+// box of the finite particles, as floats in an unsigned order
+struct StageInfo {
+    unsigned err;          // an index out of range
+    unsigned nonfinite;    // a coordinate that is infinite or NaN
+    unsigned lo[3], hi[3];
+};
+
+// the particles' bounding box (the Morton grid)
+struct StageBox {
+    float lo[3], hi[3];
+};
+
 // one chunk of cells of one block for the batched launch
 struct Chunk {
     int block;
@@ -187,6 +200,18 @@ void launch_fill_u32(unsigned *p, size_t n, unsigned v, hipStream_t s);
 void launch_ghost_sends(const float4 *pts, const int4 *tets, int ntets, int norig,
                         const float *bmin, const float *bmax, const float *boxes, int nnb,
                         int first, unsigned long long *sends, hipStream_t s);
+// staging (stage.hip): range checks, bounding box and float4 particles of a
+// block as the caller gave it; then its cells in Morton order and its tets
+// renumbered by their lowest-ranked vertex (raw, v2t_raw: the caller's
+// numbering; scratch: layout_scratch_words(np, nt) words)
+void launch_stage_check(const float *xyz, int np, const int4 *tets, int nt, const int *v2t,
+                        float4 *pts, StageInfo *info, hipStream_t s);
+size_t layout_scratch_words(int np, int nt);
+void launch_layout(const float4 *pts, int np, int norig, const StageBox &box, const int4 *raw,
+                   int nt, const int *v2t_raw, unsigned *scratch, int *order, int4 *tets,
+                   int *v2t, int *tnew, hipStream_t s);
+// circumcenters as xyz triples in the caller's tet numbering
+void launch_unpack_cc(const float4 *cc, const int *tnew, int nt, float *out, hipStream_t s);
 // xyz triples -> float4 (xyz, 0)
 void launch_pack_points(const float *xyz, int np, float4 *pts, hipStream_t s);
 // index-range check of a block in device memory: sets `bit` in *err on a violation

@@ -1,0 +1,478 @@
+// stage.hip -- device side of staging: range checks, bounding box, Morton
+// order of the cells and tets, renumbering.
+//
+// A block arrives as the caller's arrays (one copy each); everything staging
+// does to them is a device pass here.  The order is the one a host sort of
+// (Morton code, particle) and (lowest Morton rank of the vertices, tet)
+// pairs gives: cells in Morton order of their sites, tets renumbered by their
+// lowest-ranked vertex.  Both sorts are stable least-significant-digit radix
+// sorts of (key, id) pairs whose ids start ascending, so that ties stay in id
+// order.
+//
+// What bounds it: a block is read and written a few times (the tets: range
+// check 32 B, keys 16 B + 16 B of gathered ranks, three digit passes of 16 B
+// each way, renumbering 32 B in and out and 16 B of gathered numbers), which
+// takes less than its copy over PCIe (32 B per tet at ~40 GB/s).  Small
+// blocks are bound by the ~30 launches of about 3 us.
+#include "kernels.hpp"
+
+#include <algorithm>
+
+namespace t2 {
+
+namespace {
+
+// floats in an unsigned order (minus zero below plus zero)
+__device__ __forceinline__ unsigned f2ord(float x)
+{
+    const unsigned u = __float_as_uint(x);
+    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
+
+}  // namespace
+
+__global__ void k_stage_init(StageInfo *info)
+{
+    if (threadIdx.x < 3) {
+        info->lo[threadIdx.x] = 0xffffffffu;
+        info->hi[threadIdx.x] = 0u;
+    }
+    if (threadIdx.x == 3) info->err = 0u;
+    if (threadIdx.x == 4) info->nonfinite = 0u;
+}
+
+// One pass over the caller's arrays: xyz triples -> padded float4, the
+// bounding box, and the index ranges (every tet vertex in [0, np), every
+// neighbour and vert_to_tet entry in [-1, nt)).
+__global__ __launch_bounds__(256) void k_stage_check(const float *__restrict__ xyz, int np,
+                                                     const int4 *__restrict__ tets, int nt,
+                                                     const int *__restrict__ v2t,
+                                                     float4 *__restrict__ pts, StageInfo *info)
+{
+    const int stride = (int)(gridDim.x * blockDim.x);
+    const int i0 = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    bool bad = false, odd = false;
+    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+    for (long long p = i0; p < np; p += stride) {
+        const float x = xyz[3 * p], y = xyz[3 * p + 1], z = xyz[3 * p + 2];
+        pts[p] = make_float4(x, y, z, 0.0f);
+        const int t = v2t[p];
+        bad = bad || t < -1 || t >= nt;
+        odd = odd || !(fabsf(x) < INFINITY) || !(fabsf(y) < INFINITY) || !(fabsf(z) < INFINITY);
+        lo[0] = fminf(lo[0], x);
+        lo[1] = fminf(lo[1], y);
+        lo[2] = fminf(lo[2], z);
+        hi[0] = fmaxf(hi[0], x);
+        hi[1] = fmaxf(hi[1], y);
+        hi[2] = fmaxf(hi[2], z);
+    }
+    for (long long t = i0; t < nt; t += stride) {
+        const int4 v = tets[2 * t], n = tets[2 * t + 1];
+        bad = bad || (unsigned)v.x >= (unsigned)np || (unsigned)v.y >= (unsigned)np ||
+              (unsigned)v.z >= (unsigned)np || (unsigned)v.w >= (unsigned)np ||
+              n.x < -1 || n.x >= nt || n.y < -1 || n.y >= nt || n.z < -1 || n.z >= nt ||
+              n.w < -1 || n.w >= nt;
+    }
+    for (int off = 32; off >= 1; off >>= 1)
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            lo[a] = fminf(lo[a], __shfl_xor(lo[a], off));
+            hi[a] = fmaxf(hi[a], __shfl_xor(hi[a], off));
+        }
+    const bool any_bad = __ballot(bad) != 0ull, any_odd = __ballot(odd) != 0ull;
+    if ((threadIdx.x & 63) == 0) {
+        if (any_bad) atomicOr(&info->err, 1u);
+        if (any_odd) atomicOr(&info->nonfinite, 1u);
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+            if (lo[a] <= hi[a]) {
+                atomicMin(&info->lo[a], f2ord(lo[a]));
+                atomicMax(&info->hi[a], f2ord(hi[a]));
+            }
+    }
+}
+
+void launch_stage_check(const float *xyz, int np, const int4 *tets, int nt, const int *v2t,
+                        float4 *pts, StageInfo *info, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_stage_init, dim3(1), dim3(64), 0, s, info);
+    const int n = std::max(np, nt);
+    if (n <= 0) return;
+    // at most 1024 workgroups: the box takes six atomics per wave
+    const int nb = std::min(1024, (n + 255) / 256);
+    hipLaunchKernelGGL(k_stage_check, dim3(nb), dim3(256), 0, s, xyz, np, tets, nt, v2t, pts,
+                       info);
+}
+
+// ---------------------------------------------------------------------------
+// exclusive scan of n unsigned counts, in place
+// ---------------------------------------------------------------------------
+constexpr int SCAN_TILE = 4096;   // 1024 lanes of four
+constexpr int SCAN_MOST = 16;     // entries per lane of the one-workgroup scan
+
+// exclusive prefix of one value per lane over a 1024-lane workgroup, and the
+// total: wave scans by lane exchanges, the 16 wave sums through LDS
+__device__ __forceinline__ unsigned scan_1024(unsigned x, unsigned *s_w, unsigned &total)
+{
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    unsigned incl = x;
+    for (int off = 1; off < 64; off <<= 1) {
+        const unsigned t = __shfl_up(incl, off);
+        if (lane >= off) incl += t;
+    }
+    __syncthreads();   // s_w may hold an earlier call's sums
+    if (lane == 63) s_w[w] = incl;
+    __syncthreads();
+    unsigned base = 0, all = 0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const unsigned v = s_w[i];
+        base += i < w ? v : 0u;
+        all += v;
+    }
+    total = all;
+    return base + incl - x;
+}
+
+__global__ __launch_bounds__(1024) void k_scan_tiles(unsigned *__restrict__ a, unsigned n,
+                                                     unsigned *__restrict__ sums)
+{
+    __shared__ unsigned s_w[16];
+    const unsigned i = blockIdx.x * SCAN_TILE + threadIdx.x * 4;
+    unsigned v[4], run = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        v[k] = i + k < n ? a[i + k] : 0u;
+        const unsigned x = v[k];
+        v[k] = run;
+        run += x;
+    }
+    unsigned total;
+    const unsigned base = scan_1024(run, s_w, total);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        if (i + k < n) a[i + k] = base + v[k];
+    if (threadIdx.x == 0) sums[blockIdx.x] = total;
+}
+
+// one workgroup over n <= 1024 * SCAN_MOST entries
+__global__ __launch_bounds__(1024) void k_scan_one(unsigned *__restrict__ a, unsigned n)
+{
+    __shared__ unsigned s_w[16];
+    const unsigned per = (n + 1023) / 1024;
+    unsigned v[SCAN_MOST], run = 0;
+#pragma unroll
+    for (unsigned k = 0; k < SCAN_MOST; ++k) {
+        const unsigned i = threadIdx.x * per + k;
+        const unsigned x = (k < per && i < n) ? a[i] : 0u;
+        v[k] = run;
+        run += x;
+    }
+    unsigned total;
+    const unsigned base = scan_1024(run, s_w, total);
+#pragma unroll
+    for (unsigned k = 0; k < SCAN_MOST; ++k) {
+        const unsigned i = threadIdx.x * per + k;
+        if (k < per && i < n) a[i] = base + v[k];
+    }
+}
+
+__global__ __launch_bounds__(1024) void k_scan_bases(unsigned *__restrict__ a, unsigned n,
+                                                     const unsigned *__restrict__ sums)
+{
+    const unsigned base = sums[blockIdx.x];
+    const unsigned i = blockIdx.x * SCAN_TILE + threadIdx.x * 4;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        if (i + k < n) a[i + k] += base;
+}
+
+// n up to 1024 * SCAN_MOST in one workgroup, else tiles and their sums (up to
+// 4096 * 16384 = 67 M entries: 256 digits of 262144 sort tiles)
+static void scan_u32(unsigned *a, unsigned n, unsigned *sums, hipStream_t s)
+{
+    if (n == 0) return;
+    if (n <= 1024u * SCAN_MOST) {
+        hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(1024), 0, s, a, n);
+        return;
+    }
+    const unsigned tiles = (n + SCAN_TILE - 1) / SCAN_TILE;
+    hipLaunchKernelGGL(k_scan_tiles, dim3(tiles), dim3(1024), 0, s, a, n, sums);
+    hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(1024), 0, s, sums, tiles);
+    hipLaunchKernelGGL(k_scan_bases, dim3(tiles), dim3(1024), 0, s, a, n,
+                       (const unsigned *)sums);
+}
+
+// ---------------------------------------------------------------------------
+// stable radix sort of (key, id) pairs, 8 bits a pass.  A workgroup of four
+// waves owns a tile of 4096 consecutive pairs, each wave 1024 of them in
+// rounds of 64; hist is digit-major ([digit][tile]), so its exclusive scan
+// gives each tile's first slot per digit.
+// ---------------------------------------------------------------------------
+constexpr int SORT_TILE = 4096, SORT_ROUNDS = SORT_TILE / 256;
+
+__global__ __launch_bounds__(256) void k_sort_hist(const unsigned *__restrict__ key, unsigned n,
+                                                   int shift, unsigned *__restrict__ hist,
+                                                   unsigned ntiles)
+{
+    __shared__ unsigned s_h[256];
+    s_h[threadIdx.x] = 0u;
+    __syncthreads();
+    const unsigned base = blockIdx.x * SORT_TILE;
+#pragma unroll
+    for (int r = 0; r < SORT_ROUNDS; ++r) {
+        const unsigned i = base + r * 256 + threadIdx.x;
+        if (i < n) atomicAdd(&s_h[(key[i] >> shift) & 255u], 1u);
+    }
+    __syncthreads();
+    hist[threadIdx.x * ntiles + blockIdx.x] = s_h[threadIdx.x];
+}
+
+__global__ __launch_bounds__(256) void k_sort_scatter(const unsigned *__restrict__ key,
+                                                      const unsigned *__restrict__ id,
+                                                      unsigned n, int shift,
+                                                      const unsigned *__restrict__ hist,
+                                                      unsigned ntiles,
+                                                      unsigned *__restrict__ key_out,
+                                                      unsigned *__restrict__ id_out)
+{
+    __shared__ unsigned s_c[4][256];   // next slot per wave and digit
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const unsigned long long below = (1ull << lane) - 1ull;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s_c[i][threadIdx.x] = 0u;
+    __syncthreads();
+    const unsigned base = blockIdx.x * SORT_TILE + w * (SORT_TILE / 4) + lane;
+    unsigned k[SORT_ROUNDS];
+#pragma unroll
+    for (int r = 0; r < SORT_ROUNDS; ++r) {
+        const unsigned i = base + r * 64;
+        k[r] = i < n ? key[i] : 0u;
+        if (i < n) atomicAdd(&s_c[w][(k[r] >> shift) & 255u], 1u);
+    }
+    __syncthreads();
+    {
+        unsigned b = hist[threadIdx.x * ntiles + blockIdx.x];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const unsigned c = s_c[i][threadIdx.x];
+            s_c[i][threadIdx.x] = b;
+            b += c;
+        }
+    }
+    __syncthreads();
+    // a wave's rounds in order; within a round, the lanes of one digit take
+    // consecutive slots in lane order (only this wave touches s_c[w])
+#pragma unroll
+    for (int r = 0; r < SORT_ROUNDS; ++r) {
+        const unsigned i = base + r * 64;
+        const bool on = i < n;
+        const unsigned d = (k[r] >> shift) & 255u;
+        unsigned long long same = __ballot(on);
+#pragma unroll
+        for (int b = 0; b < 8; ++b) {
+            const unsigned long long m = __ballot((d >> b) & 1u);
+            same &= ((d >> b) & 1u) ? m : ~m;
+        }
+        if (on) {
+            const unsigned slot = s_c[w][d] + (unsigned)__popcll(same & below);
+            key_out[slot] = k[r];
+            id_out[slot] = id[i];
+        }
+        __builtin_amdgcn_wave_barrier();   // every lane has read its counter
+        if (on && (same & below) == 0ull) s_c[w][d] += (unsigned)__popcll(same);
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// sorts k0 / v0 (n pairs) by the low `bits` bits of the key; the result is in
+// k0 / v0 when an even number of passes ran, else in k1 / v1 (returned)
+static int radix_sort(unsigned *k0, unsigned *v0, unsigned *k1, unsigned *v1, unsigned n,
+                      int bits, unsigned *hist, unsigned *sums, hipStream_t s)
+{
+    const unsigned tiles = (n + SORT_TILE - 1) / SORT_TILE;
+    int which = 0;
+    for (int shift = 0; shift < bits; shift += 8, which ^= 1) {
+        unsigned *ka = which ? k1 : k0, *va = which ? v1 : v0;
+        unsigned *kb = which ? k0 : k1, *vb = which ? v0 : v1;
+        hipLaunchKernelGGL(k_sort_hist, dim3(tiles), dim3(256), 0, s, (const unsigned *)ka, n,
+                           shift, hist, tiles);
+        scan_u32(hist, 256 * tiles, sums, s);
+        hipLaunchKernelGGL(k_sort_scatter, dim3(tiles), dim3(256), 0, s, (const unsigned *)ka,
+                           (const unsigned *)va, n, shift, (const unsigned *)hist, tiles, kb, vb);
+    }
+    return which;
+}
+
+// ---------------------------------------------------------------------------
+// Morton layout
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ unsigned spread3(unsigned x)
+{
+    x &= 0x3ffu;
+    x = (x | (x << 16)) & 0x030000FFu;
+    x = (x | (x << 8)) & 0x0300F00Fu;
+    x = (x | (x << 4)) & 0x030C30C3u;
+    x = (x | (x << 2)) & 0x09249249u;
+    return x;
+}
+
+__global__ void k_morton_keys(const float4 *__restrict__ pts, int np, StageBox box,
+                              unsigned *__restrict__ key, unsigned *__restrict__ id)
+{
+    const int p = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (p >= np) return;
+    const float4 a = pts[p];
+    const float x[3] = {a.x, a.y, a.z};
+    unsigned q[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const double ext = (double)box.hi[i] - (double)box.lo[i];
+        const double f = ext > 0 ? ((double)x[i] - (double)box.lo[i]) / ext : 0.0;
+        double g = f * 1023.0;
+        g = g > 0.0 ? g : 0.0;         // NaN to 0
+        g = g < 1023.0 ? g : 1023.0;
+        q[i] = (unsigned)g;
+    }
+    key[p] = spread3(q[0]) | (spread3(q[1]) << 1) | (spread3(q[2]) << 2);
+    id[p] = (unsigned)p;
+}
+
+// originals (id < norig) per tile of 1024 sorted particles
+__global__ __launch_bounds__(1024) void k_order_count(const unsigned *__restrict__ id, int np,
+                                                      int norig, unsigned *__restrict__ cnt)
+{
+    __shared__ unsigned s_n[16];
+    const int k = (int)(blockIdx.x * 1024 + threadIdx.x);
+    const unsigned long long m = __ballot(k < np && (int)id[k < np ? k : 0] < norig);
+    if ((threadIdx.x & 63) == 0) s_n[threadIdx.x >> 6] = (unsigned)__popcll(m);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned t = 0;
+        for (int i = 0; i < 16; ++i) t += s_n[i];
+        cnt[blockIdx.x] = t;
+    }
+}
+
+// rank of every particle, and the originals in sorted order
+__global__ __launch_bounds__(1024) void k_order_write(const unsigned *__restrict__ id, int np,
+                                                      int norig,
+                                                      const unsigned *__restrict__ cnt,
+                                                      int *__restrict__ rank,
+                                                      int *__restrict__ order)
+{
+    __shared__ unsigned s_n[16];
+    const int k = (int)(blockIdx.x * 1024 + threadIdx.x);
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int p = k < np ? (int)id[k] : -1;
+    const bool own = p >= 0 && p < norig;
+    const unsigned long long m = __ballot(own);
+    if (lane == 0) s_n[w] = (unsigned)__popcll(m);
+    __syncthreads();
+    unsigned at = cnt[blockIdx.x];
+    for (int i = 0; i < w; ++i) at += s_n[i];
+    if (p >= 0) rank[p] = k;
+    if (own) order[at + (unsigned)__popcll(m & ((1ull << lane) - 1ull))] = p;
+}
+
+__global__ void k_tet_keys(const int4 *__restrict__ tets, int nt, const int *__restrict__ rank,
+                           unsigned *__restrict__ key, unsigned *__restrict__ id)
+{
+    const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (t >= nt) return;
+    const int4 v = tets[2 * (long long)t];
+    key[t] = (unsigned)min(min(rank[v.x], rank[v.y]), min(rank[v.z], rank[v.w]));
+    id[t] = (unsigned)t;
+}
+
+__global__ void k_tet_new(const unsigned *__restrict__ id, int nt, int *__restrict__ tnew)
+{
+    const int k = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (k < nt) tnew[id[k]] = k;
+}
+
+// tets in their new order with renumbered neighbours, vert_to_tet renumbered
+__global__ void k_renumber(const unsigned *__restrict__ id, int nt,
+                           const int *__restrict__ tnew, const int4 *__restrict__ raw,
+                           int4 *__restrict__ tets, const int *__restrict__ v2t_raw, int np,
+                           int *__restrict__ v2t)
+{
+    const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < nt) {
+        const long long t = id[k];
+        const int4 n = raw[2 * t + 1];
+        tets[2 * k] = raw[2 * t];
+        tets[2 * k + 1] = make_int4(n.x < 0 ? n.x : tnew[n.x], n.y < 0 ? n.y : tnew[n.y],
+                                    n.z < 0 ? n.z : tnew[n.z], n.w < 0 ? n.w : tnew[n.w]);
+    }
+    if (k < np) {
+        const int t = v2t_raw[k];
+        v2t[k] = t < 0 ? t : tnew[t];
+    }
+}
+
+static int bits_for(int n)
+{
+    int b = 1;
+    while (b < 31 && (1 << b) < n) ++b;
+    return b;
+}
+
+// scratch of launch_layout in unsigned words: two key and two id arrays, the
+// ranks, the digit counts and their tile sums
+size_t layout_scratch_words(int np, int nt)
+{
+    const size_t n = (size_t)std::max(std::max(np, nt), 1);
+    const size_t tiles = (n + SORT_TILE - 1) / SORT_TILE;
+    return 4 * n + (size_t)std::max(np, 1) + 256 * tiles + SCAN_TILE + tiles;
+}
+
+void launch_layout(const float4 *pts, int np, int norig, const StageBox &box, const int4 *raw,
+                   int nt, const int *v2t_raw, unsigned *scratch, int *order, int4 *tets,
+                   int *v2t, int *tnew, hipStream_t s)
+{
+    if (np <= 0) return;   // no particles, no tets
+    const size_t n = (size_t)std::max(np, nt);
+    const size_t tiles = (n + SORT_TILE - 1) / SORT_TILE;
+    unsigned *k0 = scratch, *v0 = k0 + n, *k1 = v0 + n, *v1 = k1 + n;
+    int *rank = reinterpret_cast<int *>(v1 + n);
+    unsigned *hist = reinterpret_cast<unsigned *>(rank + np), *sums = hist + 256 * tiles;
+    hipLaunchKernelGGL(k_morton_keys, dim3((np + 255) / 256), dim3(256), 0, s, pts, np, box, k0,
+                       v0);
+    const unsigned *id = radix_sort(k0, v0, k1, v1, (unsigned)np, 30, hist, sums, s) ? v1 : v0;
+    const int nob = (np + 1023) / 1024;
+    hipLaunchKernelGGL(k_order_count, dim3(nob), dim3(1024), 0, s, id, np, norig, hist);
+    scan_u32(hist, (unsigned)nob, sums, s);
+    hipLaunchKernelGGL(k_order_write, dim3(nob), dim3(1024), 0, s, id, np, norig,
+                       (const unsigned *)hist, rank, order);
+    if (nt > 0) {
+        hipLaunchKernelGGL(k_tet_keys, dim3((nt + 255) / 256), dim3(256), 0, s, raw, nt,
+                           (const int *)rank, k0, v0);
+        id = radix_sort(k0, v0, k1, v1, (unsigned)nt, bits_for(np), hist, sums, s) ? v1 : v0;
+        hipLaunchKernelGGL(k_tet_new, dim3((nt + 255) / 256), dim3(256), 0, s, id, nt, tnew);
+    }
+    const int m = std::max(np, nt);
+    hipLaunchKernelGGL(k_renumber, dim3((m + 255) / 256), dim3(256), 0, s, id, nt,
+                       (const int *)tnew, raw, tets, v2t_raw, np, v2t);
+}
+
+// circumcenters as xyz triples in the caller's numbering (tnew null: the
+// device numbering is the caller's)
+__global__ void k_unpack_cc(const float4 *__restrict__ cc, const int *__restrict__ tnew, int nt,
+                            float *__restrict__ out)
+{
+    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= nt) return;
+    const float4 q = cc[tnew ? tnew[t] : (int)t];
+    out[3 * t] = q.x;
+    out[3 * t + 1] = q.y;
+    out[3 * t + 2] = q.z;
+}
+
+void launch_unpack_cc(const float4 *cc, const int *tnew, int nt, float *out, hipStream_t s)
+{
+    if (nt <= 0) return;
+    hipLaunchKernelGGL(k_unpack_cc, dim3((nt + 255) / 256), dim3(256), 0, s, cc, tnew, nt, out);
+}
+
+}  // namespace t2
