@@ -492,14 +492,6 @@ static int validate_ranges(tess2_ctx *c, const tess2_block_t &b)
     return 0;
 }
 
-static float ord2f(unsigned u)
-{
-    u = (u & 0x80000000u) ? (u & 0x7fffffffu) : ~u;
-    float x;
-    memcpy(&x, &u, sizeof x);
-    return x;
-}
-
 // the block's cells and tets in Morton order: buffers in the new numbering
 // replace those in the caller's
 static int lay_out(tess2_ctx *c, DevBlock &d)
@@ -677,27 +669,40 @@ static int stage_block(tess2_ctx *c, const tess2_block_t &hb, DevBlock &d, bool 
     if (e == hipSuccess && d.np && hb.vert_to_tet)
         e = hipMemcpyAsync(d.v2t, hb.vert_to_tet, sizeof(int) * (size_t)d.np,
                            hipMemcpyHostToDevice, s);
+    int nrec = 0;
     if (e == hipSuccess) {
         if (!hb.vert_to_tet) launch_fill_u32((unsigned *)d.v2t, (size_t)d.np, 0xffffffffu, s);
-        launch_stage_check(xyz, d.np, d.tets, d.nt, d.v2t, d.pts, c->d_info, s);
-        e = hipMemcpyAsync(c->h_info, c->d_info, sizeof(StageInfo), hipMemcpyDeviceToHost, s);
+        nrec = launch_stage_check(xyz, d.np, d.tets, d.nt, d.v2t, d.pts, c->d_info, s);
+        if (nrec)
+            e = hipMemcpyAsync(c->h_info, c->d_info, sizeof(StageInfo) * nrec,
+                               hipMemcpyDeviceToHost, s);
     }
     // the caller's arrays are read until here
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     dfree(c, xyz);
     if (e != hipSuccess)
         return fail(c, TESS2_E_HIP, "block %d: upload: %s", d.gid, hipGetErrorString(e));
-    if (c->h_info->err) {
+    bool bad = false, odd = false;
+    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+    for (int k = 0; k < nrec; ++k) {
+        const StageInfo &q = c->h_info[k];
+        bad = bad || q.err;
+        odd = odd || q.nonfinite;
+        for (int i = 0; i < 3; ++i) {
+            lo[i] = std::min(lo[i], q.lo[i]);
+            hi[i] = std::max(hi[i], q.hi[i]);
+        }
+    }
+    if (bad) {
         r = validate_ranges(c, hb);
         return r ? r : fail(c, TESS2_E_INTERNAL, "block %d: the device's range check failed", d.gid);
     }
-    float lo[3] = {0, 0, 0}, hi[3] = {1, 1, 1};
-    if (d.np && !c->h_info->nonfinite)
+    if (d.np == 0)
         for (int i = 0; i < 3; ++i) {
-            lo[i] = ord2f(c->h_info->lo[i]);
-            hi[i] = ord2f(c->h_info->hi[i]);
+            lo[i] = 0;
+            hi[i] = 1;
         }
-    else   // infinities and NaN: comparisons in particle order
+    if (odd)   // infinities and NaN: comparisons in particle order
         for (int p = 0; p < d.np; ++p)
             for (int i = 0; i < 3; ++i) {
                 const float x = hb.particles[3 * p + i];
@@ -771,9 +776,10 @@ static int stage_blocks(tess2_ctx *c, const tess2_block_t *blocks, int nblocks, 
         }
     }
     int r = 0;
-    if (!c->d_info && (r = dalloc(c, &c->d_info, 1))) return r;
+    if (!c->d_info && (r = dalloc(c, &c->d_info, STAGE_RECORDS))) return r;
     if (!c->h_info &&
-        hipHostMalloc((void **)&c->h_info, sizeof(StageInfo), hipHostMallocDefault) != hipSuccess)
+        hipHostMalloc((void **)&c->h_info, sizeof(StageInfo) * STAGE_RECORDS,
+                      hipHostMallocDefault) != hipSuccess)
         return fail(c, TESS2_E_NOMEM, "pinned host buffer");
     // the new blocks beside the old ones, which stay staged when an input is
     // refused; without room for both, the inputs are checked on the host
@@ -871,7 +877,7 @@ static int alloc_lists(tess2_ctx *c, DevBlock &d, unsigned cap)
 }
 
 // grid + list buffers for one run
-static int ensure_grid(tess2_ctx *c, DevBlock &d, size_t n)
+static int ensure_grid(tess2_ctx *c, DevBlock &d, size_t n, bool cic)
 {
     d.ngrid = n;
     if (n > d.grid_cap) {
@@ -883,8 +889,14 @@ static int ensure_grid(tess2_ctx *c, DevBlock &d, size_t n)
         d.grid_cap = n;
     }
     if (!d.ovf) {
-        int r = alloc_lists(c, d, (unsigned)std::min<size_t>(std::max<size_t>(1u << 16, n / 8),
-                                                             1u << 30));
+        // an eighth of the grid's points is usually more than a scan shares;
+        // a CIC run makes 8 contributions a cell, and on a grid coarser than
+        // the particles nearly all share a point: room for them (up to 16M
+        // entries) spares the overflow and the second run (125k particles on
+        // a 301^2 plane: about 190 us of a 2.0 ms call)
+        size_t cap = std::max<size_t>(1u << 16, n / 8);
+        if (cic) cap = std::max(cap, std::min<size_t>(8 * (size_t)d.norig, 1u << 24));
+        int r = alloc_lists(c, d, (unsigned)std::min<size_t>(cap, 1u << 30));
         if (r) return r;
     }
     return 0;
@@ -1055,7 +1067,7 @@ static int prepare_run(tess2_ctx *c, const RunArgs &a)
         gp.project = a.project;
         const size_t n = (size_t)gp.bnum_idx[0] * gp.bnum_idx[1] *
                          (a.project ? 1 : (size_t)gp.bnum_idx[2]);
-        int r = ensure_grid(c, d, n);
+        int r = ensure_grid(c, d, n, a.alg == TESS2_DENSE_CIC);
         if (r) return r;
         if (exact && d.owner_cap < n) {
             r = dalloc(c, &d.owner, n);

@@ -107,13 +107,14 @@ struct Router {
     int rbase[3], rlen[3], roff[3], rn[3];
 };
 
-// what staging checks of a block's arrays (device); lo / hi: the bounding
-// box of the finite particles, as floats in an unsigned order
+// what one workgroup of the staging pass found in its part of a block's
+// arrays; lo / hi: the bounding box of its particles (lo > hi: none)
 struct StageInfo {
     unsigned err;          // an index out of range
     unsigned nonfinite;    // a coordinate that is infinite or NaN
-    unsigned lo[3], hi[3];
+    float lo[3], hi[3];
 };
+enum { STAGE_RECORDS = 1024 };   // workgroups of the pass at most
 
 // the particles' bounding box (the Morton grid)
 struct StageBox {
@@ -204,8 +205,9 @@ void launch_ghost_sends(const float4 *pts, const int4 *tets, int ntets, int nori
 // block as the caller gave it; then its cells in Morton order and its tets
 // renumbered by their lowest-ranked vertex (raw, v2t_raw: the caller's
 // numbering; scratch: layout_scratch_words(np, nt) words)
-void launch_stage_check(const float *xyz, int np, const int4 *tets, int nt, const int *v2t,
-                        float4 *pts, StageInfo *info, hipStream_t s);
+// (returns the records written)
+int launch_stage_check(const float *xyz, int np, const int4 *tets, int nt, const int *v2t,
+                       float4 *pts, StageInfo *info, hipStream_t s);
 size_t layout_scratch_words(int np, int nt);
 void launch_layout(const float4 *pts, int np, int norig, const StageBox &box, const int4 *raw,
                    int nt, const int *v2t_raw, unsigned *scratch, int *order, int4 *tets,
