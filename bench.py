@@ -454,7 +454,9 @@ def main():
     b_alg = 16 * N_all + 32 * T + 4 * N + 4 * G
     achieved = b_alg / (kern_ms * 1e-3) / 1e9
     ck = run.get_option("cell_kernel")
-    if multi:
+    if ck == -1 and (multi or N >= 16384):
+        kernel = "k_cell_geom + k_cell_scan"
+    elif multi:
         kernel = {1: "k_cells_mc_batched", 2: "k_cells_mc_batched",
                   4: "k_cells_mc_items"}.get(ck, "k_cells_ref_batched")
     else:

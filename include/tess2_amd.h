@@ -270,10 +270,11 @@ enum {
     TESS2_OPT_CHUNK_SMALL = 2,    /* cells per work item, blocks with < 20000 cells */
     TESS2_OPT_CHUNK_MEDIUM = 3,   /* cells per work item, blocks with < 100000 cells */
     TESS2_OPT_CHUNK_LARGE = 4,    /* cells per work item, larger blocks */
-    TESS2_OPT_CELL_KERNEL = 5     /* cell kernel: -1 (default) chosen per run (one block:
-                                   * 1, or 2 when cell boxes are large, 16 or more grid
-                                   * points per cell; several blocks: 3); 0 one cell per
-                                   * wave; 1 two cells per wave in the star / face / ring
+    TESS2_OPT_CELL_KERNEL = 5     /* cell kernel: -1 (default) chosen per run (several blocks,
+                                   * or 16384 cells and more: a geometry kernel and a scan
+                                   * kernel over all cells; else 1, or 2 when cell boxes are
+                                   * not small, 6 or more grid points per cell); 0 one cell
+                                   * per wave; 1 two cells per wave in the star / face / ring
                                    * phase; 2 the same with the verdict masks of boxes up
                                    * to 512 points (several blocks: 1 and 2 both run the
                                    * two-cell persistent kernel with those masks); 3 one
@@ -283,7 +284,7 @@ enum {
                                    * without the work queue, a workgroup per two cells,
                                    * two cells per wave as 2 (one block runs 2);
                                    * with the option at -1, tess2_autotune also times
-                                   * 1 and 4 and keeps the fastest */
+                                   * 3, 1 and 4 and keeps the fastest */
 };
 
 /* Set / read one option.  Chunk sizes 1..4096, waves per CU 1..64, cell
@@ -292,10 +293,11 @@ int tess2_set_option(tess2_ctx *ctx, int option, int value);
 int tess2_get_option(tess2_ctx *ctx, int option, int *value);
 
 /* Time the last tess2_run's arguments under each candidate work split of the
- * multi-block cell kernel (chunk sizes x persistent waves per CU), and, when
- * TESS2_OPT_CELL_KERNEL is -1, the two-cell kernels (cell kernels 1 and 4), `reps`
- * runs each, keep the fastest, and leave it set.  Results of the staged
- * blocks are those of the last timed run (identical for every candidate).
+ * multi-block persistent cell kernel (chunk sizes x persistent waves per CU),
+ * and, when TESS2_OPT_CELL_KERNEL is -1, the geometry and scan kernels and the
+ * two-cell kernels (cell kernels 1 and 4), `reps` runs each, keep the fastest,
+ * and leave it set.  Results of the staged blocks are those of the last timed
+ * run (identical for every candidate).
  * best_ms (may be NULL) receives the fastest median run time. */
 int tess2_autotune(tess2_ctx *ctx, int reps, float *best_ms);
 

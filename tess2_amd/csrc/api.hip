@@ -140,14 +140,18 @@ struct tess2_ctx {
     XcdQueues ixr{};                     // the item list's XCD ranges
     unsigned *d_queue = nullptr;
     XcdQueues xq{};
+    CellTile *d_tiles = nullptr;         // 64 cells of one block each (several blocks)
+    int ntiles = 0;
+    PlaneBuf planes{};                   // cell planes of one launch, plane_tiles tiles
+    int plane_tiles = 0;
     std::vector<BlockIn> h_ins;
     std::vector<GridP> h_gps;
     std::vector<CellOut> h_outs;
     // batched schedule (tess2_autotune): chunk size per block size class and
     // persistent waves per CU
     int chunk_small = 16, chunk_medium = 32, chunk_large = 64, waves_per_cu = 24;
-    // single-block cell kernel: -1 = chosen per run (cell_kernel_for), 0 =
-    // one cell per wave, 1 / 2 = two cells per wave in the geometry phase
+    // cell kernel: -1 = chosen per run (split_cells, cell_kernel_for), 0 = one
+    // cell per wave, 1 / 2 = two cells per wave in the geometry phase
     // (launch_cells_mc), 2 with the multi-word verdict masks
     int cell_kernel = -1;
     // graph replay of the steady-state sequence (tess2_set_option)
@@ -181,10 +185,10 @@ static bool same_args(const RunArgs &x, const RunArgs &y)
     return memcmp(&x, &y, sizeof(RunArgs)) == 0;
 }
 
-// The single-block cell kernel of a run: the option when set, else two cells
-// per wave, with the multi-word verdict masks when cell boxes are large
-// (16 or more grid points per cell: 2.1M cells on 512^3, 20.2 vs 24.7 ms;
-// at 8 points per cell the masks cost 2 %).
+// The one-pass single-block cell kernel of a run: the option when set, else
+// two cells per wave, with the multi-word verdict masks when cell boxes are
+// not small (6 or more grid points per cell: 4000 cells on 31^3 0.164 ->
+// 0.123 ms, on 15^3 0.147 and 0.148).
 static int cell_kernel_for(const tess2_ctx *c, int ncells, unsigned long long ngrid)
 {
     // the multi-block choices; one block: one cell per wave, or two with
@@ -192,8 +196,24 @@ static int cell_kernel_for(const tess2_ctx *c, int ncells, unsigned long long ng
     if (c->cell_kernel == 3) return 0;
     if (c->cell_kernel == 4) return 2;
     if (c->cell_kernel >= 0) return c->cell_kernel;
-    return ngrid >= 16ull * (unsigned long long)std::max(ncells, 1) ? 2 : 1;
+    return ngrid >= 6ull * (unsigned long long)std::max(ncells, 1) ? 2 : 1;
 }
+
+// Whether the cells take the geometry and scan kernels (several cells per wave,
+// 64 per workgroup) rather than a one-pass cell kernel: always for several
+// blocks (8 Plummer blocks, 57k cells on 128^3: 1.74 -> 0.74 ms; 11k cells on
+// 9 x 10 x 11: 0.96 -> 0.31), for one block from 16384 cells on.  Below that
+// their waves are too few to hide their longer chains: 4000 cells on 31^3
+// 0.153 against 0.123 ms, 16000 on 25^3 0.181 against 0.218, on 50^3 0.186
+// against 0.176, on 100^3 0.397 against 0.486; 262k on 128^3 0.61 against 0.95.
+static bool split_cells(const tess2_ctx *c, float eps, int nb, int ncells)
+{
+    return c->cell_kernel < 0 && eps >= 0.0f && (nb > 1 || ncells >= 16384);
+}
+
+// tiles per launch of those kernels: 2M cells, 664 bytes of planes each
+// (fewer tiles cost their tails: 2.1M cells in 4 turns 3.04 ms, in one 2.88)
+static constexpr int PLANE_TILES = 1 << 15;
 
 static void drop_graph(tess2_ctx *c)
 {
@@ -340,6 +360,13 @@ static void free_multi(tess2_ctx *c)
     dfree(c, c->d_chunks);
     dfree(c, c->d_items);
     dfree(c, c->d_queue);
+    dfree(c, c->d_tiles);
+    dfree(c, c->planes.hdr);
+    dfree(c, c->planes.fa);
+    dfree(c, c->planes.fb);
+    dfree(c, c->planes.big);
+    dfree(c, c->planes.nbig);
+    c->ntiles = c->plane_tiles = 0;
     dfree(c, c->d_stats);
     dfree(c, c->d_gpart);
     dfree(c, c->d_npts_tab);
@@ -567,6 +594,14 @@ static int build_chunks(tess2_ctx *c)
     if (r) return r;
     if (!ch.empty())
         HIPCHK(c, upload(c, c->d_chunks, ch.data(), sizeof(Chunk) * ch.size()));
+    std::vector<CellTile> tl;
+    for (int b = 0; b < (int)c->blocks.size(); ++b)
+        for (int s0 = 0; s0 < c->blocks[b].norig; s0 += CELL_TILE)
+            tl.push_back(CellTile{b, s0, std::min((int)CELL_TILE, c->blocks[b].norig - s0), 0});
+    c->ntiles = (int)tl.size();
+    if ((r = dalloc(c, &c->d_tiles, std::max<size_t>(tl.size(), 1)))) return r;
+    if (!tl.empty())
+        HIPCHK(c, upload(c, c->d_tiles, tl.data(), sizeof(CellTile) * tl.size()));
     // the item list of the queue-free launches: two cells at a time
     std::vector<Chunk> it;
     for (int b = 0; b < (int)c->blocks.size(); ++b)
@@ -1088,6 +1123,23 @@ static int prepare_run(tess2_ctx *c, const RunArgs &a)
         c->h_gps[k] = gp;
         c->h_outs[k] = make_out(d, a.want_vol != 0);
     }
+    if (a.alg == TESS2_DENSE_TESS && !exact && split_cells(c, a.eps, nb, c->blocks[0].norig)) {
+        int nt = c->ntiles;
+        if (nb == 1) nt = (c->blocks[0].norig + CELL_TILE - 1) / CELL_TILE;
+        const int chunks = (nt + PLANE_TILES - 1) / PLANE_TILES;
+        const int most = std::min(nt, PLANE_TILES);
+        if (most > c->plane_tiles) {
+            const size_t n = (size_t)most * CELL_TILE;
+            PlaneBuf &p = c->planes;
+            int r = 0;
+            c->plane_tiles = 0;
+            if ((r = dalloc(c, &p.hdr, 2 * n)) || (r = dalloc(c, &p.fa, n * PLANE_STRIDE)) ||
+                (r = dalloc(c, &p.fb, n * PLANE_STRIDE)) || (r = dalloc(c, &p.big, n)) ||
+                (r = dalloc(c, &p.nbig, (size_t)chunks)))
+                return r;
+            c->plane_tiles = most;
+        }
+    }
     if (c->desc_gen == c->gen && same_args(a, c->desc_args)) return 0;   // unchanged
     if (nb > 1) {
         // XCD ranges of the item list by estimated cost: a cell, plus its
@@ -1131,6 +1183,37 @@ static int prepare_run(tess2_ctx *c, const RunArgs &a)
     return 0;
 }
 
+// geometry, then scan and deposit, of all cells of a scan run, at most
+// PLANE_TILES tiles at a time
+template <bool MULTI>
+static void enqueue_split(tess2_ctx *c, CellSet<MULTI> set, int ntiles, hipStream_t s)
+{
+    const int chunks = (ntiles + PLANE_TILES - 1) / PLANE_TILES;
+    launch_fill_u32(c->planes.nbig, (size_t)chunks, 0u, s);
+    PlaneBuf pb = c->planes;
+    for (int k = 0; k < chunks; ++k, ++pb.nbig) {
+        set.tile0 = k * PLANE_TILES;
+        set.ntiles = std::min(PLANE_TILES, ntiles - set.tile0);
+        launch_cell_geom(set, pb, 1, s);
+        launch_cell_scan(set, pb, s);
+    }
+}
+
+// volume() of one block's cells (o.vol), the deferred ones too
+static void launch_volumes(const tess2_ctx *c, const BlockIn &in, const CellOut &o, hipStream_t s)
+{
+    const GridP gp{};   // no density: the grid is not read
+    const int ck = cell_kernel_for(c, in.ncells, 0);
+    if (split_cells(c, 0.0f, 1, in.ncells))
+        launch_cell_geom(CellSet<false>{in, o, nullptr, 0, (in.ncells + CELL_TILE - 1) / CELL_TILE},
+                         PlaneBuf{}, 0, s);
+    else if (ck == 0)
+        launch_cells_ref(in, gp, o, 0, s);
+    else
+        launch_cells_mc(in, nullptr, o, 0, ck, s);
+    launch_cells_ref_slow(in, gp, o, 0, s);
+}
+
 // the kernel sequence of a run (captured into a graph in graph mode)
 static int enqueue_kernels(tess2_ctx *c, const RunArgs &a)
 {
@@ -1159,20 +1242,17 @@ static int enqueue_kernels(tess2_ctx *c, const RunArgs &a)
         const bool multi = nb > 1;
         int *const *ntab = multi ? c->d_npts_tab : nullptr;
         const int *const *stab = multi ? c->d_stex_tab : nullptr;
+        if (a.want_vol && multi && c->cell_kernel < 0) {   // every block's volumes in one launch
+            launch_cell_geom(CellSet<true>{c->d_ins, c->d_outs, c->d_gps, c->d_router, c->d_tiles,
+                                           0, c->ntiles}, PlaneBuf{}, 0, s);
+            launch_cells_ref_slow_batched(c->d_ins, c->d_router, 0, s);
+        }
         for (int k = 0; k < nb; ++k) {
             DevBlock &d = c->blocks[k];
             const BlockIn &in = c->h_ins[k];
             const GridP &gp = c->h_gps[k];
-            if (a.want_vol) {
-                // volume() as the reference computes it
-                CellOut ov = make_out(d, true);
-                const int ck = nb > 1 ? 0 : cell_kernel_for(c, d.norig, d.ngrid);
-                if (ck == 0)
-                    launch_cells_ref(in, gp, ov, 0, s);
-                else if (launch_cells_mc(in, c->d_gps + k, ov, 0, ck, s))
-                    return fail(c, TESS2_E_ARG, "unknown cell kernel %d", ck);
-                launch_cells_ref_slow(in, gp, ov, 0, s);
-            }
+            // volume() as the reference computes it
+            if (a.want_vol && !(multi && c->cell_kernel < 0)) launch_volumes(c, in, c->h_outs[k], s);
             launch_hash_build(d.pts, d.np, d.hash, d.hstart, d.hfill, d.hsums, d.hbk, d.hsorted,
                               multi ? d.hkey : nullptr, s);
             launch_exact_status(in, gp, d.status_ex, a.precision, d.ctrs,
@@ -1202,6 +1282,17 @@ static int enqueue_kernels(tess2_ctx *c, const RunArgs &a)
             launch_cic(c->h_ins[k], c->h_gps[k], c->h_outs[k], nb > 1 ? c->d_router : nullptr, k,
                        s);
         if (ev) HIPCHK(c, hipEventRecord(c->ev_k1, s));
+    } else if (split_cells(c, a.eps, nb, c->blocks[0].norig)) {
+        if (ev) HIPCHK(c, hipEventRecord(c->ev_k0, s));
+        if (nb == 1)
+            enqueue_split(c, CellSet<false>{c->h_ins[0], c->h_outs[0], c->d_gps, 0, 0},
+                          (c->blocks[0].norig + CELL_TILE - 1) / CELL_TILE, s);
+        else
+            enqueue_split(c, CellSet<true>{c->d_ins, c->d_outs, c->d_gps, c->d_router, c->d_tiles,
+                                           0, 0}, c->ntiles, s);
+        if (ev) HIPCHK(c, hipEventRecord(c->ev_k1, s));
+        if (nb == 1) launch_cells_ref_slow(c->h_ins[0], c->h_gps[0], c->h_outs[0], 1, s);
+        else launch_cells_ref_slow_batched(c->d_ins, c->d_router, 1, s);
     } else if (nb == 1) {
         if (ev) HIPCHK(c, hipEventRecord(c->ev_k0, s));
         const int ck = cell_kernel_for(c, c->blocks[0].norig, c->blocks[0].ngrid);
@@ -1493,9 +1584,16 @@ extern "C" int tess2_autotune(tess2_ctx *c, int reps, float *best_ms)
     if (r) return r;
     if (c->blocks.size() > 1) {
         // chunk sizes for (small, medium, large) blocks and persistent waves
+        // of the persistent kernels, then the two-cell kernels with the chosen
+        // split; with the cell kernel on automatic they compete with the
+        // geometry and scan kernels timed above
         static const int chunks[][3] = {{8, 16, 32}, {16, 32, 64}, {32, 64, 128}, {64, 128, 256}};
         static const int waves[] = {8, 16, 24, 32};
+        const bool any = c->cell_kernel == -1;
+        int bk = c->cell_kernel;
         int bc[3] = {c->chunk_small, c->chunk_medium, c->chunk_large}, bw = c->waves_per_cu;
+        float bsplit = any ? INFINITY : best;
+        if (any && (r = tess2_set_option(c, TESS2_OPT_CELL_KERNEL, 3))) return r;
         for (const auto &ch : chunks)
             for (int w : waves) {
                 if ((r = tess2_set_option(c, TESS2_OPT_CHUNK_SMALL, ch[0])) ||
@@ -1505,8 +1603,8 @@ extern "C" int tess2_autotune(tess2_ctx *c, int reps, float *best_ms)
                     return r;
                 float t = 0.0f;
                 if ((r = time_runs(c, 1, &t)) || (r = time_runs(c, reps, &t))) return r;
-                if (t < best) {
-                    best = t;
+                if (t < bsplit) {
+                    bsplit = t;
                     bc[0] = ch[0];
                     bc[1] = ch[1];
                     bc[2] = ch[2];
@@ -1518,10 +1616,11 @@ extern "C" int tess2_autotune(tess2_ctx *c, int reps, float *best_ms)
             (r = tess2_set_option(c, TESS2_OPT_CHUNK_LARGE, bc[2])) ||
             (r = tess2_set_option(c, TESS2_OPT_WAVES_PER_CU, bw)))
             return r;
-        // the persistent and the queue-free two-cell kernels with the chosen
-        // split, unless a cell kernel was asked for
-        if (c->cell_kernel == -1) {
-            int bk = -1;
+        if (bsplit < best) {
+            best = bsplit;
+            if (any) bk = 3;
+        }
+        if (any) {
             for (int k : {1, 4}) {
                 float t = 0.0f;
                 if ((r = tess2_set_option(c, TESS2_OPT_CELL_KERNEL, k)) ||
@@ -1642,10 +1741,7 @@ extern "C" int tess2_volumes(tess2_ctx *c, const tess2_block_t *block, float *ou
     BlockIn in = make_in(d);
     CellOut o = make_out(d, true);
     GridP gp{};
-    const int ck = c->cell_kernel >= 0 ? c->cell_kernel : 1;
-    if (ck == 0) launch_cells_ref(in, gp, o, 0, s);
-    else launch_cells_mc(in, nullptr, o, 0, ck, s);   // no density: the grid is not read
-    launch_cells_ref_slow(in, gp, o, 0, s);
+    launch_volumes(c, in, o, s);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipMemcpyAsync(d.hm->ctrs, d.ctrs, sizeof(unsigned) * C_NCTR, hipMemcpyDeviceToHost,
                              s));

@@ -33,6 +33,7 @@
 #include "deposit.hpp"
 #include "scan_bits.hpp"
 #include "scan_deposit.hpp"
+#include "scan_lines.hpp"
 
 namespace t2 {
 
@@ -79,11 +80,14 @@ __device__ __forceinline__ int comp(const int4 &q, int i)
 template <int NS> constexpr int hash_entries() { return 2 * 64 * NS; }
 template <int NS> constexpr int hash_ints() { return 2 * hash_entries<NS>() + 2 * 64 * NS; }
 
-template <int NS, int NF, int RMAX, bool WIDE = false, bool SPEC = false>
+// LINES: boxes that fit scan by lines (scan_cell_lines; eps >= 0), in *sl,
+// which may overlay s_u
+template <int NS, int NF, int RMAX, bool WIDE = false, bool SPEC = false, bool LINES = false>
 __device__ void cell_ref_body(const int v, const BlockIn &in, const GridP *gpp,
                               const CellOut &o, const int want_density, const bool can_defer,
                               int4 *s_v, int *s_ns, float4 *s_cc, int4 *s_u, int *s_h,
-                              const Router *rt = nullptr, const int self = 0)
+                              const Router *rt = nullptr, const int self = 0,
+                              LineShared *sl = nullptr)
 {
     constexpr int SMAX = 64 * NS;
     constexpr int FMAX = 64 * NF;
@@ -402,6 +406,23 @@ __device__ void cell_ref_body(const int v, const BlockIn &in, const GridP *gpp,
             if (isnan(c00.y)) { mny = c00.y; mxy = c00.y; }
             if (isnan(c00.z)) { mnz = c00.z; mxz = c00.z; }
         }
+        if constexpr (LINES) {
+            __syncthreads();
+            float4 *fa = s_cc;
+            float2 *fb = reinterpret_cast<float2 *>(s_v);
+#pragma unroll
+            for (int j = 0; j < NF; ++j) {
+                const int f = j * 64 + lane;
+                if (f < F) {
+                    fa[f] = make_float4(fnx[j], fny[j], fnz[j], ffx[j]);
+                    fb[f] = make_float2(ffy[j], ffz[j]);
+                }
+            }
+            __syncthreads();
+            if (scan_cell_lines(v, site, F, fa, fb, mnx, mny, mnz, mxx, mxy, mxz, *gpp, o, rt,
+                                self, *sl))
+                return;
+        }
         scan_deposit<NF, RMAX, WIDE, WIDE>(v, site, F, fnx, fny, fnz, ffx, ffy, ffz, mnx, mny, mnz,
                                      mxx, mxy, mxz, *gpp, o, rt, self, s_cc,
                                      reinterpret_cast<float2 *>(s_v), false, s_u);
@@ -437,6 +458,13 @@ __global__ __launch_bounds__(64) void k_cells_ref(BlockIn in, GridP gp, CellOut 
     cell_ref_body<NS, NF, RMAX>(v, in, &gp, o, want_density, true, s_v, s_ns, s_cc, s_u, s_h);
 }
 
+// the large-capacity pass's neighbour slots (and scan runs), later its lines
+template <int NS, int RMAX>
+union SlowShared {
+    int4 slots[(64 * NS > RMAX) ? 64 * NS : RMAX];
+    LineShared lines;
+};
+
 // large-capacity pass over the cells the fast kernel deferred; the grid is
 // fixed and each workgroup strides over the deferred list
 template <int NS, int NF, int RMAX>
@@ -446,14 +474,15 @@ __global__ __launch_bounds__(64) void k_cells_ref_slow(BlockIn in, GridP gp, Cel
     __shared__ int4 s_v[64 * NS];
     __shared__ int s_ns[64 * NS * 4];
     __shared__ float4 s_cc[64 * NS];
-    __shared__ int4 s_u[(64 * NS > RMAX) ? 64 * NS : RMAX];
+    __shared__ SlowShared<NS, RMAX> s_u;
     __shared__ int s_h[hash_ints<NS>()];
     unsigned n = o.ctrs[C_SLOW];
     if (n > o.slow_cap) n = o.slow_cap;
     for (unsigned k = blockIdx.x; k < n; k += gridDim.x) {
         const int v = o.slow[k];
-        cell_ref_body<NS, NF, RMAX>(v, in, &gp, o, want_density, false, s_v, s_ns, s_cc, s_u,
-                                    s_h);
+        cell_ref_body<NS, NF, RMAX, false, false, true>(v, in, &gp, o, want_density, false, s_v,
+                                                        s_ns, s_cc, s_u.slots, s_h, nullptr, 0,
+                                                        &s_u.lines);
         __syncthreads();
     }
 }
@@ -515,7 +544,7 @@ __global__ __launch_bounds__(64) void k_cells_ref_slow_batched(const BlockIn *__
     __shared__ int4 s_v[64 * NS];
     __shared__ int s_ns[64 * NS * 4];
     __shared__ float4 s_cc[64 * NS];
-    __shared__ int4 s_u[(64 * NS > RMAX) ? 64 * NS : RMAX];
+    __shared__ SlowShared<NS, RMAX> s_u;
     __shared__ int s_h[hash_ints<NS>()];
     // the lists of up to 64 blocks at a time, concatenated and dealt to the
     // workgroups in turn (one block per lane: list lengths and their
@@ -540,9 +569,10 @@ __global__ __launch_bounds__(64) void k_cells_ref_slow_batched(const BlockIn *__
             const unsigned first = __shfl(incl - n, lb);
             const int b = b0 + lb;
             const CellOut &o = rt->outs[b];
-            cell_ref_body<NS, NF, RMAX, true>(o.slow[g - first], ins[b], rt->gps + b, o,
-                                              want_density, false, s_v, s_ns, s_cc, s_u, s_h,
-                                              rt, b);
+            cell_ref_body<NS, NF, RMAX, true, false, true>(o.slow[g - first], ins[b], rt->gps + b,
+                                                           o, want_density, false, s_v, s_ns,
+                                                           s_cc, s_u.slots, s_h, rt, b,
+                                                           &s_u.lines);
             __syncthreads();
         }
     }
@@ -593,17 +623,33 @@ void launch_cells_ref_slow(const BlockIn &in, const GridP &gp, const CellOut &o,
 // ---------------------------------------------------------------------------
 __global__ void k_cic(BlockIn in, GridP gp, CellOut o, const Router *rt, int self)
 {
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= in.ncells) return;
+    const int v0 = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool on = v0 < in.ncells;
+    const int v = on ? v0 : in.ncells - 1;   // idle lanes stay for the wave's pushes
     const float4 p = in.pts[v];
     int mn[3];
     float m8[8];
     cic_weights(p.x, p.y, p.z, gp.mass, gp, mn, m8);
-    for (int k = 0; k < 8; ++k)
-        deposit_point(mn[0] + (k & 1), mn[1] + ((k >> 1) & 1), mn[2] + (k >> 2), m8[k],
-                      cell_key(v, gp.project ? (k >> 2) : 0), gp, o, rt, self);
-    o.status[v] = ST_CIC;
-    o.npts[v] = 8;
+    long long at[8];
+    unsigned key[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const int gx = mn[0] + (k & 1), gy = mn[1] + ((k >> 1) & 1), gz = mn[2] + (k >> 2);
+        key[k] = cell_key(v, gp.project ? (k >> 2) : 0);
+        at[k] = -1;
+        if (on) {
+            at[k] = own_lidx(gx, gy, gz, gp);
+            if (at[k] < 0)
+                atomicAdd(&o.ctrs[route_point(gx, gy, gz, m8[k], key[k], rt, self) ? C_ROUTED
+                                                                                  : C_OFFBLOCK],
+                          1u);
+        }
+    }
+    wave_push<8>(at, m8, key, gp.div, o);
+    if (on) {
+        o.status[v] = ST_CIC;
+        o.npts[v] = 8;
+    }
 }
 
 void launch_cic(const BlockIn &in, const GridP &gp, const CellOut &o, const Router *rt_dev,

@@ -146,6 +146,62 @@ struct BlockIn {
     int ntets;
 };
 
+// 64 consecutive cells (of the Morton order) of one block; base: the position
+// of the first in the buffers that run over all cells of a launch
+enum { CELL_TILE = 64 };
+struct CellTile {
+    int block, start, count, base;
+};
+
+// The cells of a launch: one block given by value, or all blocks of a run by
+// their descriptors in device memory and a tile list (no tile holds cells of
+// two blocks).
+template <bool MULTI> struct CellSet;
+template <> struct CellSet<false> {
+    BlockIn bin;
+    CellOut bout;
+    const GridP *gp;     // device memory, null without density
+    int tile0, ntiles;   // the launch's tiles; positions count from the first
+    __device__ __forceinline__ CellTile tile(int t) const
+    {
+        const int s = (tile0 + t) * CELL_TILE;
+        return CellTile{0, s, min((int)CELL_TILE, bin.ncells - s), t * CELL_TILE};
+    }
+    __device__ __forceinline__ const BlockIn &in(int) const { return bin; }
+    __device__ __forceinline__ const CellOut &out(int) const { return bout; }
+    __device__ __forceinline__ const GridP &grid(int) const { return *gp; }
+    __device__ __forceinline__ const Router *router() const { return nullptr; }
+};
+template <> struct CellSet<true> {
+    const BlockIn *ins;
+    const CellOut *outs;
+    const GridP *gps;
+    const Router *rt;
+    const CellTile *tiles;
+    int tile0, ntiles;
+    __device__ __forceinline__ CellTile tile(int t) const
+    {
+        const CellTile q = tiles[tile0 + t];
+        return CellTile{q.block, q.start, q.count, t * CELL_TILE};
+    }
+    __device__ __forceinline__ const BlockIn &in(int b) const { return ins[b]; }
+    __device__ __forceinline__ const CellOut &out(int b) const { return outs[b]; }
+    __device__ __forceinline__ const GridP &grid(int b) const { return gps[b]; }
+    __device__ __forceinline__ const Router *router() const { return rt; }
+};
+
+// What the geometry kernel leaves for the scan, by position: bbox and face
+// count (0: nothing to scan), {min xyz, faces}, {max xyz, cell}; the face
+// planes {n, f0.x}, {f0.y, f0.z}, PLANE_STRIDE per cell
+enum { PLANE_STRIDE = 26 };
+struct PlaneBuf {
+    float4 *hdr;
+    float4 *fa;
+    float2 *fb;
+    int2 *big;         // {block, position} of the cells for one wave each
+    unsigned *nbig;    // their number, cleared with the run's counters
+};
+
 // find or insert key (>= 0) in an open-addressing table of HS entries in
 // LDS (-1 = empty); returns the entry, or -1 when HS probes found no room
 template <int HS>
@@ -226,6 +282,16 @@ void launch_cells_ref(const BlockIn &in, const GridP &gp, const CellOut &o,
                       int want_density, hipStream_t s);
 void launch_cells_ref_slow(const BlockIn &in, const GridP &gp, const CellOut &o,
                            int want_density, hipStream_t s);
+// stars, faces, volumes of all tiles' cells (cells_geom.hip); with
+// want_density also what the scan needs, in pb (else unused)
+void launch_cell_geom(const CellSet<false> &set, const PlaneBuf &pb, int want_density,
+                      hipStream_t s);
+void launch_cell_geom(const CellSet<true> &set, const PlaneBuf &pb, int want_density,
+                      hipStream_t s);
+// scan and deposit of the cells whose planes are in pb (cells_scan.hip);
+// eps >= 0
+void launch_cell_scan(const CellSet<false> &set, const PlaneBuf &pb, hipStream_t s);
+void launch_cell_scan(const CellSet<true> &set, const PlaneBuf &pb, hipStream_t s);
 // several cells per wave in the geometry phase (cells_mc.hip); variant 1..2
 // picks the verdict masks; returns -1 for an unknown variant.  gp is the
 // block's grid descriptor in device memory (read only by the scan, so that

@@ -7,14 +7,13 @@
 // cell's faces are held one per lane (face j*64 + lane in register j).
 #pragma once
 
+#include "cell_status.hpp"
 #include "deposit.hpp"
 #include "geom.hpp"
 #include "kernels.hpp"
 #include "scan_bits.hpp"
 
 namespace t2 {
-
-enum { ST_SCAN = 0, ST_CIC = 1, ST_INCOMPLETE = 2, ST_OUTSIDE = 3, ST_DEGENERATE = 4 };
 
 __device__ __forceinline__ bool wide_bit(unsigned long long w, int b) { return (w >> b) & 1ull; }
 
