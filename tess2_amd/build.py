@@ -15,7 +15,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libtess2_amd.so")
 SOURCES = ["api.hip", "common.hip", "cells_ref.hip", "cells_mc.hip", "cells_geom.hip", "cells_scan.hip",
            "exact.hip", "fold.hip",
-           "ghosts.hip", "stage.hip"]
+           "ghosts.hip", "stage.hip", "transfer.hip"]
 HOST_SOURCES = ["grid_io.cpp"]      # host-only C++ (file output)
 
 HIPCC_FLAGS = [

@@ -453,6 +453,7 @@ extern "C" int tess2_create(tess2_ctx **out, int device)
     const hipError_t se = scratch_lookup(device);
     if (se != hipSuccess)
         fail(c, TESS2_E_HIP, "scratch lookup on device %d: %s", device, hipGetErrorString(se));
+    transfer_open();
     *out = c;
     return 0;
 }
@@ -474,6 +475,7 @@ extern "C" int tess2_destroy(tess2_ctx *c)
     if (c->ev_k0) (void)hipEventDestroy(c->ev_k0);
     if (c->ev_k1) (void)hipEventDestroy(c->ev_k1);
     if (c->stream) (void)hipStreamDestroy(c->stream);
+    transfer_close();
     delete c;
     return 0;
 }
@@ -697,13 +699,11 @@ static int stage_block(tess2_ctx *c, const tess2_block_t &hb, DevBlock &d, bool 
         (r = dalloc(c, &d.npts, (size_t)d.norig)) || (r = dalloc(c, &xyz, 3 * (size_t)d.np)))
         return r;
     hipError_t e = hipSuccess;
-    if (d.np) e = hipMemcpyAsync(xyz, hb.particles, 12 * (size_t)d.np, hipMemcpyHostToDevice, s);
-    if (e == hipSuccess && d.nt)
-        e = hipMemcpyAsync(d.tets, hb.tets, sizeof(tess2_tet_t) * (size_t)d.nt,
-                           hipMemcpyHostToDevice, s);
-    if (e == hipSuccess && d.np && hb.vert_to_tet)
-        e = hipMemcpyAsync(d.v2t, hb.vert_to_tet, sizeof(int) * (size_t)d.np,
-                           hipMemcpyHostToDevice, s);
+    e = copy_to_device(xyz, hb.particles, 12 * (size_t)d.np, s);
+    if (e == hipSuccess)
+        e = copy_to_device(d.tets, hb.tets, sizeof(tess2_tet_t) * (size_t)d.nt, s);
+    if (e == hipSuccess && hb.vert_to_tet)
+        e = copy_to_device(d.v2t, hb.vert_to_tet, sizeof(int) * (size_t)d.np, s);
     int nrec = 0;
     if (e == hipSuccess) {
         if (!hb.vert_to_tet) launch_fill_u32((unsigned *)d.v2t, (size_t)d.np, 0xffffffffu, s);
@@ -1658,11 +1658,11 @@ extern "C" int tess2_fetch(tess2_ctx *c, int b, float *density, float *volumes,
     HIPCHK(c, hipStreamSynchronize(c->stream));
     DevBlock &d = c->blocks[b];
     if (density && d.density)
-        HIPCHK(c, hipMemcpy(density, d.density, sizeof(float) * d.ngrid, hipMemcpyDeviceToHost));
+        HIPCHK(c, copy_to_host(density, d.density, sizeof(float) * d.ngrid, c->stream));
     if (volumes && d.norig) {
         if (!d.vol_valid)
             return fail(c, TESS2_E_ARG, "block %d: the last run computed no volumes", b);
-        HIPCHK(c, hipMemcpy(volumes, d.vol, sizeof(float) * d.norig, hipMemcpyDeviceToHost));
+        HIPCHK(c, copy_to_host(volumes, d.vol, sizeof(float) * (size_t)d.norig, c->stream));
     }
     if (circumcenters && d.nt) {
         // packed on the device, in the caller's numbering
@@ -1670,9 +1670,7 @@ extern "C" int tess2_fetch(tess2_ctx *c, int b, float *density, float *volumes,
         const int r = dalloc(c, &tmp, 3 * (size_t)d.nt);
         if (r) return r;
         launch_unpack_cc(d.cc, d.laid ? d.tet_new : nullptr, d.nt, tmp, c->stream);
-        hipError_t e = hipMemcpyAsync(circumcenters, tmp, 12 * (size_t)d.nt,
-                                      hipMemcpyDeviceToHost, c->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+        const hipError_t e = copy_to_host(circumcenters, tmp, 12 * (size_t)d.nt, c->stream);
         dfree(c, tmp);
         HIPCHK(c, e);
     }
@@ -1688,7 +1686,7 @@ extern "C" int tess2_fetch_owner(tess2_ctx *c, int b, int *owner)
     DevBlock &d = c->blocks[b];
     if (!d.owner || d.owner_cap < d.ngrid)
         return fail(c, TESS2_E_ARG, "no exact-assignment run on block %d", b);
-    HIPCHK(c, hipMemcpy(owner, d.owner, sizeof(int) * d.ngrid, hipMemcpyDeviceToHost));
+    HIPCHK(c, copy_to_host(owner, d.owner, sizeof(int) * d.ngrid, c->stream));
     return 0;
 }
 
@@ -1699,9 +1697,9 @@ extern "C" int tess2_dense_cells(tess2_ctx *c, int b, int *status, int *npts)
     HIPCHK(c, hipStreamSynchronize(c->stream));
     DevBlock &d = c->blocks[b];
     if (status && d.norig)
-        HIPCHK(c, hipMemcpy(status, d.status, sizeof(int) * d.norig, hipMemcpyDeviceToHost));
+        HIPCHK(c, copy_to_host(status, d.status, sizeof(int) * (size_t)d.norig, c->stream));
     if (npts && d.norig)
-        HIPCHK(c, hipMemcpy(npts, d.npts, sizeof(int) * d.norig, hipMemcpyDeviceToHost));
+        HIPCHK(c, copy_to_host(npts, d.npts, sizeof(int) * (size_t)d.norig, c->stream));
     return 0;
 }
 

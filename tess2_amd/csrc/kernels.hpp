@@ -229,6 +229,14 @@ __device__ __forceinline__ int xcd_item(int b, int n)
 }
 __host__ __forceinline__ int xcd_grid(int n) { return ((n + 7) >> 3) << 3; }
 
+// copies between pageable host memory and device memory (transfer.hip), after
+// the stream's earlier work.  copy_to_host is done when it returns; the array
+// given to copy_to_device may be read until the stream has been waited for.
+// The pinned slots behind them live while a context is open.
+void transfer_open();
+void transfer_close();
+hipError_t copy_to_host(void *dst, const void *src, size_t bytes, hipStream_t s);
+hipError_t copy_to_device(void *dst, const void *src, size_t bytes, hipStream_t s);
 // circumcenters; cc.w = error bound of the float solve (inf when undefined)
 void launch_circumcenters(const float4 *pts, const int4 *tets, int ntets, float4 *cc,
                           hipStream_t s);
