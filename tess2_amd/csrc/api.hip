@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdint>
 #include <cmath>
 #include <cstdarg>
@@ -164,6 +165,7 @@ struct tess2_ctx {
     BlockStats *d_stats = nullptr, *h_stats = nullptr;   // per-block counters, device / pinned
     int h_stats_cap = 0;
     StageInfo *d_info = nullptr, *h_info = nullptr;      // one block's staging checks
+    unsigned *h_noalloc = nullptr;   // pinned: the counters of an allocation-free call
     // device buffers given back by earlier stagings, for the next one to use
     std::unordered_map<void *, size_t> live;             // bytes of every buffer in use
     std::vector<std::pair<void *, size_t>> spare;        // oldest first
@@ -444,6 +446,12 @@ extern "C" int tess2_create(tess2_ctx **out, int device)
         delete c;
         return TESS2_E_HIP;
     }
+    // allocated here, since the entry point that reads it allocates nothing
+    if (hipHostMalloc((void **)&c->h_noalloc, sizeof(unsigned) * (C_NCTR + 1),
+                      hipHostMallocDefault) != hipSuccess) {
+        delete c;
+        return TESS2_E_HIP;
+    }
     int ncu = 0;
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess &&
         ncu > 0)
@@ -470,6 +478,7 @@ extern "C" int tess2_destroy(tess2_ctx *c)
     drop_spare(c);
     if (c->h_stats) (void)hipHostFree(c->h_stats);
     if (c->h_info) (void)hipHostFree(c->h_info);
+    if (c->h_noalloc) (void)hipHostFree(c->h_noalloc);
     if (c->ev_run0) (void)hipEventDestroy(c->ev_run0);
     if (c->ev_run1) (void)hipEventDestroy(c->ev_run1);
     if (c->ev_k0) (void)hipEventDestroy(c->ev_k0);
@@ -966,7 +975,7 @@ static CellOut make_out(DevBlock &d, bool want_vol)
 
 static BlockIn make_in(DevBlock &d)
 {
-    BlockIn in;
+    BlockIn in{};
     in.pts = d.pts;
     in.tets = d.tets;
     in.v2t = d.v2t;
@@ -1203,7 +1212,8 @@ static void enqueue_split(tess2_ctx *c, CellSet<MULTI> set, int ntiles, hipStrea
 static void launch_volumes(const tess2_ctx *c, const BlockIn &in, const CellOut &o, hipStream_t s)
 {
     const GridP gp{};   // no density: the grid is not read
-    const int ck = cell_kernel_for(c, in.ncells, 0);
+    // 4096 cells or fewer: a wave per cell, which ends soonest
+    const int ck = c->cell_kernel < 0 && in.ncells <= 4096 ? 0 : cell_kernel_for(c, in.ncells, 0);
     if (split_cells(c, 0.0f, 1, in.ncells))
         launch_cell_geom(CellSet<false>{in, o, nullptr, 0, (in.ncells + CELL_TILE - 1) / CELL_TILE},
                          PlaneBuf{}, 0, s);
@@ -1782,7 +1792,8 @@ extern "C" int tess2_volumes_noalloc(tess2_ctx *c, const float *particles, int n
     // status, point counts, deferred-cell list (one slot per cell, so it
     // cannot overflow); 256-byte aligned regions
     auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
-    const size_t o_ctrs = 0, o_pts = up(o_ctrs + sizeof(unsigned) * C_NCTR),
+    // the counters, the word a range violation marks, then (o_pts) the arrays
+    const size_t o_ctrs = 0, o_pts = up(o_ctrs + sizeof(unsigned) * (C_NCTR + 1)),
                  o_cc = up(o_pts + sizeof(float4) * (size_t)np),
                  o_st = up(o_cc + sizeof(float4) * (size_t)nt),
                  o_np = up(o_st + sizeof(int) * (size_t)norig),
@@ -1797,18 +1808,14 @@ extern "C" int tess2_volumes_noalloc(tess2_ctx *c, const float *particles, int n
     float4 *cc = reinterpret_cast<float4 *>(base + o_cc);
     const int4 *t4 = reinterpret_cast<const int4 *>(tets);
     hipStream_t s = c->stream;
-    // the counters start at zero on every call (the array keeps the last
-    // call's contents); a kernel, not a memset
-    launch_fill_u32(ctrs, C_NCTR, 0u, s);
-    launch_check_block(t4, nt, vert_to_tet, np, &ctrs[C_ERR], 16u, s);
-    unsigned err = 0;
-    HIPCHK(c, hipGetLastError());
-    HIPCHK(c, hipMemcpyAsync(&err, &ctrs[C_ERR], sizeof err, hipMemcpyDeviceToHost, s));
-    HIPCHK(c, hipStreamSynchronize(s));
-    if (err & 16u) return fail(c, TESS2_E_ARG, "a tet or vert_to_tet index is out of range");
-    launch_pack_points(particles, np, pts, s);
-    launch_circumcenters(pts, t4, nt, cc, s);
+    unsigned *stop = ctrs + C_NCTR;
+    static std::atomic<unsigned> calls{0};
+    unsigned token = ++calls;
+    if (token == 0u) token = ++calls;   // 0 is the array's first content
+    launch_device_block(particles, np, t4, nt, vert_to_tet, pts, cc, ctrs, stop, token, s);
     BlockIn in{};
+    in.stop = stop;
+    in.token = token;
     in.pts = pts;
     in.tets = t4;
     in.v2t = vert_to_tet;
@@ -1824,13 +1831,15 @@ extern "C" int tess2_volumes_noalloc(tess2_ctx *c, const float *particles, int n
     o.slow = reinterpret_cast<int *>(base + o_sl);
     o.slow_cap = (unsigned)norig;
     o.ncells = norig;
-    GridP gp{};
-    launch_cells_ref(in, gp, o, 0, s);
-    launch_cells_ref_slow(in, gp, o, 0, s);
+    launch_volumes(c, in, o, s);
     HIPCHK(c, hipGetLastError());
-    HIPCHK(c, hipMemcpyAsync(&err, &ctrs[C_ERR], sizeof err, hipMemcpyDeviceToHost, s));
+    HIPCHK(c, hipMemcpyAsync(c->h_noalloc, ctrs, sizeof(unsigned) * (C_NCTR + 1),
+                             hipMemcpyDeviceToHost, s));
     HIPCHK(c, hipStreamSynchronize(s));
-    if (err & 4u) return fail(c, TESS2_E_CAPACITY, "a cell exceeds the per-cell capacities");
+    if (c->h_noalloc[C_NCTR] == token)
+        return fail(c, TESS2_E_ARG, "a tet or vert_to_tet index is out of range");
+    if (c->h_noalloc[C_ERR] & 4u)
+        return fail(c, TESS2_E_CAPACITY, "a cell exceeds the per-cell capacities");
     return 0;
 }
 

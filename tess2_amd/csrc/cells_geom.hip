@@ -159,6 +159,7 @@ __global__ __launch_bounds__(64) void k_cell_geom(CellSet<MULTI> set, PlaneBuf p
     if (item < 0) return;
     const CellTile tile = set.tile(item / WPT);
     const BlockIn in = set.in(tile.block);
+    if (!MULTI && !PLANES && in.stopped()) return;
     const int rel = (item % WPT) * CPW + g;   // this group's cell in the tile
     const bool have = rel < tile.count;
     const int v = have ? (in.order ? in.order[tile.start + rel] : tile.start + rel) : -1;

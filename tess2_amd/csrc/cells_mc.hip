@@ -458,7 +458,7 @@ __global__ __launch_bounds__(64, MINW) void k_cells_mc(BlockIn in,
     __shared__ __align__(16) unsigned char smem[CPW * McLayout<SG, HG>::BYTES];
     const int nitems = (in.ncells + CPW - 1) / CPW;
     const int item = xcd_item((int)blockIdx.x, nitems);
-    if (item < 0) return;
+    if (item < 0 || in.stopped()) return;
     const int k = item * CPW + (int)(threadIdx.x & 63) / (64 / CPW);
     const int v = k < in.ncells ? (in.order ? in.order[k] : k) : -1;
     cells_mc_body<CPW, SG, HG, FG, RMAX, WIDE, false>(v, in, gp, o, want_density, nullptr, 0,

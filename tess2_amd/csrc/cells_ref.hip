@@ -453,7 +453,7 @@ __global__ __launch_bounds__(64) void k_cells_ref(BlockIn in, GridP gp, CellOut 
     __shared__ int4 s_u[(64 * NS > RMAX) ? 64 * NS : RMAX];
     __shared__ int s_h[hash_ints<NS>()];
     const int k = xcd_item((int)blockIdx.x, in.ncells);
-    if (k < 0) return;
+    if (k < 0 || in.stopped()) return;
     const int v = in.order ? in.order[k] : k;
     cell_ref_body<NS, NF, RMAX>(v, in, &gp, o, want_density, true, s_v, s_ns, s_cc, s_u, s_h);
 }

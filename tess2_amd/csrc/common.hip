@@ -101,46 +101,52 @@ void launch_fill_u32(unsigned *p, size_t n, unsigned v, hipStream_t s)
                        p + n4 * 4, ntail, v);
 }
 
-// particles given as xyz triples -> the padded float4 layout of the kernels
-__global__ void k_pack_points(const float *__restrict__ xyz, int np, float4 *__restrict__ pts)
-{
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= np) return;
-    pts[p] = make_float4(xyz[3 * p], xyz[3 * p + 1], xyz[3 * p + 2], 0.0f);
-}
-
-void launch_pack_points(const float *xyz, int np, float4 *pts, hipStream_t s)
-{
-    if (np <= 0) return;
-    hipLaunchKernelGGL(k_pack_points, dim3((np + 255) / 256), dim3(256), 0, s, xyz, np, pts);
-}
-
-// index ranges of a block held in device memory: every tet vertex in
-// [0, np), every neighbour in [-1, nt), every vert_to_tet entry in [-1, nt);
-// a violation sets bit `bit` of *err
-__global__ void k_check_block(const int4 *__restrict__ tets, int nt, const int *__restrict__ v2t,
-                              int np, unsigned *__restrict__ err, unsigned bit)
+// One pass over a block that the caller keeps in device memory: xyz triples ->
+// padded float4, circumcenters of its tets, zeroed counters, and the index
+// ranges (every tet vertex in [0, np), every neighbour and vert_to_tet entry
+// in [-1, nt)).  A tet is read only once its own indices are in range; a
+// violation stores `token` in *stop, and the kernels behind this one that
+// carry the token return at once.  One word that holds this call's token needs no
+// clearing first, and no wait of the host between check and use.
+__global__ void k_device_block(const float *__restrict__ xyz, int np,
+                               const int4 *__restrict__ tets, int nt,
+                               const int *__restrict__ v2t, float4 *__restrict__ pts,
+                               float4 *__restrict__ cc, unsigned *__restrict__ ctrs,
+                               unsigned *stop, unsigned token)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < C_NCTR) ctrs[i] = 0u;
     bool bad = false;
-    if (i < nt) {
-        const int4 v = tets[2 * i], n = tets[2 * i + 1];
-        bad = (unsigned)v.x >= (unsigned)np || (unsigned)v.y >= (unsigned)np ||
-              (unsigned)v.z >= (unsigned)np || (unsigned)v.w >= (unsigned)np ||
-              n.x < -1 || n.x >= nt || n.y < -1 || n.y >= nt || n.z < -1 || n.z >= nt ||
-              n.w < -1 || n.w >= nt;
+    if (i < np) {
+        pts[i] = make_float4(xyz[3ll * i], xyz[3ll * i + 1], xyz[3ll * i + 2], 0.0f);
+        const int t = v2t[i];
+        bad = t < -1 || t >= nt;
     }
-    if (i < np) bad = bad || v2t[i] < -1 || v2t[i] >= nt;
-    if (bad) atomicOr(err, bit);
+    if (i < nt) {
+        const int4 v = tets[2ll * i], n = tets[2ll * i + 1];
+        const bool out = (unsigned)v.x >= (unsigned)np || (unsigned)v.y >= (unsigned)np ||
+                         (unsigned)v.z >= (unsigned)np || (unsigned)v.w >= (unsigned)np;
+        bad = bad || out || n.x < -1 || n.x >= nt || n.y < -1 || n.y >= nt || n.z < -1 ||
+              n.z >= nt || n.w < -1 || n.w >= nt;
+        if (!out) {
+            const float *a = xyz + 3ll * v.x, *b = xyz + 3ll * v.y, *c = xyz + 3ll * v.z,
+                        *d = xyz + 3ll * v.w;
+            float x, y, z;
+            circumcenter(a[0], a[1], a[2], b[0], b[1], b[2], c[0], c[1], c[2], d[0], d[1], d[2],
+                         x, y, z);
+            cc[i] = make_float4(x, y, z, 0.0f);   // no error bound: volumes do not read it
+        }
+    }
+    if (bad) *stop = token;
 }
 
-void launch_check_block(const int4 *tets, int nt, const int *v2t, int np, unsigned *err,
-                        unsigned bit, hipStream_t s)
+void launch_device_block(const float *xyz, int np, const int4 *tets, int nt, const int *v2t,
+                         float4 *pts, float4 *cc, unsigned *ctrs, unsigned *stop, unsigned token,
+                         hipStream_t s)
 {
-    const int n = nt > np ? nt : np;
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_check_block, dim3((n + 255) / 256), dim3(256), 0, s, tets, nt, v2t, np,
-                       err, bit);
+    const int n = std::max(std::max(np, nt), (int)C_NCTR);
+    hipLaunchKernelGGL(k_device_block, dim3((n + 255) / 256), dim3(256), 0, s, xyz, np, tets, nt,
+                       v2t, pts, cc, ctrs, stop, token);
 }
 
 // per block (blockIdx.y): status histogram (5 codes) and total points of

@@ -144,6 +144,11 @@ struct BlockIn {
     const int *order;    // cells in processing (Morton) order, or nullptr
     int ncells;          // original particles
     int ntets;
+    // set for a block whose indices are checked on the device: its kernels
+    // return at once when *stop holds the token
+    const unsigned *stop;
+    unsigned token;
+    __device__ __forceinline__ bool stopped() const { return stop && *stop == token; }
 };
 
 // 64 consecutive cells (of the Morton order) of one block; base: the position
@@ -278,11 +283,11 @@ void launch_layout(const float4 *pts, int np, int norig, const StageBox &box, co
                    int *v2t, int *tnew, hipStream_t s);
 // circumcenters as xyz triples in the caller's tet numbering
 void launch_unpack_cc(const float4 *cc, const int *tnew, int nt, float *out, hipStream_t s);
-// xyz triples -> float4 (xyz, 0)
-void launch_pack_points(const float *xyz, int np, float4 *pts, hipStream_t s);
-// index-range check of a block in device memory: sets `bit` in *err on a violation
-void launch_check_block(const int4 *tets, int nt, const int *v2t, int np, unsigned *err,
-                        unsigned bit, hipStream_t s);
+// a block in the caller's device memory: float4 particles, circumcenters,
+// zeroed counters; an index out of range stores token in *stop (BlockIn::stop)
+void launch_device_block(const float *xyz, int np, const int4 *tets, int nt, const int *v2t,
+                         float4 *pts, float4 *cc, unsigned *ctrs, unsigned *stop, unsigned token,
+                         hipStream_t s);
 // zero every block's density and count grids; circumcenters of every block
 void launch_block_prep(const BlockIn *ins, const CellOut *outs, int nb, int max_tets,
                        unsigned long long max_grid, bool circumcenters, hipStream_t s);
