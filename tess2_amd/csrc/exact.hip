@@ -231,52 +231,177 @@ __device__ int nearest_f64(float gx, float gy, float gz, const HashP &h,
     return bid;
 }
 
-// search in float with the tie window; returns owner or -1 when undecided
-__device__ int nearest_f32(float gx, float gy, float gz, const HashP &h,
-                           const unsigned *__restrict__ start, const float4 *__restrict__ hp)
+// ---------------------------------------------------------------------------
+// The nearest sites of the 64 points of a tile at once: the wave takes the
+// buckets around the tile's box shell by shell, and every lane meets every
+// particle of a bucket.  The particles are wave-uniform (scalar loads, no
+// per-lane runs), a row of buckets farther from the box than the largest best
+// distance of the lanes is skipped, and nothing diverges.  A lane by itself
+// sees 27 buckets where the tile sees up to 64, but its wave runs the longest
+// of 64 different row sequences, and in a cluster's core it cannot skip the
+// full buckets around its own: 262k particles on 192^3 0.48 -> 0.29 ms, 8 Plummer
+// blocks on 128^3 6.4 -> 1.06, 262k on 63^3 (a tile spans three buckets)
+// 0.108 -> 0.067.  Vector issue bounds it: 13 instructions per particle met.
+// ---------------------------------------------------------------------------
+struct Tile {
+    float lo[3], hi[3];   // box of the tile's points (uniform)
+};
+
+__device__ __forceinline__ float uniform_f(float x)
 {
-    int c[3];
-    home_bucket(gx, gy, gz, h, c);
-    float best = INFINITY, second = INFINITY;
-    int bid = -1;
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x)));
+}
+
+// largest value of the lanes
+template <class T> __device__ __forceinline__ T wave_max(T x)
+{
+    for (int off = 32; off >= 1; off >>= 1) {
+        const T y = __shfl_xor(x, off);
+        x = y > x ? y : x;
+    }
+    return x;
+}
+
+// Calls visit(particle) for every particle that may be the nearest of a lane's
+// point, all lanes together, until no unvisited one can be: reach() is the
+// wave's largest squared distance still to beat (infinite before the first
+// particle), widened by the caller's rounding margin.
+template <class Visit, class Reach>
+__device__ __forceinline__ void tile_search(const Tile &t, const HashP &h,
+                                            const unsigned *__restrict__ start,
+                                            const float4 *__restrict__ hp, Visit visit,
+                                            Reach reach)
+{
+    const int lane = (int)(threadIdx.x & 63);
+    int c0[3], c1[3];
+    home_bucket(t.lo[0], t.lo[1], t.lo[2], h, c0);
+    home_bucket(t.hi[0], t.hi[1], t.hi[2], h, c1);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        c0[a] = __builtin_amdgcn_readfirstlane(c0[a]);
+        c1[a] = __builtin_amdgcn_readfirstlane(c1[a]);
+    }
+    // distance of the box to bucket i's slab on axis a, short of it by the
+    // ~1e-4 of a cell that the float bucket arithmetic can be off
+    const float slack = 0.001f * h.cell;
+    auto gap = [&](int i, int a) {
+        const float b = h.lo[a] + (float)i * h.cell;
+        return fmaxf(0.0f, fmaxf(b - t.hi[a], t.lo[a] - (b + h.cell)) - slack);
+    };
+    auto run = [&](unsigned s0, unsigned s1) {
+        unsigned s = s0;
+        for (; s + 4 <= s1; s += 4) {
+            const float4 p0 = hp[s], p1 = hp[s + 1], p2 = hp[s + 2], p3 = hp[s + 3];
+            visit(p0);
+            visit(p1);
+            visit(p2);
+            visit(p3);
+        }
+        for (; s < s1; ++s) visit(hp[s]);
+    };
     const int rmax = h.dims[0] + h.dims[1] + h.dims[2];
+    double m2 = INFINITY;
+    auto near = [&](float d2, int x) {   // bucket x of a row at squared distance d2
+        const float gx = gap(x, 0);
+        return x < 0 || x >= h.dims[0] || (double)(d2 + gx * gx) <= m2;
+    };
     for (int r = 0; r <= rmax; ++r) {
-        for (int dz = -r; dz <= r; ++dz) {
-            const int z = c[2] + dz;
-            if (z < 0 || z >= h.dims[2]) continue;
-            for (int dy = -r; dy <= r; ++dy) {
-                const int y = c[1] + dy;
-                if (y < 0 || y >= h.dims[1]) continue;
-                const ShellRow sr = shell_row(r, dz, dy, y, z, c[0], h, start);
-                for (int k = 0; k < 2; ++k) {
-                    const unsigned s1 = k ? sr.b1 : sr.a1;
-                    for (unsigned s = k ? sr.b0 : sr.a0; s < s1; ++s) {
-                        const float4 p = hp[s];
-                        const float ex = gx - p.x, ey = gy - p.y, ez = gz - p.z;
-                        const float d = ex * ex + ey * ey + ez * ez;
-                        if (d < best) {
-                            second = best;
-                            best = d;
-                            bid = __float_as_int(p.w);
-                        } else if (d < second) {
-                            second = d;
-                        }
+        // the shell's rows, one per lane: its buckets' runs
+        const int z0 = max(c0[2] - r, 0), z1 = min(c1[2] + r, h.dims[2] - 1);
+        const int y0 = max(c0[1] - r, 0), y1 = min(c1[1] + r, h.dims[1] - 1);
+        const int ny = y1 - y0 + 1, nrow = ny * (z1 - z0 + 1);
+        const int xa = max(c0[0] - r, 0), xb = min(c1[0] + r, h.dims[0] - 1);
+        for (int i0 = 0; i0 < nrow; i0 += 64) {
+            const int i = i0 + lane;
+            unsigned a0 = 0, a1 = 0, b0 = 0, b1 = 0;
+            float d2 = 0.0f;
+            if (i < nrow) {
+                const int z = z0 + i / ny, y = y0 + i % ny;
+                const long long row = ((long long)z * h.dims[1] + y) * h.dims[0];
+                const float gy = gap(y, 1), gz = gap(z, 2);
+                d2 = gy * gy + gz * gz;
+                // the row's end buckets only when they are near enough
+                const bool lo = near(d2, c0[0] - r), hi = near(d2, c1[0] + r);
+                if (r == 0 || z < c0[2] - r + 1 || z > c1[2] + r - 1 || y < c0[1] - r + 1 ||
+                    y > c1[1] + r - 1) {
+                    a0 = start[row + (lo ? xa : min(xa + 1, xb))];
+                    a1 = start[row + (hi ? xb + 1 : max(xb, xa))];
+                } else {
+                    if (lo && c0[0] - r >= 0) {
+                        a0 = start[row + c0[0] - r];
+                        a1 = start[row + c0[0] - r + 1];
+                    }
+                    if (hi && c1[0] + r < h.dims[0]) {
+                        b0 = start[row + c1[0] + r];
+                        b1 = start[row + c1[0] + r + 1];
                     }
                 }
             }
+            unsigned long long todo = __ballot((a0 < a1 || b0 < b1) && (double)d2 <= m2);
+            while (todo) {
+                const int l = __ffsll(todo) - 1;
+                todo &= todo - 1ull;
+                run((unsigned)__builtin_amdgcn_readlane((int)a0, l),
+                    (unsigned)__builtin_amdgcn_readlane((int)a1, l));
+                const unsigned e0 = (unsigned)__builtin_amdgcn_readlane((int)b0, l),
+                               e1 = (unsigned)__builtin_amdgcn_readlane((int)b1, l);
+                if (e0 < e1) run(e0, e1);
+            }
         }
-        const float lb = ((float)r - 0.001f) * h.cell;
-        if (bid >= 0 && r > 0 && lb * lb > best * 1.0001f + 1e-30f) break;
+        m2 = (double)reach();
+        // every bucket beyond shell r is at least r cells from the box
+        const double lb = ((double)r - 0.001) * (double)h.cell;
+        if (r > 0 && lb * lb > m2) break;
     }
+}
+
+// on: this lane has a point (the others see the same particles and are ignored)
+__device__ __forceinline__ int tile_nearest_f32(float gx, float gy, float gz, bool on,
+                                                const Tile &t, const HashP &h,
+                                                const unsigned *__restrict__ start,
+                                                const float4 *__restrict__ hp)
+{
+    float best = INFINITY, second = INFINITY;
+    int bid = -1;
+    tile_search(
+        t, h, start, hp,
+        [&](const float4 p) {
+            const float ex = gx - p.x, ey = gy - p.y, ez = gz - p.z;
+            const float d = ex * ex + ey * ey + ez * ez;
+            second = fminf(second, fmaxf(best, d));
+            bid = d < best ? __float_as_int(p.w) : bid;
+            best = fminf(best, d);
+        },
+        [&] { return wave_max(on ? best * 1.0001f + 1e-30f : 0.0f); });
     // decided only if the runner-up is clearly farther (32 ulp window) and
-    // nothing underflowed
+    // nothing underflowed, or the point coincides with a site: exact in float
     const float tau = 32.0f * 5.9604645e-8f;
     if (bid >= 0 && best > 1e-30f && second > best * (1.0f + tau)) return bid;
-    if (bid >= 0 && best == 0.0f && second > 1e-30f) {
-        // the grid point coincides with a site: exact in float
-        return bid;
-    }
+    if (bid >= 0 && best == 0.0f && second > 1e-30f) return bid;
     return -1;
+}
+
+__device__ __forceinline__ int tile_nearest_f64(float gx, float gy, float gz, bool on,
+                                                const Tile &t, const HashP &h,
+                                                const unsigned *__restrict__ start,
+                                                const float4 *__restrict__ hp)
+{
+    double best = 1e300;
+    int bid = 0x7fffffff;
+    tile_search(
+        t, h, start, hp,
+        [&](const float4 p) {
+            const double ex = (double)gx - (double)p.x;
+            const double ey = (double)gy - (double)p.y;
+            const double ez = (double)gz - (double)p.z;
+            const double d = ex * ex + ey * ey + ez * ez;
+            const int id = __float_as_int(p.w);
+            const bool b = better64(d, id, best, bid);
+            best = b ? d : best;
+            bid = b ? id : bid;
+        },
+        [&] { return wave_max(on ? best * (1.0 + 1e-9) + 1e-300 : 0.0); });
+    return bid;
 }
 
 // one thread per block grid point; a 64-lane wave covers a 4x4x4 tile
@@ -311,9 +436,20 @@ __global__ __launch_bounds__(256) void k_owner(GridP gp, HashP h,
     if (!in_block && on_grid) owner[lidx] = -1;
     int o = -1;
     bool failed = false;
-    if (in_block && on_grid) {
-        if (prec == 0) o = nearest_f32(px, py, pz, h, start, hp);
-        failed = o < 0 && prec == 0;
+    const bool on = in_block && on_grid;
+    if (__ballot(on)) {
+        Tile t;
+        const int g0[3] = {tx * 4, ty * 4, tz * 4};
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            t.lo[a] = uniform_f(idx2phys1(gp.bmin_idx[a] + g0[a], gp.step[a], gp.gmin[a]));
+            t.hi[a] = uniform_f(idx2phys1(gp.bmin_idx[a] + min(g0[a] + 3, gp.bnum_idx[a] - 1),
+                                          gp.step[a], gp.gmin[a]));
+        }
+        if (prec == 0) o = tile_nearest_f32(px, py, pz, on, t, h, start, hp);
+        else o = tile_nearest_f64(px, py, pz, on, t, h, start, hp);
+        if (!on) o = -1;
+        failed = on && o < 0 && prec == 0;
     }
     // FP32 filter failures go to a queue that k_owner_deferred searches in
     // FP64 with full waves: searched here, one failing lane would hold its
@@ -398,9 +534,9 @@ void launch_owner(const GridP &gp, const HashP &h, const unsigned *start, const 
               tz = (gp.bnum_idx[2] + 3) / 4;
     const int ntiles = tx * ty * tz;
     if (ntiles <= 0) return;
-    hipLaunchKernelGGL(k_owner, dim3((ntiles + 3) / 4), dim3(256), 0, s, gp, h, start, hp, owner,
-                       prec, ctrs, tx, ty, ntiles, status, npts, ncells, npts_tab, stex_tab,
-                       defq, prec == 0 ? defq_cap : 0u);
+    hipLaunchKernelGGL(k_owner, dim3((ntiles + 3) / 4), dim3(256),
+                       0, s, gp, h, start, hp, owner, prec, ctrs, tx, ty, ntiles, status, npts,
+                       ncells, npts_tab, stex_tab, defq, prec == 0 ? defq_cap : 0u);
     if (prec == 0 && defq_cap > 0) {
         const unsigned nblk = defq_cap / 256 + 1;
         hipLaunchKernelGGL(k_owner_deferred, dim3(nblk < 2048 ? nblk : 2048), dim3(256), 0, s,
