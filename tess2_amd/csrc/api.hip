@@ -89,8 +89,8 @@ struct DevBlock {
     int *status_ex = nullptr;                // [ncells] deposit decision
     unsigned *exflags = nullptr;             // [3 * ncells bytes] its per-vertex flags
     HashP hash{};
-    unsigned *hstart = nullptr, *hfill = nullptr, *hsums = nullptr;
-    int *hbk = nullptr;
+    unsigned *hstart = nullptr, *hsums = nullptr;
+    int2 *hbk = nullptr;                     // each particle's bucket, and rank in it
     float4 *hsorted = nullptr;
     int *hkey = nullptr;                     // [np] home key of each particle (several blocks)
     std::vector<int> ghost_gid, ghost_cell;  // home of each ghost, when given
@@ -170,7 +170,7 @@ struct tess2_ctx {
     std::unordered_map<void *, size_t> live;             // bytes of every buffer in use
     std::vector<std::pair<void *, size_t>> spare;        // oldest first
     size_t spare_bytes = 0;
-    double *d_gpart = nullptr;                           // partial grid sums, 1024 per block
+    RunPart *d_gpart = nullptr;                          // partial statistics, RUN_PARTS a block
     // exact assignment over several blocks: every particle's home key
     // (rank << 23 | cell), and the per-rank npts / deposit-status tables
     bool homes_ok = false;
@@ -342,7 +342,6 @@ static void free_block(tess2_ctx *c, DevBlock &b)
     dfree(c, b.status_ex);
     dfree(c, b.exflags);
     dfree(c, b.hstart);
-    dfree(c, b.hfill);
     dfree(c, b.hsums);
     dfree(c, b.hbk);
     dfree(c, b.hsorted);
@@ -765,10 +764,9 @@ static int stage_block(tess2_ctx *c, const tess2_block_t &hb, DevBlock &d, bool 
     if (layout && (r = lay_out(c, d))) return r;
     d.slow_cap = (unsigned)std::max(1024, d.norig / 32);
     if ((r = dalloc(c, &d.slow, d.slow_cap))) return r;
-    // bucket hash over the particle bounding box, about one particle
-    // per bucket (two: 262k particles on 192^3 0.313 against 0.285 ms, 8
-    // Plummer blocks on 256^3 1.79 against 1.22); at most 2^24 - 1024 buckets, so that the bucket scan
-    // needs at most 16384 blocks of 1024 (k_scan_sums' limit)
+    // bucket hash over the particle bounding box, about one particle per
+    // bucket (two: 262k particles on 192^3 0.313 against 0.285 ms, 8 Plummer
+    // blocks on 256^3 1.79 against 1.22); at most 2^24 - 1024 buckets
     double vol = 1.0;
     for (int i = 0; i < 3; ++i) vol *= std::max((double)hi[i] - lo[i], 1e-12);
     double cell = std::cbrt(vol / std::max(d.np, 1));
@@ -786,8 +784,8 @@ static int stage_block(tess2_ctx *c, const tess2_block_t &hb, DevBlock &d, bool 
         d.hash.dims[i] = (int)((hi[i] - lo[i]) / cell) + 1;
     }
     const size_t nbk = (size_t)d.hash.dims[0] * d.hash.dims[1] * d.hash.dims[2];
-    if ((r = dalloc(c, &d.hstart, nbk + 1)) || (r = dalloc(c, &d.hfill, nbk + 1)) ||
-        (r = dalloc(c, &d.hsums, (nbk + 1 + 1023) / 1024)) ||
+    if ((r = dalloc(c, &d.hstart, nbk + 1)) ||
+        (r = dalloc(c, &d.hsums, scan_sums_words(nbk + 1))) ||
         (r = dalloc(c, &d.hbk, (size_t)d.np)) || (r = dalloc(c, &d.hsorted, (size_t)d.np)) ||
         (r = dalloc(c, &d.status_ex, (size_t)d.norig)) ||
         (r = dalloc(c, &d.exflags, ((size_t)d.norig * 3 + 3) / 4)))
@@ -864,7 +862,7 @@ static int stage_blocks(tess2_ctx *c, const tess2_block_t *blocks, int nblocks, 
         if ((r = dalloc(c, &c->d_ins, (size_t)nblocks)) || (r = dalloc(c, &c->d_gps, (size_t)nblocks)) ||
             (r = dalloc(c, &c->d_outs, (size_t)nblocks)) || (r = dalloc(c, &c->d_router, 1)) ||
             (r = dalloc(c, &c->d_queue, 16)) || (r = dalloc(c, &c->d_stats, (size_t)nblocks)) ||
-            (r = dalloc(c, &c->d_gpart, (size_t)nblocks * 1024)))
+            (r = dalloc(c, &c->d_gpart, (size_t)nblocks * RUN_PARTS)))
             return r;
         // counters and statistics of all blocks: one device array, one pinned
         // host copy (so that the copy can sit in a captured graph)
@@ -1194,12 +1192,11 @@ static int prepare_run(tess2_ctx *c, const RunArgs &a)
 }
 
 // geometry, then scan and deposit, of all cells of a scan run, at most
-// PLANE_TILES tiles at a time
+// PLANE_TILES tiles at a time (planes.nbig is zero on entry)
 template <bool MULTI>
 static void enqueue_split(tess2_ctx *c, CellSet<MULTI> set, int ntiles, hipStream_t s)
 {
     const int chunks = (ntiles + PLANE_TILES - 1) / PLANE_TILES;
-    launch_fill_u32(c->planes.nbig, (size_t)chunks, 0u, s);
     PlaneBuf pb = c->planes;
     for (int k = 0; k < chunks; ++k, ++pb.nbig) {
         set.tile0 = k * PLANE_TILES;
@@ -1233,8 +1230,11 @@ static int enqueue_kernels(tess2_ctx *c, const RunArgs &a)
     hipStream_t s = c->stream;
     const bool ev = !c->in_capture;
 
-    // phase A: clear per-block outputs and counters, circumcenters
-    launch_fill_u32(reinterpret_cast<unsigned *>(c->d_stats), sizeof(BlockStats) / 4 * nb, 0u, s);
+    // phase A: clear per-block outputs and counters, circumcenters, and the
+    // arrays that phase B adds to
+    const bool split = a.alg == TESS2_DENSE_TESS && !exact &&
+                       split_cells(c, a.eps, nb, c->blocks[0].norig);
+    const int ntiles = nb > 1 ? c->ntiles : (c->blocks[0].norig + CELL_TILE - 1) / CELL_TILE;
     {
         int mt = 0;
         unsigned long long mg = 0;
@@ -1242,7 +1242,23 @@ static int enqueue_kernels(tess2_ctx *c, const RunArgs &a)
             mt = std::max(mt, d.nt);
             mg = std::max<unsigned long long>(mg, d.ngrid);
         }
-        launch_block_prep(c->d_ins, c->d_outs, nb, mt, mg, a.alg == TESS2_DENSE_TESS, s);
+        ZeroList z{};
+        z.p[0] = reinterpret_cast<unsigned *>(c->d_stats);
+        z.n[0] = sizeof(BlockStats) / 4 * (unsigned long long)nb;
+        if (split) {
+            z.p[1] = c->planes.nbig;
+            z.n[1] = (unsigned long long)((ntiles + PLANE_TILES - 1) / PLANE_TILES);
+        }
+        if (exact && nb == 1) {
+            const DevBlock &d = c->blocks[0];
+            z.p[1] = d.hstart;
+            z.n[1] = (unsigned long long)d.hash.dims[0] * d.hash.dims[1] * d.hash.dims[2] + 1;
+            z.p[2] = d.exflags;
+            z.n[2] = ((unsigned long long)d.norig * 3 + 3) / 4;
+            z.p[3] = (unsigned *)d.npts;
+            z.n[3] = (unsigned long long)d.norig;
+        }
+        launch_run_prep(c->d_ins, c->d_outs, nb, a.alg == TESS2_DENSE_TESS ? mt : 0, mg, z, s);
     }
     // phase B: the estimator
     if (exact) {
@@ -1264,11 +1280,18 @@ static int enqueue_kernels(tess2_ctx *c, const RunArgs &a)
             const GridP &gp = c->h_gps[k];
             // volume() as the reference computes it
             if (a.want_vol && !(multi && c->cell_kernel < 0)) launch_volumes(c, in, c->h_outs[k], s);
-            launch_hash_build(d.pts, d.np, d.hash, d.hstart, d.hfill, d.hsums, d.hbk, d.hsorted,
+            if (multi) {   // one block's are zero from the start
+                launch_fill_u32(d.hstart, (size_t)d.hash.dims[0] * d.hash.dims[1] *
+                                d.hash.dims[2] + 1, 0u, s);
+                if (d.norig > 0) {
+                    launch_fill_u32((unsigned *)d.exflags, ((size_t)d.norig * 3 + 3) / 4, 0u, s);
+                    launch_fill_u32((unsigned *)d.npts, (size_t)d.norig, 0u, s);
+                }
+            }
+            launch_hash_build(d.pts, d.np, d.hash, d.hstart, d.hsums, d.hbk, d.hsorted,
                               multi ? d.hkey : nullptr, s);
             launch_exact_status(in, gp, d.status_ex, a.precision, d.ctrs,
                                 reinterpret_cast<unsigned char *>(d.exflags), s);
-            if (multi && d.norig > 0) launch_fill_u32((unsigned *)d.npts, (size_t)d.norig, 0u, s);
         }
         if (ev) HIPCHK(c, hipEventRecord(c->ev_k0, s));
         for (int k = 0; k < nb; ++k) {
@@ -1293,14 +1316,14 @@ static int enqueue_kernels(tess2_ctx *c, const RunArgs &a)
             launch_cic(c->h_ins[k], c->h_gps[k], c->h_outs[k], nb > 1 ? c->d_router : nullptr, k,
                        s);
         if (ev) HIPCHK(c, hipEventRecord(c->ev_k1, s));
-    } else if (split_cells(c, a.eps, nb, c->blocks[0].norig)) {
+    } else if (split) {
         if (ev) HIPCHK(c, hipEventRecord(c->ev_k0, s));
         if (nb == 1)
             enqueue_split(c, CellSet<false>{c->h_ins[0], c->h_outs[0], c->d_gps, 0, 0},
-                          (c->blocks[0].norig + CELL_TILE - 1) / CELL_TILE, s);
+                          ntiles, s);
         else
             enqueue_split(c, CellSet<true>{c->d_ins, c->d_outs, c->d_gps, c->d_router, c->d_tiles,
-                                           0, 0}, c->ntiles, s);
+                                           0, 0}, ntiles, s);
         if (ev) HIPCHK(c, hipEventRecord(c->ev_k1, s));
         if (nb == 1) launch_cells_ref_slow(c->h_ins[0], c->h_gps[0], c->h_outs[0], 1, s);
         else launch_cells_ref_slow_batched(c->d_ins, c->d_router, 1, s);
@@ -1349,8 +1372,8 @@ static int enqueue_kernels(tess2_ctx *c, const RunArgs &a)
         mcells = std::max(mcells, d.norig);
         mgrid = std::max<unsigned long long>(mgrid, d.ngrid);
     }
-    launch_fold(c->d_outs, c->d_gps, nb, mcap, mfold, mgrid, sovf, smid, s);
-    launch_stats(c->d_outs, c->d_gpart, nb, mcells, mgrid, s);
+    launch_fold(c->d_outs, c->d_gps, nb, mcap, mfold, sovf, smid, s);
+    launch_run_finish(c->d_outs, c->d_gps, c->d_gpart, nb, mcells, mgrid, s);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipMemcpyAsync(c->h_stats, c->d_stats, sizeof(BlockStats) * nb,
                              hipMemcpyDeviceToHost, s));

@@ -30,51 +30,58 @@ void launch_circumcenters(const float4 *pts, const int4 *tets, int ntets, float4
                        ntets, cc);
 }
 
-// circumcenters of every staged block, block = blockIdx.y
-__global__ void k_circumcenters_blocks(const BlockIn *__restrict__ ins)
+// What a run starts with, in one launch: circumcenters of every staged block
+// (workgroups below bt of row blockIdx.y = block), its density and count grids
+// cleared, and up to four more arrays zeroed (first row).  Both halves are
+// streams; apart they were three to six launches of ~4 us each (4,000 cells,
+// exact assignment, 49^3, whole run with the fused last pass: 185 against
+// 156 us).
+__global__ __launch_bounds__(256) void k_run_prep(const BlockIn *__restrict__ ins,
+                                                  const CellOut *__restrict__ outs, int bt,
+                                                  ZeroList z)
 {
-    const BlockIn &in = ins[blockIdx.y];
-    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < in.ntets;
-         t += gridDim.x * blockDim.x) {
-        const int4 vv = in.tets[2 * t];
-        const float4 a = in.pts[vv.x], b = in.pts[vv.y], c = in.pts[vv.z], d = in.pts[vv.w];
-        float x, y, z;
-        circumcenter(a.x, a.y, a.z, b.x, b.y, b.z, c.x, c.y, c.z, d.x, d.y, d.z, x, y, z);
-        const float e = circumcenter_err(a.x, a.y, a.z, b.x, b.y, b.z, c.x, c.y, c.z, d.x, d.y,
-                                         d.z, x, y, z);
-        const_cast<float4 *>(in.cc)[t] = make_float4(x, y, z, e);   // read-only downstream
+    if ((int)blockIdx.x < bt) {
+        const BlockIn &in = ins[blockIdx.y];
+        for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < in.ntets; t += bt * blockDim.x) {
+            const int4 vv = in.tets[2 * t];
+            const float4 a = in.pts[vv.x], b = in.pts[vv.y], c = in.pts[vv.z], d = in.pts[vv.w];
+            float x, y, z0;
+            circumcenter(a.x, a.y, a.z, b.x, b.y, b.z, c.x, c.y, c.z, d.x, d.y, d.z, x, y, z0);
+            const float e = circumcenter_err(a.x, a.y, a.z, b.x, b.y, b.z, c.x, c.y, c.z, d.x,
+                                             d.y, d.z, x, y, z0);
+            const_cast<float4 *>(in.cc)[t] = make_float4(x, y, z0, e);   // read-only downstream
+        }
+        return;
     }
-}
-
-// zero the density and count grids of every block, block = blockIdx.y
-__global__ void k_clear_grids(const CellOut *__restrict__ outs)
-{
     const CellOut &o = outs[blockIdx.y];
     const unsigned long long n = o.ngrid, n4 = n / 4;
-    const unsigned long long stride = (unsigned long long)gridDim.x * blockDim.x;
-    const unsigned long long i0 = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const uint4 z = make_uint4(0u, 0u, 0u, 0u);
+    const unsigned long long stride = (unsigned long long)(gridDim.x - bt) * blockDim.x;
+    const unsigned long long i0 = (unsigned long long)(blockIdx.x - bt) * blockDim.x + threadIdx.x;
+    const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
     for (unsigned long long i = i0; i < n4; i += stride) {
-        reinterpret_cast<uint4 *>(o.density)[i] = z;
-        reinterpret_cast<uint4 *>(o.count)[i] = z;
+        reinterpret_cast<uint4 *>(o.density)[i] = zero;
+        reinterpret_cast<uint4 *>(o.count)[i] = zero;
     }
     if (i0 < n - n4 * 4) {
         o.density[n4 * 4 + i0] = 0.0f;
         o.count[n4 * 4 + i0] = 0u;
     }
+    if (blockIdx.y == 0)
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            for (unsigned long long i = i0; i < z.n[k]; i += stride) z.p[k][i] = 0u;
 }
 
-void launch_block_prep(const BlockIn *ins, const CellOut *outs, int nb, int max_tets,
-                       unsigned long long max_grid, bool circumcenters, hipStream_t s)
+void launch_run_prep(const BlockIn *ins, const CellOut *outs, int nb, int max_tets,
+                     unsigned long long max_grid, const ZeroList &z, hipStream_t s)
 {
     if (nb <= 0) return;
-    unsigned bg = (unsigned)std::min<unsigned long long>(2048, (max_grid / 4 + 255) / 256);
-    if (bg == 0) bg = 1;
-    hipLaunchKernelGGL(k_clear_grids, dim3(bg, nb), dim3(256), 0, s, outs);
-    if (circumcenters && max_tets > 0) {
-        const unsigned bt = (unsigned)std::min(16384, (max_tets + 255) / 256);
-        hipLaunchKernelGGL(k_circumcenters_blocks, dim3(bt, nb), dim3(256), 0, s, ins);
-    }
+    unsigned long long most = max_grid / 4;
+    for (int k = 0; k < 4; ++k) most = std::max<unsigned long long>(most, z.n[k]);
+    const unsigned bg = (unsigned)std::max<unsigned long long>(
+        1, std::min<unsigned long long>(2048, (most + 255) / 256));
+    const unsigned bt = (unsigned)std::min(16384, (max_tets + 255) / 256);
+    hipLaunchKernelGGL(k_run_prep, dim3(bt + bg, nb), dim3(256), 0, s, ins, outs, (int)bt, z);
 }
 
 __global__ void k_fill_u32(uint4 *__restrict__ p4, size_t n4, unsigned *__restrict__ tail,
@@ -149,16 +156,113 @@ void launch_device_block(const float *xyz, int np, const int4 *tets, int nt, con
                        v2t, pts, cc, ctrs, stop, token);
 }
 
-// per block (blockIdx.y): status histogram (5 codes) and total points of
-// deposited cells
-__global__ __launch_bounds__(256) void k_cell_stats(const CellOut *__restrict__ outs)
+// ---------------------------------------------------------------------------
+// The end of a run, after the fold of points with three and more
+// contributions: the points with exactly two (the common case: a point on
+// the face between two cells) hold both next to the point and are added here,
+// in the order the sort would give the pair (the second first unless its key
+// is larger); sum and maximum of the density; cells per status and points
+// of deposited cells.  Each workgroup leaves a record and k_run_stats combines
+// them in a fixed order, so that the sum is the same on every run, without
+// an atomic per workgroup on the block's counters.  A stream over count and
+// density, bound by it and by the lines of first and second that hold pairs
+// (16.8M points, 2M cells: 88 us; as passes of their own, pairs 78, sums 55
+// and cells 21).  Four points per lane and iteration: a small grid is then
+// over in one (117,000 points: 5 us, 8 with sixteen).
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void k_run_finish(const CellOut *__restrict__ outs,
+                                                    const GridP *__restrict__ gps,
+                                                    RunPart *__restrict__ part, int bg)
 {
-    // cells per status counted by ballots (wave-uniform counters), points of
-    // deposited cells summed per lane; one atomic per counter per workgroup
+    __shared__ double s_acc[4];
+    __shared__ float s_mx[4];
     __shared__ unsigned long long s_c[4][6];
     const CellOut &o = outs[blockIdx.y];
+    RunPart &out = part[(size_t)blockIdx.y * RUN_PARTS + blockIdx.x];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    if ((int)blockIdx.x < bg) {
+        const double dd = (double)gps[blockIdx.y].div;
+        // 16-byte loads, four independent partial sums per lane (the grid
+        // arrays are 256-byte aligned allocations); the last n mod 4 points
+        // go to the first lanes of workgroup 0
+        const unsigned long long n = o.ngrid, n4 = n >> 2;
+        const unsigned *__restrict__ count = o.count;
+        const uint2 *__restrict__ first = o.first, *__restrict__ second = o.second;
+        float *__restrict__ density = o.density;
+        auto pair = [&](uint2 f, uint2 q) {
+            const bool sw = q.x > f.x;
+            const unsigned m0 = sw ? f.y : q.y, m1 = sw ? q.y : f.y;
+            const float x = (float)(0.0 + (double)__uint_as_float(m0) / dd);
+            return (float)((double)x + (double)__uint_as_float(m1) / dd);
+        };
+        double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
+        float mx = 0.0f;
+        unsigned np = 0;
+        for (unsigned long long i = (unsigned long long)blockIdx.x * 256 + threadIdx.x; i < n4;
+             i += (unsigned long long)bg * 256) {
+            const uint4 c4 = reinterpret_cast<const uint4 *>(count)[i];
+            const float4 x4 = reinterpret_cast<const float4 *>(density)[i];
+            const unsigned c[4] = {c4.x, c4.y, c4.z, c4.w};
+            float x[4] = {x4.x, x4.y, x4.z, x4.w};
+            uint2 f[4], q[4];
+            bool any = false;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                f[k] = q[k] = make_uint2(0u, 0u);
+                if (c[k] == 2u) {
+                    f[k] = first[4 * i + k];
+                    q[k] = second[4 * i + k];
+                }
+                any |= c[k] == 2u;
+                np += c[k] >= 2u ? 1u : 0u;
+            }
+            if (any) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) x[k] = c[k] == 2u ? pair(f[k], q[k]) : x[k];
+                reinterpret_cast<float4 *>(density)[i] = make_float4(x[0], x[1], x[2], x[3]);
+            }
+            a0 += (double)x[0];
+            a1 += (double)x[1];
+            a2 += (double)x[2];
+            a3 += (double)x[3];
+            mx = fmaxf(mx, fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])));
+        }
+        if (blockIdx.x == 0 && threadIdx.x < (unsigned)(n & 3ull)) {
+            const unsigned long long g = (n4 << 2) + threadIdx.x;
+            float x = density[g];
+            if (count[g] == 2u) {
+                x = pair(first[g], second[g]);
+                density[g] = x;
+            }
+            np += count[g] >= 2u ? 1u : 0u;
+            a0 += (double)x;
+            mx = fmaxf(mx, x);
+        }
+        double acc = (a0 + a1) + (a2 + a3);
+        for (int off = 32; off >= 1; off >>= 1) {
+            acc += __shfl_xor(acc, off);
+            mx = fmaxf(mx, __shfl_xor(mx, off));
+            np += __shfl_xor(np, off);
+        }
+        if (lane == 0) {
+            s_acc[w] = acc;
+            s_mx[w] = mx;
+            s_c[w][0] = np;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            out.sum = ((s_acc[0] + s_acc[1]) + s_acc[2]) + s_acc[3];
+            out.mx = fmaxf(fmaxf(s_mx[0], s_mx[1]), fmaxf(s_mx[2], s_mx[3]));
+            out.pairs = (unsigned)(s_c[0][0] + s_c[1][0] + s_c[2][0] + s_c[3][0]);
+        }
+        if (threadIdx.x < 6) out.c[threadIdx.x] = 0;
+        return;
+    }
+    // cells per status counted by ballots (wave-uniform counters), points of
+    // deposited cells summed per lane
+    const int b = (int)blockIdx.x - bg, nbc = (int)gridDim.x - bg;
     unsigned long long c[5] = {0, 0, 0, 0, 0}, np = 0;
-    for (int base = blockIdx.x * blockDim.x; base < o.ncells; base += gridDim.x * blockDim.x) {
+    for (int base = b * 256; base < o.ncells; base += nbc * 256) {
         const int i = base + threadIdx.x;
         int s = -1;
         if (i < o.ncells) {
@@ -169,8 +273,7 @@ __global__ __launch_bounds__(256) void k_cell_stats(const CellOut *__restrict__ 
         for (int k = 0; k < 5; ++k) c[k] += (unsigned long long)__popcll(__ballot(s == k));
     }
     for (int off = 32; off >= 1; off >>= 1) np += __shfl_xor(np, off);
-    const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) {
+    if (lane == 0) {
 #pragma unroll
         for (int k = 0; k < 5; ++k) s_c[w][k] = c[k];
         s_c[w][5] = np;
@@ -178,84 +281,66 @@ __global__ __launch_bounds__(256) void k_cell_stats(const CellOut *__restrict__ 
     __syncthreads();
     if (threadIdx.x < 6) {
         const int k = threadIdx.x;
-        const unsigned long long x = s_c[0][k] + s_c[1][k] + s_c[2][k] + s_c[3][k];
-        if (x) atomicAdd(&o.st->cstat[k], x);
+        out.c[k] = s_c[0][k] + s_c[1][k] + s_c[2][k] + s_c[3][k];
+    }
+    if (threadIdx.x == 6) {
+        out.sum = 0.0;
+        out.mx = 0.0f;
+        out.pairs = 0u;
     }
 }
 
-// per block (blockIdx.y): sum (double) and max of the density grid.  The
-// sum is reduced in a fixed order (lanes, waves, then workgroups in
-// k_grid_final) so that it is the same on every run.
-constexpr int GRID_PARTS = 1024;
-
-__global__ __launch_bounds__(256) void k_grid_stats(const CellOut *__restrict__ outs,
-                                                    double *__restrict__ part)
+// one workgroup per block: its records into its statistics, four lanes' worth
+// of a fixed tree per record
+__global__ __launch_bounds__(256) void k_run_stats(const CellOut *__restrict__ outs,
+                                                   const RunPart *__restrict__ part, int nparts)
 {
-    __shared__ double s_acc[4];
-    const CellOut &o = outs[blockIdx.y];
-    // 16-byte loads, four independent partial sums per lane (the grid
-    // arrays are 256-byte aligned allocations); the last n mod 4 points
-    // go to the first lanes of workgroup 0
-    const unsigned long long n = o.ngrid, n4 = n >> 2;
-    const float4 *d4 = reinterpret_cast<const float4 *>(o.density);
-    double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-    float mx = 0.0f;
-#pragma unroll 4
-    for (unsigned long long i = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x; i < n4;
-         i += (unsigned long long)gridDim.x * blockDim.x) {
-        const float4 x = d4[i];
-        a0 += (double)x.x;
-        a1 += (double)x.y;
-        a2 += (double)x.z;
-        a3 += (double)x.w;
-        mx = fmaxf(mx, fmaxf(fmaxf(x.x, x.y), fmaxf(x.z, x.w)));
+    __shared__ RunPart s_p[256];
+    RunPart a{};
+    for (int k = threadIdx.x; k < nparts; k += 256) {
+        const RunPart &q = part[(size_t)blockIdx.x * RUN_PARTS + k];
+        a.sum += q.sum;
+        a.mx = fmaxf(a.mx, q.mx);
+        a.pairs += q.pairs;
+#pragma unroll
+        for (int i = 0; i < 6; ++i) a.c[i] += q.c[i];
     }
-    if (blockIdx.x == 0 && threadIdx.x < (unsigned)(n & 3ull)) {
-        const float x = o.density[(n4 << 2) + threadIdx.x];
-        a0 += (double)x;
-        mx = fmaxf(mx, x);
+    s_p[threadIdx.x] = a;
+    for (int off = 128; off >= 1; off >>= 1) {
+        __syncthreads();
+        if ((int)threadIdx.x < off) {
+            const RunPart &q = s_p[threadIdx.x + off];
+            a.sum += q.sum;
+            a.mx = fmaxf(a.mx, q.mx);
+            a.pairs += q.pairs;
+#pragma unroll
+            for (int i = 0; i < 6; ++i) a.c[i] += q.c[i];
+            s_p[threadIdx.x] = a;
+        }
     }
-    double acc = (a0 + a1) + (a2 + a3);
-    for (int off = 32; off >= 1; off >>= 1) {
-        acc += __shfl_xor(acc, off);
-        mx = fmaxf(mx, __shfl_xor(mx, off));
+    if (threadIdx.x == 0) {
+        BlockStats &st = *outs[blockIdx.x].st;
+        st.gsum = a.sum;
+        st.gmax = __float_as_uint(a.mx);
+        st.ctrs[C_PAIRS] = a.pairs;
+        for (int i = 0; i < 6; ++i) st.cstat[i] = a.c[i];
     }
-    if ((threadIdx.x & 63) == 0) {
-        s_acc[threadIdx.x >> 6] = acc;
-        if (mx != 0.0f) atomicMax(&o.st->gmax, __float_as_uint(mx));   // order-free
-    }
-    __syncthreads();
-    if (threadIdx.x == 0)
-        part[blockIdx.y * GRID_PARTS + blockIdx.x] = ((s_acc[0] + s_acc[1]) + s_acc[2]) + s_acc[3];
 }
 
-__global__ __launch_bounds__(256) void k_grid_final(const CellOut *__restrict__ outs,
-                                                    const double *__restrict__ part, int nparts)
-{
-    __shared__ double s[GRID_PARTS];
-    for (int k = threadIdx.x; k < nparts; k += blockDim.x) s[k] = part[blockIdx.x * GRID_PARTS + k];
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    double acc = 0.0;
-    for (int k = 0; k < nparts; ++k) acc += s[k];
-    outs[blockIdx.x].st->gsum = acc;
-}
-
-void launch_stats(const CellOut *outs, double *part, int nb, int max_cells,
-                  unsigned long long max_grid, hipStream_t s)
+void launch_run_finish(const CellOut *outs, const GridP *gps, RunPart *part, int nb, int max_cells,
+                       unsigned long long max_grid, hipStream_t s)
 {
     if (nb <= 0) return;
-    // about 16 items per lane, at most GRID_PARTS workgroups per block (a
+    // four items per lane, at most RUN_PARTS workgroups per block (a
     // single block fills the chip; many blocks share it)
-    const long long cap = std::max<long long>(16, GRID_PARTS / std::max(1, nb / 4));
-    unsigned bc = (unsigned)std::min<long long>(cap, ((long long)max_cells + 4095) / 4096);
-    unsigned bg = (unsigned)std::min<unsigned long long>(cap, (max_grid + 4095) / 4096);
-    if (bc == 0) bc = 1;
-    if (bg == 0) bg = 1;
-    hipLaunchKernelGGL(k_cell_stats, dim3(bc, nb), dim3(256), 0, s, outs);
-    hipLaunchKernelGGL(k_grid_stats, dim3(bg, nb), dim3(256), 0, s, outs, part);
-    hipLaunchKernelGGL(k_grid_final, dim3(nb), dim3(256), 0, s, outs, (const double *)part,
-                       (int)bg);
+    const long long cap = std::max<long long>(16, RUN_PARTS / std::max(1, nb / 4));
+    const unsigned bc = (unsigned)std::max<long long>(
+        1, std::min<long long>(cap / 8, ((long long)max_cells + 1023) / 1024));
+    const unsigned bg = (unsigned)std::max<unsigned long long>(
+        1, std::min<unsigned long long>(cap - cap / 8, (max_grid + 1023) / 1024));
+    hipLaunchKernelGGL(k_run_finish, dim3(bg + bc, nb), dim3(256), 0, s, outs, gps, part, (int)bg);
+    hipLaunchKernelGGL(k_run_stats, dim3(nb), dim3(256), 0, s, outs, (const RunPart *)part,
+                       (int)(bg + bc));
 }
 
 }  // namespace t2

@@ -38,104 +38,44 @@ __device__ __forceinline__ int bucket_of(float4 p, const HashP &h)
     return (c[2] * h.dims[1] + c[1]) * h.dims[0] + c[0];
 }
 
+// bucket of every particle and its rank there (in no set order: the searches
+// decide ties by id)
 __global__ void k_hash_count(const float4 *__restrict__ pts, int np, HashP h,
-                             unsigned *__restrict__ cnt, int *__restrict__ bk)
+                             unsigned *__restrict__ cnt, int2 *__restrict__ bk)
 {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= np) return;
     const int b = bucket_of(pts[p], h);
-    bk[p] = b;
-    atomicAdd(&cnt[b], 1u);
-}
-
-// exclusive scan in three passes (1024 elements per block)
-__global__ void k_scan_local(const unsigned *__restrict__ in, unsigned *__restrict__ out,
-                             unsigned *__restrict__ sums, int n)
-{
-    __shared__ unsigned s[1024];
-    const int i = blockIdx.x * 1024 + threadIdx.x;
-    const unsigned x = i < n ? in[i] : 0u;
-    s[threadIdx.x] = x;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-        const unsigned y = threadIdx.x >= (unsigned)off ? s[threadIdx.x - off] : 0u;
-        __syncthreads();
-        s[threadIdx.x] += y;
-        __syncthreads();
-    }
-    if (i < n) out[i] = s[threadIdx.x] - x;
-    if (threadIdx.x == 1023) sums[blockIdx.x] = s[1023];
-}
-
-__global__ void k_scan_sums(unsigned *__restrict__ sums, int nb)
-{
-    // one block of 1024 threads; nb <= 1024 * 16
-    __shared__ unsigned s[1024];
-    unsigned loc[16];
-    unsigned run = 0;
-    const int per = (nb + 1023) / 1024;
-    for (int k = 0; k < per; ++k) {
-        const int i = threadIdx.x * per + k;
-        const unsigned x = i < nb ? sums[i] : 0u;
-        loc[k] = run;
-        run += x;
-    }
-    s[threadIdx.x] = run;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-        const unsigned y = threadIdx.x >= (unsigned)off ? s[threadIdx.x - off] : 0u;
-        __syncthreads();
-        s[threadIdx.x] += y;
-        __syncthreads();
-    }
-    const unsigned base = s[threadIdx.x] - run;
-    for (int k = 0; k < per; ++k) {
-        const int i = threadIdx.x * per + k;
-        if (i < nb) sums[i] = base + loc[k];
-    }
-}
-
-__global__ void k_scan_add(unsigned *__restrict__ out, const unsigned *__restrict__ sums, int n,
-                           unsigned *__restrict__ fill)
-{
-    const int i = blockIdx.x * 1024 + threadIdx.x;
-    if (i < n) {
-        const unsigned v = out[i] + sums[blockIdx.x];
-        out[i] = v;
-        fill[i] = v;
-    }
+    bk[p] = make_int2(b, (int)atomicAdd(&cnt[b], 1u));
 }
 
 // the fourth word is the particle's id: its index, or with several blocks
 // its home key (rank << 23 | cell), which also breaks distance ties
-__global__ void k_hash_scatter(const float4 *__restrict__ pts, int np, const int *__restrict__ bk,
-                               unsigned *__restrict__ fill, float4 *__restrict__ sorted,
-                               const int *__restrict__ key)
+__global__ void k_hash_scatter(const float4 *__restrict__ pts, int np,
+                               const int2 *__restrict__ bk, const unsigned *__restrict__ start,
+                               float4 *__restrict__ sorted, const int *__restrict__ key)
 {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= np) return;
-    const unsigned slot = atomicAdd(&fill[bk[p]], 1u);
+    const int2 b = bk[p];
     const float4 q = pts[p];
-    sorted[slot] = make_float4(q.x, q.y, q.z, __int_as_float(key ? key[p] : p));
+    sorted[start[b.x] + (unsigned)b.y] =
+        make_float4(q.x, q.y, q.z, __int_as_float(key ? key[p] : p));
 }
 
+// start: one word more than there are buckets (the extra one turns into the
+// total)
 void launch_hash_build(const float4 *pts, int np, const HashP &h, unsigned *start,
-                       unsigned *fill, unsigned *sums, int *bk, float4 *sorted, const int *key,
-                       hipStream_t s)
+                       unsigned *sums, int2 *bk, float4 *sorted, const int *key, hipStream_t s)
 {
     const int nbk = h.dims[0] * h.dims[1] * h.dims[2];
-    launch_fill_u32(start, (size_t)nbk + 1, 0u, s);
     if (np > 0)
         hipLaunchKernelGGL(k_hash_count, dim3((np + 255) / 256), dim3(256), 0, s, pts, np, h,
                            start, bk);
-    const int n = nbk + 1;   // the extra slot turns into the total
-    const int nblk = (n + 1023) / 1024;
-    hipLaunchKernelGGL(k_scan_local, dim3(nblk), dim3(1024), 0, s, start, start, sums, n);
-    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(1024), 0, s, sums, nblk);
-    hipLaunchKernelGGL(k_scan_add, dim3(nblk), dim3(1024), 0, s, start, sums, n, fill);
+    launch_scan_u32(start, (unsigned)nbk + 1u, sums, s);
     if (np > 0)
         hipLaunchKernelGGL(k_hash_scatter, dim3((np + 255) / 256), dim3(256), 0, s, pts, np, bk,
-                           fill, sorted, key);
+                           (const unsigned *)start, sorted, key);
 }
 
 // ---------------------------------------------------------------------------
@@ -527,9 +467,6 @@ void launch_owner(const GridP &gp, const HashP &h, const unsigned *start, const 
                   int *const *npts_tab, const int *const *stex_tab, unsigned *defq,
                   unsigned defq_cap, hipStream_t s)
 {
-    // one block: its counts start here; several: the caller clears all
-    // blocks' counts before the first owner pass
-    if (!npts_tab && ncells > 0) launch_fill_u32((unsigned *)npts, (size_t)ncells, 0u, s);
     const int tx = (gp.bnum_idx[0] + 3) / 4, ty = (gp.bnum_idx[1] + 3) / 4,
               tz = (gp.bnum_idx[2] + 3) / 4;
     const int ntiles = tx * ty * tz;
@@ -663,7 +600,6 @@ void launch_exact_status(const BlockIn &in, const GridP &gp, int *status, int pr
                          unsigned char *flags, hipStream_t s)
 {
     if (in.ncells <= 0) return;
-    launch_fill_u32((unsigned *)flags, ((size_t)in.ncells * 3 + 3) / 4, 0u, s);
     if (in.ntets > 0) {
         const int blocks = std::min(4096, (in.ntets + 255) / 256);
         hipLaunchKernelGGL(k_exact_flags, dim3(blocks), dim3(256), 0, s, in, gp, prec, flags, ctrs);

@@ -9,7 +9,7 @@
 // shared list; this pass replays the additions of every point that got more
 // than one in ascending key order (key = cell id, or the received-point key
 // above 2^31):
-//   0. pairs: a grid pass adds the points with exactly two contributions;
+// (points with exactly two are added by the pass that ends the run):
 //   1. gather: each larger point (through its representative list entry,
 //      the third contribution) reserves a contiguous segment, sized by its
 //      contribution count, is filed in one of three classes by that count,
@@ -43,39 +43,6 @@ __device__ __forceinline__ int4 *fold_list(const CellOut &o, int cls)
 __device__ __forceinline__ unsigned fold_capacity(const CellOut &o, int cls)
 {
     return cls == 0 ? o.fold_cap[0] : (cls == 1 ? o.fold_cap[1] : o.fold_cap[2]);
-}
-
-// 0. points with exactly two contributions (the common case: a point on the
-// face between two cells) hold both next to the point: added here in the
-// order the sort gives the pair (the second first unless its key is
-// larger); every point with a second contribution is counted
-__global__ __launch_bounds__(256) void k_fold_pairs(const CellOut *__restrict__ outs,
-                                                    const GridP *__restrict__ gps)
-{
-    __shared__ unsigned s_n;
-    const CellOut &o = outs[blockIdx.y];
-    const double dd = (double)gps[blockIdx.y].div;
-    if (threadIdx.x == 0) s_n = 0;
-    __syncthreads();
-    unsigned np = 0;
-    for (unsigned long long g = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x;
-         g < o.ngrid; g += (unsigned long long)gridDim.x * blockDim.x) {
-        const unsigned c = o.count[g];
-        if (c < 2u) continue;
-        ++np;
-        if (c != 2u) continue;
-        const uint2 f = o.first[g], q = o.second[g];
-        const bool sw = q.x > f.x;
-        const unsigned m0 = sw ? f.y : q.y, m1 = sw ? q.y : f.y;
-        float rho = (float)(0.0 + (double)__uint_as_float(m0) / dd);
-        rho = (float)((double)rho + (double)__uint_as_float(m1) / dd);
-        o.density[g] = rho;
-    }
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) np += __shfl_xor(np, m);
-    if ((threadIdx.x & 63) == 0 && np) atomicAdd(&s_n, np);
-    __syncthreads();
-    if (threadIdx.x == 0 && s_n) atomicAdd(&o.ctrs[C_PAIRS], s_n);
 }
 
 // 1. one segment per shared point; slot and segment reservations are
@@ -528,16 +495,14 @@ static unsigned capped_blocks(unsigned long long work, unsigned per, unsigned ca
 }
 
 void launch_fold(const CellOut *outs, const GridP *gps, int nb, unsigned max_ovf_cap,
-                 const unsigned max_fold_cap[3], unsigned long long max_grid,
-                 unsigned long long sum_ovf_cap, unsigned long long sum_mid_cap, hipStream_t s)
+                 const unsigned max_fold_cap[3], unsigned long long sum_ovf_cap,
+                 unsigned long long sum_mid_cap, hipStream_t s)
 {
     if (nb <= 0) return;
     // per-block grids sized by the largest block's capacities, fewer
     // workgroups per block when there are many blocks (the loops stride);
     // the dealt passes are sized by the capacities of all blocks
     const unsigned per = nb > 16 ? 256 : 4096;
-    const unsigned bg = (unsigned)std::min<unsigned long long>(per, max_grid / 256 + 1);
-    hipLaunchKernelGGL(k_fold_pairs, dim3(bg, nb), dim3(256), 0, s, outs, gps);
     hipLaunchKernelGGL(k_fold_gather, dim3(capped_blocks(max_ovf_cap, 1024, per / 4), nb),
                        dim3(1024), 0, s, outs);
     hipLaunchKernelGGL(k_fold_scatter, dim3(capped_blocks(sum_ovf_cap, 256, 4096)), dim3(256), 0,

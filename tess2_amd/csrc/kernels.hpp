@@ -245,9 +245,9 @@ hipError_t copy_to_device(void *dst, const void *src, size_t bytes, hipStream_t 
 // circumcenters; cc.w = error bound of the float solve (inf when undefined)
 void launch_circumcenters(const float4 *pts, const int4 *tets, int ntets, float4 *cc,
                           hipStream_t s);
+// start, npts and flags below are zero on entry
 void launch_hash_build(const float4 *pts, int np, const HashP &h, unsigned *start,
-                       unsigned *fill, unsigned *sums, int *bk, float4 *sorted, const int *key,
-                       hipStream_t s);
+                       unsigned *sums, int2 *bk, float4 *sorted, const int *key, hipStream_t s);
 // npts_tab / stex_tab (by rank) when several blocks share the assignment,
 // else nullptr; defq: queue of defq_cap grid points for the FP64 re-search
 // of the mixed precision (0: searched inline)
@@ -255,7 +255,7 @@ void launch_owner(const GridP &gp, const HashP &h, const unsigned *start, const 
                   int *owner, int prec, unsigned *ctrs, const int *status, int *npts,
                   int ncells, int *const *npts_tab, const int *const *stex_tab, unsigned *defq,
                   unsigned defq_cap, hipStream_t s);
-// flags: 3 * ncells bytes of scratch (incomplete, outside, defined)
+// flags: 3 * ncells bytes (incomplete, outside, defined)
 void launch_exact_status(const BlockIn &in, const GridP &gp, int *status, int prec,
                          unsigned *ctrs, unsigned char *flags, hipStream_t s);
 // parts: 1 = densities of the owned points, 2 = CIC of cells that own none;
@@ -264,6 +264,10 @@ void launch_exact_tail(const BlockIn &in, const GridP &gp, const int *owner,
                        const int *status_ex, const CellOut &o, int prec, int *const *npts_tab,
                        const int *const *stex_tab, const Router *rt, int self, int parts,
                        hipStream_t s);
+// exclusive scan of n counts in place (n up to 67 M); sums: scan_sums_words(n)
+// words of scratch
+size_t scan_sums_words(size_t n);
+void launch_scan_u32(unsigned *a, unsigned n, unsigned *sums, hipStream_t s);
 void launch_fill_u32(unsigned *p, size_t n, unsigned v, hipStream_t s);
 // ghost selection (incomplete_cells): bit i of sends[p] for neighbour box i
 // (6 floats each, [first, nnb)), for original particles p < norig
@@ -288,9 +292,15 @@ void launch_unpack_cc(const float4 *cc, const int *tnew, int nt, float *out, hip
 void launch_device_block(const float *xyz, int np, const int4 *tets, int nt, const int *v2t,
                          float4 *pts, float4 *cc, unsigned *ctrs, unsigned *stop, unsigned token,
                          hipStream_t s);
-// zero every block's density and count grids; circumcenters of every block
-void launch_block_prep(const BlockIn *ins, const CellOut *outs, int nb, int max_tets,
-                       unsigned long long max_grid, bool circumcenters, hipStream_t s);
+// up to four arrays of n words to zero at the start of a run
+struct ZeroList {
+    unsigned *p[4];
+    unsigned long long n[4];
+};
+// the start of a run: circumcenters of every block (max_tets > 0), density and
+// count grids and the listed arrays zeroed
+void launch_run_prep(const BlockIn *ins, const CellOut *outs, int nb, int max_tets,
+                     unsigned long long max_grid, const ZeroList &z, hipStream_t s);
 void launch_cells_ref(const BlockIn &in, const GridP &gp, const CellOut &o,
                       int want_density, hipStream_t s);
 void launch_cells_ref_slow(const BlockIn &in, const GridP &gp, const CellOut &o,
@@ -333,14 +343,22 @@ void launch_cells_ref_batched(const BlockIn *ins, const GridP *gps, const CellOu
                               const Router *rt, const Chunk *chunks, const XcdQueues &xq,
                               unsigned *queue, int waves, int want_density, hipStream_t s,
                               bool spec);
-// ordered fold of shared grid points and per-block statistics for nb blocks
-// at once (outs/gps: device arrays; the capacities size the grids)
+// ordered fold of the points with three and more contributions of nb blocks at
+// once (outs/gps: device arrays; the capacities size the grids)
 // nb <= 128; the sums are the list capacities of all blocks
 void launch_fold(const CellOut *outs, const GridP *gps, int nb, unsigned max_ovf_cap,
-                 const unsigned max_fold_cap[3], unsigned long long max_grid,
-                 unsigned long long sum_ovf_cap, unsigned long long sum_mid_cap, hipStream_t s);
-// part: nb * 1024 doubles of scratch for the fixed-order grid sums
-void launch_stats(const CellOut *outs, double *part, int nb, int max_cells,
-                  unsigned long long max_grid, hipStream_t s);
+                 const unsigned max_fold_cap[3], unsigned long long sum_ovf_cap,
+                 unsigned long long sum_mid_cap, hipStream_t s);
+// the end of a run: points with two contributions, statistics.  part: nb *
+// RUN_PARTS records of scratch
+enum { RUN_PARTS = 1024 };
+struct RunPart {
+    double sum;                  // of the density
+    float mx;                    // its maximum
+    unsigned pairs;              // points with two and more contributions
+    unsigned long long c[6];     // cells per status 0..4, points of deposited cells
+};
+void launch_run_finish(const CellOut *outs, const GridP *gps, RunPart *part, int nb, int max_cells,
+                       unsigned long long max_grid, hipStream_t s);
 
 }  // namespace t2

@@ -99,101 +99,114 @@ int launch_stage_check(const float *xyz, int np, const int4 *tets, int nt, const
 // ---------------------------------------------------------------------------
 // exclusive scan of n unsigned counts, in place
 // ---------------------------------------------------------------------------
-constexpr int SCAN_TILE = 4096;   // 1024 lanes of four
-constexpr int SCAN_MOST = 16;     // entries per lane of the one-workgroup scan
+constexpr unsigned SCAN_TILE = 4096;   // 1024 lanes of four
+constexpr unsigned SCAN_MOST = 16;     // entries per lane of the one-workgroup scan
 
-// exclusive prefix of one value per lane over a 1024-lane workgroup, and the
-// total: wave scans by lane exchanges, the 16 wave sums through LDS
-__device__ __forceinline__ unsigned scan_1024(unsigned x, unsigned *s_w, unsigned &total)
+// inclusive prefix sums over a wave in six additions (rows of 16 by shifts,
+// then the last lane of rows 0 and 2 into 1 and 3, of row 1 into 2 and 3)
+__device__ __forceinline__ unsigned wave_scan(unsigned x)
 {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    unsigned incl = x;
-    for (int off = 1; off < 64; off <<= 1) {
-        const unsigned t = __shfl_up(incl, off);
-        if (lane >= off) incl += t;
+    x += (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false);
+    x += (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false);
+    x += (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false);
+    x += (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false);
+    x += (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);
+    x += (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);
+    return x;
+}
+
+// Exclusive scan of a[0 .. n) by a workgroup of 16 waves, n <= 1024 * per and
+// per <= ROWS: each wave takes per * 64 neighbouring entries as per coalesced
+// rows, scans them independently of each other, and the 16 waves' totals meet
+// in LDS.  (Each lane reading its own per entries in a row instead touches a
+// cache line per entry: 14,000 entries in one workgroup 11.7 against 3.8 us.)
+// Returns the total.
+template <unsigned ROWS>
+__device__ __forceinline__ unsigned scan_1024(unsigned *__restrict__ a, unsigned n, unsigned per)
+{
+    __shared__ unsigned s_w[16];
+    const unsigned lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const unsigned i0 = w * per * 64 + lane;
+    unsigned v[ROWS], x[ROWS];
+#pragma unroll
+    for (unsigned k = 0; k < ROWS; ++k) {
+        const unsigned i = i0 + k * 64;
+        v[k] = x[k] = (k < per && i < n) ? a[i] : 0u;
     }
-    __syncthreads();   // s_w may hold an earlier call's sums
-    if (lane == 63) s_w[w] = incl;
+    unsigned run = 0;
+#pragma unroll
+    for (unsigned k = 0; k < ROWS; ++k) {
+        x[k] = wave_scan(x[k]);
+        v[k] = run + x[k] - v[k];
+        run += (unsigned)__builtin_amdgcn_readlane((int)x[k], 63);
+    }
+    if (lane == 0) s_w[w] = run;
     __syncthreads();
     unsigned base = 0, all = 0;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const unsigned v = s_w[i];
-        base += i < w ? v : 0u;
-        all += v;
+    for (unsigned i = 0; i < 16; ++i) {
+        const unsigned t = s_w[i];
+        base += i < w ? t : 0u;
+        all += t;
     }
-    total = all;
-    return base + incl - x;
+#pragma unroll
+    for (unsigned k = 0; k < ROWS; ++k) {
+        const unsigned i = i0 + k * 64;
+        if (k < per && i < n) a[i] = base + v[k];
+    }
+    return all;
 }
 
 __global__ __launch_bounds__(1024) void k_scan_tiles(unsigned *__restrict__ a, unsigned n,
                                                      unsigned *__restrict__ sums)
 {
-    __shared__ unsigned s_w[16];
-    const unsigned i = blockIdx.x * SCAN_TILE + threadIdx.x * 4;
-    unsigned v[4], run = 0;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        v[k] = i + k < n ? a[i + k] : 0u;
-        const unsigned x = v[k];
-        v[k] = run;
-        run += x;
-    }
-    unsigned total;
-    const unsigned base = scan_1024(run, s_w, total);
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-        if (i + k < n) a[i + k] = base + v[k];
+    const unsigned i0 = blockIdx.x * SCAN_TILE;
+    const unsigned total = scan_1024<4>(a + i0, min(n - i0, (unsigned)SCAN_TILE), 4);
     if (threadIdx.x == 0) sums[blockIdx.x] = total;
 }
 
-// one workgroup over n <= 1024 * SCAN_MOST entries
+// one workgroup over n <= 1024 * ROWS entries
+template <unsigned ROWS>
 __global__ __launch_bounds__(1024) void k_scan_one(unsigned *__restrict__ a, unsigned n)
 {
-    __shared__ unsigned s_w[16];
-    const unsigned per = (n + 1023) / 1024;
-    unsigned v[SCAN_MOST], run = 0;
-#pragma unroll
-    for (unsigned k = 0; k < SCAN_MOST; ++k) {
-        const unsigned i = threadIdx.x * per + k;
-        const unsigned x = (k < per && i < n) ? a[i] : 0u;
-        v[k] = run;
-        run += x;
-    }
-    unsigned total;
-    const unsigned base = scan_1024(run, s_w, total);
-#pragma unroll
-    for (unsigned k = 0; k < SCAN_MOST; ++k) {
-        const unsigned i = threadIdx.x * per + k;
-        if (k < per && i < n) a[i] = base + v[k];
-    }
+    scan_1024<ROWS>(a, n, (n + 1023) / 1024);
+}
+
+static void scan_one(unsigned *a, unsigned n, hipStream_t s)
+{
+    if (n <= 4096)
+        hipLaunchKernelGGL((k_scan_one<4>), dim3(1), dim3(1024), 0, s, a, n);
+    else
+        hipLaunchKernelGGL((k_scan_one<SCAN_MOST>), dim3(1), dim3(1024), 0, s, a, n);
 }
 
 __global__ __launch_bounds__(1024) void k_scan_bases(unsigned *__restrict__ a, unsigned n,
                                                      const unsigned *__restrict__ sums)
 {
     const unsigned base = sums[blockIdx.x];
-    const unsigned i = blockIdx.x * SCAN_TILE + threadIdx.x * 4;
+    const unsigned i = blockIdx.x * SCAN_TILE + threadIdx.x;
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
-        if (i + k < n) a[i + k] += base;
+    for (unsigned k = 0; k < 4; ++k)
+        if (i + k * 1024 < n) a[i + k * 1024] += base;
 }
 
 // n up to 1024 * SCAN_MOST in one workgroup, else tiles and their sums (up to
 // 4096 * 16384 = 67 M entries: 256 digits of 262144 sort tiles)
-static void scan_u32(unsigned *a, unsigned n, unsigned *sums, hipStream_t s)
+void launch_scan_u32(unsigned *a, unsigned n, unsigned *sums, hipStream_t s)
 {
     if (n == 0) return;
     if (n <= 1024u * SCAN_MOST) {
-        hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(1024), 0, s, a, n);
+        scan_one(a, n, s);
         return;
     }
     const unsigned tiles = (n + SCAN_TILE - 1) / SCAN_TILE;
     hipLaunchKernelGGL(k_scan_tiles, dim3(tiles), dim3(1024), 0, s, a, n, sums);
-    hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(1024), 0, s, sums, tiles);
+    scan_one(sums, tiles, s);
     hipLaunchKernelGGL(k_scan_bases, dim3(tiles), dim3(1024), 0, s, a, n,
                        (const unsigned *)sums);
 }
+
+size_t scan_sums_words(size_t n) { return (n + SCAN_TILE - 1) / SCAN_TILE; }
 
 // ---------------------------------------------------------------------------
 // stable radix sort of (key, id) pairs, 8 bits a pass.  A workgroup of four
@@ -289,7 +302,7 @@ static int radix_sort(unsigned *k0, unsigned *v0, unsigned *k1, unsigned *v1, un
         unsigned *kb = which ? k0 : k1, *vb = which ? v0 : v1;
         hipLaunchKernelGGL(k_sort_hist, dim3(tiles), dim3(256), 0, s, (const unsigned *)ka, n,
                            shift, hist, tiles);
-        scan_u32(hist, 256 * tiles, sums, s);
+        launch_scan_u32(hist, 256 * tiles, sums, s);
         hipLaunchKernelGGL(k_sort_scatter, dim3(tiles), dim3(256), 0, s, (const unsigned *)ka,
                            (const unsigned *)va, n, shift, (const unsigned *)hist, tiles, kb, vb);
     }
@@ -434,7 +447,7 @@ void launch_layout(const float4 *pts, int np, int norig, const StageBox &box, co
     const unsigned *id = radix_sort(k0, v0, k1, v1, (unsigned)np, 30, hist, sums, s) ? v1 : v0;
     const int nob = (np + 1023) / 1024;
     hipLaunchKernelGGL(k_order_count, dim3(nob), dim3(1024), 0, s, id, np, norig, hist);
-    scan_u32(hist, (unsigned)nob, sums, s);
+    launch_scan_u32(hist, (unsigned)nob, sums, s);
     hipLaunchKernelGGL(k_order_write, dim3(nob), dim3(1024), 0, s, id, np, norig,
                        (const unsigned *)hist, rank, order);
     if (nt > 0) {
