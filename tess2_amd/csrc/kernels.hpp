@@ -264,8 +264,8 @@ void launch_exact_tail(const BlockIn &in, const GridP &gp, const int *owner,
                        const int *status_ex, const CellOut &o, int prec, int *const *npts_tab,
                        const int *const *stex_tab, const Router *rt, int self, int parts,
                        hipStream_t s);
-// exclusive scan of n counts in place (n up to 67 M); sums: scan_sums_words(n)
-// words of scratch
+// exclusive scan of n counts in place; sums: scan_sums_words(n) words of
+// scratch
 size_t scan_sums_words(size_t n);
 void launch_scan_u32(unsigned *a, unsigned n, unsigned *sums, hipStream_t s);
 void launch_fill_u32(unsigned *p, size_t n, unsigned v, hipStream_t s);

@@ -2,18 +2,18 @@
 // order of the cells and tets, renumbering.
 //
 // A block arrives as the caller's arrays (one copy each); everything staging
-// does to them is a device pass here.  The order is the one a host sort of
-// (Morton code, particle) and (lowest Morton rank of the vertices, tet)
-// pairs gives: cells in Morton order of their sites, tets renumbered by their
-// lowest-ranked vertex.  Both sorts are stable least-significant-digit radix
-// sorts of (key, id) pairs whose ids start ascending, so that ties stay in id
-// order.
+// does to them is a device pass here: cells in Morton order of their sites
+// (a stable radix sort of (key, id) pairs whose ids start ascending, so that
+// ties stay in id order; ghosts after all originals), tets renumbered by
+// their lowest-ranked vertex, in no set order among one vertex's.
 //
 // What bounds it: a block is read and written a few times (the tets: range
-// check 32 B, keys 16 B + 16 B of gathered ranks, three digit passes of 16 B
-// each way, renumbering 32 B in and out and 16 B of gathered numbers), which
-// takes less than its copy over PCIe (32 B per tet at ~40 GB/s).  Small
-// blocks are bound by the ~30 launches of about 3 us.
+// check 32 B, keys 16 B + 16 B of gathered ranks and an atomic, renumbering
+// 32 B in and out and 16 B of gathered numbers), which takes less than its
+// copy over PCIe (32 B per tet at ~40 GB/s).  Small blocks are bound by the
+// ~19 launches of about 3 us (with a sort of the tets and 4096-pair tiles 33;
+// whole calls: volume() of 64,000 particles 1115 against 1029 us, 32,000
+// particles on 64^3 1058 against 991).
 #include "kernels.hpp"
 
 #include <algorithm>
@@ -190,8 +190,7 @@ __global__ __launch_bounds__(1024) void k_scan_bases(unsigned *__restrict__ a, u
         if (i + k * 1024 < n) a[i + k * 1024] += base;
 }
 
-// n up to 1024 * SCAN_MOST in one workgroup, else tiles and their sums (up to
-// 4096 * 16384 = 67 M entries: 256 digits of 262144 sort tiles)
+// n up to 1024 * SCAN_MOST in one workgroup, else tiles and their sums
 void launch_scan_u32(unsigned *a, unsigned n, unsigned *sums, hipStream_t s)
 {
     if (n == 0) return;
@@ -201,21 +200,25 @@ void launch_scan_u32(unsigned *a, unsigned n, unsigned *sums, hipStream_t s)
     }
     const unsigned tiles = (n + SCAN_TILE - 1) / SCAN_TILE;
     hipLaunchKernelGGL(k_scan_tiles, dim3(tiles), dim3(1024), 0, s, a, n, sums);
-    scan_one(sums, tiles, s);
+    launch_scan_u32(sums, tiles, sums + tiles, s);
     hipLaunchKernelGGL(k_scan_bases, dim3(tiles), dim3(1024), 0, s, a, n,
                        (const unsigned *)sums);
 }
 
-size_t scan_sums_words(size_t n) { return (n + SCAN_TILE - 1) / SCAN_TILE; }
+size_t scan_sums_words(size_t n)
+{
+    if (n <= 1024 * SCAN_MOST) return 0;
+    const size_t tiles = (n + SCAN_TILE - 1) / SCAN_TILE;
+    return tiles + scan_sums_words(tiles);
+}
 
 // ---------------------------------------------------------------------------
 // stable radix sort of (key, id) pairs, 8 bits a pass.  A workgroup of four
-// waves owns a tile of 4096 consecutive pairs, each wave 1024 of them in
-// rounds of 64; hist is digit-major ([digit][tile]), so its exclusive scan
-// gives each tile's first slot per digit.
+// waves owns a tile of 256 * ROUNDS consecutive pairs, each wave a quarter of
+// them in rounds of 64; hist is digit-major ([digit][tile]), so its exclusive
+// scan gives each tile's first slot per digit.
 // ---------------------------------------------------------------------------
-constexpr int SORT_TILE = 4096, SORT_ROUNDS = SORT_TILE / 256;
-
+template <int ROUNDS>
 __global__ __launch_bounds__(256) void k_sort_hist(const unsigned *__restrict__ key, unsigned n,
                                                    int shift, unsigned *__restrict__ hist,
                                                    unsigned ntiles)
@@ -223,9 +226,9 @@ __global__ __launch_bounds__(256) void k_sort_hist(const unsigned *__restrict__ 
     __shared__ unsigned s_h[256];
     s_h[threadIdx.x] = 0u;
     __syncthreads();
-    const unsigned base = blockIdx.x * SORT_TILE;
+    const unsigned base = blockIdx.x * (256 * ROUNDS);
 #pragma unroll
-    for (int r = 0; r < SORT_ROUNDS; ++r) {
+    for (int r = 0; r < ROUNDS; ++r) {
         const unsigned i = base + r * 256 + threadIdx.x;
         if (i < n) atomicAdd(&s_h[(key[i] >> shift) & 255u], 1u);
     }
@@ -233,13 +236,17 @@ __global__ __launch_bounds__(256) void k_sort_hist(const unsigned *__restrict__ 
     hist[threadIdx.x * ntiles + blockIdx.x] = s_h[threadIdx.x];
 }
 
+// LAST: a pair's slot is its rank, id_out takes the ids of the first nfirst
+// only
+template <int ROUNDS, bool LAST>
 __global__ __launch_bounds__(256) void k_sort_scatter(const unsigned *__restrict__ key,
                                                       const unsigned *__restrict__ id,
                                                       unsigned n, int shift,
                                                       const unsigned *__restrict__ hist,
                                                       unsigned ntiles,
                                                       unsigned *__restrict__ key_out,
-                                                      unsigned *__restrict__ id_out)
+                                                      unsigned *__restrict__ id_out,
+                                                      unsigned nfirst)
 {
     __shared__ unsigned s_c[4][256];   // next slot per wave and digit
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -247,12 +254,13 @@ __global__ __launch_bounds__(256) void k_sort_scatter(const unsigned *__restrict
 #pragma unroll
     for (int i = 0; i < 4; ++i) s_c[i][threadIdx.x] = 0u;
     __syncthreads();
-    const unsigned base = blockIdx.x * SORT_TILE + w * (SORT_TILE / 4) + lane;
-    unsigned k[SORT_ROUNDS];
+    const unsigned base = blockIdx.x * (256 * ROUNDS) + w * (64 * ROUNDS) + lane;
+    unsigned k[ROUNDS], v[ROUNDS];
 #pragma unroll
-    for (int r = 0; r < SORT_ROUNDS; ++r) {
+    for (int r = 0; r < ROUNDS; ++r) {
         const unsigned i = base + r * 64;
         k[r] = i < n ? key[i] : 0u;
+        v[r] = i < n ? id[i] : 0u;
         if (i < n) atomicAdd(&s_c[w][(k[r] >> shift) & 255u], 1u);
     }
     __syncthreads();
@@ -269,7 +277,7 @@ __global__ __launch_bounds__(256) void k_sort_scatter(const unsigned *__restrict
     // a wave's rounds in order; within a round, the lanes of one digit take
     // consecutive slots in lane order (only this wave touches s_c[w])
 #pragma unroll
-    for (int r = 0; r < SORT_ROUNDS; ++r) {
+    for (int r = 0; r < ROUNDS; ++r) {
         const unsigned i = base + r * 64;
         const bool on = i < n;
         const unsigned d = (k[r] >> shift) & 255u;
@@ -281,8 +289,13 @@ __global__ __launch_bounds__(256) void k_sort_scatter(const unsigned *__restrict
         }
         if (on) {
             const unsigned slot = s_c[w][d] + (unsigned)__popcll(same & below);
-            key_out[slot] = k[r];
-            id_out[slot] = id[i];
+            if (LAST) {
+                key_out[v[r]] = slot;
+                if (slot < nfirst) id_out[slot] = v[r];
+            } else {
+                key_out[slot] = k[r];
+                id_out[slot] = v[r];
+            }
         }
         __builtin_amdgcn_wave_barrier();   // every lane has read its counter
         if (on && (same & below) == 0ull) s_c[w][d] += (unsigned)__popcll(same);
@@ -290,24 +303,35 @@ __global__ __launch_bounds__(256) void k_sort_scatter(const unsigned *__restrict
     }
 }
 
-// sorts k0 / v0 (n pairs) by the low `bits` bits of the key; the result is in
-// k0 / v0 when an even number of passes ran, else in k1 / v1 (returned)
-static int radix_sort(unsigned *k0, unsigned *v0, unsigned *k1, unsigned *v1, unsigned n,
-                      int bits, unsigned *hist, unsigned *sums, hipStream_t s)
+// rank of each of n ids in the order of their 32-bit keys (k0 / v0), and the
+// first nfirst ids in it; k1 / v1: as much scratch
+template <int ROUNDS>
+static void radix_rank(unsigned *k0, unsigned *v0, unsigned *k1, unsigned *v1, unsigned n,
+                       unsigned *rank, unsigned *first, unsigned nfirst, unsigned *hist,
+                       unsigned *sums, hipStream_t s)
 {
-    const unsigned tiles = (n + SORT_TILE - 1) / SORT_TILE;
-    int which = 0;
-    for (int shift = 0; shift < bits; shift += 8, which ^= 1) {
-        unsigned *ka = which ? k1 : k0, *va = which ? v1 : v0;
-        unsigned *kb = which ? k0 : k1, *vb = which ? v0 : v1;
-        hipLaunchKernelGGL(k_sort_hist, dim3(tiles), dim3(256), 0, s, (const unsigned *)ka, n,
-                           shift, hist, tiles);
+    const unsigned tiles = (n + 256 * ROUNDS - 1) / (256 * ROUNDS);
+    for (int shift = 0; shift < 32; shift += 8) {
+        hipLaunchKernelGGL((k_sort_hist<ROUNDS>), dim3(tiles), dim3(256), 0, s,
+                           (const unsigned *)k0, n, shift, hist, tiles);
         launch_scan_u32(hist, 256 * tiles, sums, s);
-        hipLaunchKernelGGL(k_sort_scatter, dim3(tiles), dim3(256), 0, s, (const unsigned *)ka,
-                           (const unsigned *)va, n, shift, (const unsigned *)hist, tiles, kb, vb);
+        if (shift < 24)
+            hipLaunchKernelGGL((k_sort_scatter<ROUNDS, false>), dim3(tiles), dim3(256), 0, s,
+                               (const unsigned *)k0, (const unsigned *)v0, n, shift,
+                               (const unsigned *)hist, tiles, k1, v1, 0u);
+        else
+            hipLaunchKernelGGL((k_sort_scatter<ROUNDS, true>), dim3(tiles), dim3(256), 0, s,
+                               (const unsigned *)k0, (const unsigned *)v0, n, shift,
+                               (const unsigned *)hist, tiles, rank, first, nfirst);
+        std::swap(k0, k1);
+        std::swap(v0, v1);
     }
-    return which;
 }
+
+// 16 rounds of 64 pairs a wave, fewer where the chip would be idle and the
+// 256 counts a tile still fit the one-workgroup scan: 42,000 pairs in 11
+// workgroups of 4096 took 22 us a pass, in 42 of 1024 12
+static int sort_rounds(int n) { return n <= 65536 ? 4 : (n <= 131072 ? 8 : 16); }
 
 // ---------------------------------------------------------------------------
 // Morton layout
@@ -322,8 +346,10 @@ __device__ __forceinline__ unsigned spread3(unsigned x)
     return x;
 }
 
-__global__ void k_morton_keys(const float4 *__restrict__ pts, int np, StageBox box,
-                              unsigned *__restrict__ key, unsigned *__restrict__ id)
+// Morton keys of 10 bits an axis, originals before ghosts; ntet: zeroed
+__global__ void k_morton_keys(const float4 *__restrict__ pts, int np, int norig, StageBox box,
+                              unsigned *__restrict__ key, unsigned *__restrict__ id,
+                              unsigned *__restrict__ ntet)
 {
     const int p = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (p >= np) return;
@@ -339,64 +365,42 @@ __global__ void k_morton_keys(const float4 *__restrict__ pts, int np, StageBox b
         g = g < 1023.0 ? g : 1023.0;
         q[i] = (unsigned)g;
     }
-    key[p] = spread3(q[0]) | (spread3(q[1]) << 1) | (spread3(q[2]) << 2);
+    key[p] = spread3(q[0]) | (spread3(q[1]) << 1) | (spread3(q[2]) << 2) |
+             (p < norig ? 0u : 1u << 30);
     id[p] = (unsigned)p;
+    ntet[p] = 0u;
 }
 
-// originals (id < norig) per tile of 1024 sorted particles
-__global__ __launch_bounds__(1024) void k_order_count(const unsigned *__restrict__ id, int np,
-                                                      int norig, unsigned *__restrict__ cnt)
-{
-    __shared__ unsigned s_n[16];
-    const int k = (int)(blockIdx.x * 1024 + threadIdx.x);
-    const unsigned long long m = __ballot(k < np && (int)id[k < np ? k : 0] < norig);
-    if ((threadIdx.x & 63) == 0) s_n[threadIdx.x >> 6] = (unsigned)__popcll(m);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        unsigned t = 0;
-        for (int i = 0; i < 16; ++i) t += s_n[i];
-        cnt[blockIdx.x] = t;
-    }
-}
-
-// rank of every particle, and the originals in sorted order
-__global__ __launch_bounds__(1024) void k_order_write(const unsigned *__restrict__ id, int np,
-                                                      int norig,
-                                                      const unsigned *__restrict__ cnt,
-                                                      int *__restrict__ rank,
-                                                      int *__restrict__ order)
-{
-    __shared__ unsigned s_n[16];
-    const int k = (int)(blockIdx.x * 1024 + threadIdx.x);
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int p = k < np ? (int)id[k] : -1;
-    const bool own = p >= 0 && p < norig;
-    const unsigned long long m = __ballot(own);
-    if (lane == 0) s_n[w] = (unsigned)__popcll(m);
-    __syncthreads();
-    unsigned at = cnt[blockIdx.x];
-    for (int i = 0; i < w; ++i) at += s_n[i];
-    if (p >= 0) rank[p] = k;
-    if (own) order[at + (unsigned)__popcll(m & ((1ull << lane) - 1ull))] = p;
-}
-
-__global__ void k_tet_keys(const int4 *__restrict__ tets, int nt, const int *__restrict__ rank,
-                           unsigned *__restrict__ key, unsigned *__restrict__ id)
+// each tet's first-ranked vertex (an original when it has one), and the tet's
+// place among that vertex's (in no set order: no result depends on it).  One
+// atomic per tet bounds it, 13.5M in 691 us; a stable sort by that vertex, a
+// histogram, scan and scatter per 8 bits, took 744 and 256,000 tets 100
+// against 40 with the scan
+__global__ void k_tet_keys(const int4 *__restrict__ tets, int nt,
+                           const unsigned *__restrict__ rank, unsigned *__restrict__ ntet,
+                           uint2 *__restrict__ key)
 {
     const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (t >= nt) return;
     const int4 v = tets[2 * (long long)t];
-    key[t] = (unsigned)min(min(rank[v.x], rank[v.y]), min(rank[v.z], rank[v.w]));
-    id[t] = (unsigned)t;
+    const unsigned r = min(min(rank[v.x], rank[v.y]), min(rank[v.z], rank[v.w]));
+    key[t] = make_uint2(r, atomicAdd(&ntet[r], 1u));
 }
 
-__global__ void k_tet_new(const unsigned *__restrict__ id, int nt, int *__restrict__ tnew)
+__global__ void k_tet_new(const uint2 *__restrict__ key, const unsigned *__restrict__ start,
+                          int nt, int *__restrict__ tnew, unsigned *__restrict__ id)
 {
-    const int k = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (k < nt) tnew[id[k]] = k;
+    const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (t >= nt) return;
+    const uint2 k = key[t];
+    const unsigned m = start[k.x] + k.y;
+    tnew[t] = (int)m;
+    id[m] = (unsigned)t;
 }
 
-// tets in their new order with renumbered neighbours, vert_to_tet renumbered
+// tets in their new order with renumbered neighbours, vert_to_tet renumbered.
+// Gathers by new id: by old id, scattering 32-byte records, 13.5M tets take
+// 851 against 640 us
 __global__ void k_renumber(const unsigned *__restrict__ id, int nt,
                            const int *__restrict__ tnew, const int4 *__restrict__ raw,
                            int4 *__restrict__ tets, const int *__restrict__ v2t_raw, int np,
@@ -416,20 +420,23 @@ __global__ void k_renumber(const unsigned *__restrict__ id, int nt,
     }
 }
 
-static int bits_for(int n)
+// scratch of launch_layout in unsigned words: the ranks and the tets per rank,
+// two key and two id arrays of the particles or three words per tet, the digit
+// counts and scan sums
+static size_t layout_sort_words(int np, int nt)
 {
-    int b = 1;
-    while (b < 31 && (1 << b) < n) ++b;
-    return b;
+    return std::max<size_t>(4 * (size_t)np, 3 * (size_t)nt);
 }
-
-// scratch of launch_layout in unsigned words: two key and two id arrays, the
-// ranks, the digit counts and their tile sums
+static size_t layout_hist_words(int np)
+{
+    const size_t tile = 256 * (size_t)sort_rounds(np);
+    return 256 * ((np + tile - 1) / tile);
+}
 size_t layout_scratch_words(int np, int nt)
 {
-    const size_t n = (size_t)std::max(std::max(np, nt), 1);
-    const size_t tiles = (n + SORT_TILE - 1) / SORT_TILE;
-    return 4 * n + (size_t)std::max(np, 1) + 256 * tiles + SCAN_TILE + tiles;
+    const size_t h = layout_hist_words(np);
+    return layout_sort_words(np, nt) + 2 * (size_t)np + h +
+           scan_sums_words(std::max<size_t>(h, (size_t)np)) + 1;
 }
 
 void launch_layout(const float4 *pts, int np, int norig, const StageBox &box, const int4 *raw,
@@ -437,27 +444,27 @@ void launch_layout(const float4 *pts, int np, int norig, const StageBox &box, co
                    int *v2t, int *tnew, hipStream_t s)
 {
     if (np <= 0) return;   // no particles, no tets
-    const size_t n = (size_t)std::max(np, nt);
-    const size_t tiles = (n + SORT_TILE - 1) / SORT_TILE;
-    unsigned *k0 = scratch, *v0 = k0 + n, *k1 = v0 + n, *v1 = k1 + n;
-    int *rank = reinterpret_cast<int *>(v1 + n);
-    unsigned *hist = reinterpret_cast<unsigned *>(rank + np), *sums = hist + 256 * tiles;
-    hipLaunchKernelGGL(k_morton_keys, dim3((np + 255) / 256), dim3(256), 0, s, pts, np, box, k0,
-                       v0);
-    const unsigned *id = radix_sort(k0, v0, k1, v1, (unsigned)np, 30, hist, sums, s) ? v1 : v0;
-    const int nob = (np + 1023) / 1024;
-    hipLaunchKernelGGL(k_order_count, dim3(nob), dim3(1024), 0, s, id, np, norig, hist);
-    launch_scan_u32(hist, (unsigned)nob, sums, s);
-    hipLaunchKernelGGL(k_order_write, dim3(nob), dim3(1024), 0, s, id, np, norig,
-                       (const unsigned *)hist, rank, order);
+    unsigned *k0 = scratch, *v0 = k0 + np, *k1 = v0 + np, *v1 = k1 + np;
+    uint2 *tkey = reinterpret_cast<uint2 *>(scratch);   // when the sort is over
+    unsigned *tid = scratch + 2 * (size_t)nt;
+    unsigned *rank = scratch + layout_sort_words(np, nt), *ntet = rank + np, *hist = ntet + np,
+             *sums = hist + layout_hist_words(np);
+    hipLaunchKernelGGL(k_morton_keys, dim3((np + 255) / 256), dim3(256), 0, s, pts, np, norig,
+                       box, k0, v0, ntet);
+    unsigned *first = reinterpret_cast<unsigned *>(order);
+    const int rounds = sort_rounds(np);
+    (rounds == 4 ? radix_rank<4> : (rounds == 8 ? radix_rank<8> : radix_rank<16>))(
+        k0, v0, k1, v1, (unsigned)np, rank, first, (unsigned)norig, hist, sums, s);
     if (nt > 0) {
-        hipLaunchKernelGGL(k_tet_keys, dim3((nt + 255) / 256), dim3(256), 0, s, raw, nt,
-                           (const int *)rank, k0, v0);
-        id = radix_sort(k0, v0, k1, v1, (unsigned)nt, bits_for(np), hist, sums, s) ? v1 : v0;
-        hipLaunchKernelGGL(k_tet_new, dim3((nt + 255) / 256), dim3(256), 0, s, id, nt, tnew);
+        const dim3 g((nt + 255) / 256);
+        hipLaunchKernelGGL(k_tet_keys, g, dim3(256), 0, s, raw, nt, (const unsigned *)rank, ntet,
+                           tkey);
+        launch_scan_u32(ntet, (unsigned)np, sums, s);
+        hipLaunchKernelGGL(k_tet_new, g, dim3(256), 0, s, (const uint2 *)tkey,
+                           (const unsigned *)ntet, nt, tnew, tid);
     }
     const int m = std::max(np, nt);
-    hipLaunchKernelGGL(k_renumber, dim3((m + 255) / 256), dim3(256), 0, s, id, nt,
+    hipLaunchKernelGGL(k_renumber, dim3((m + 255) / 256), dim3(256), 0, s, (const unsigned *)tid, nt,
                        (const int *)tnew, raw, tets, v2t_raw, np, v2t);
 }
 
