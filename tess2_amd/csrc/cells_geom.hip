@@ -27,6 +27,16 @@
 // hold a slot (or face number), or 48 + lane while a round decides who takes
 // it; atomicMin leaves the lowest.  Each user then compares the slot's full id, so
 // two ids that share 26 bits only defer the cell.
+// What bounds it: vector instructions, about 450 a cell, three fifths of them in
+// the star's rounds (2.1M cells of a GRF box with planes: 1.86 ms, 24 GB of
+// tets at 32 B out of the caches; volumes of 216k cells 188 us, of 64k 64).
+// Each table probe, index and mask in a round is therefore the cheapest form
+// that holds: tables of 64 words that cannot fill up (with 32 words for the
+// vertices and a probe count 2.04 ms, 219 and 74 us), 24-bit hash products,
+// wrap-arounds by one subtraction, hull links seen when a tet is taken rather
+// than when it is visited, a group's ballot in one register, the bbox by
+// row exchanges instead of LDS.  Eight cells a wave (8 lanes each) has the
+// same rate and a longer latency.
 // Cells beyond SG star tets or FG faces, and stars whose links are not those
 // of a tessellation, go to the large-capacity pass (k_cells_ref_slow).
 #include "kernels.hpp"
@@ -68,26 +78,28 @@ __device__ __forceinline__ unsigned eq4(const int4 &q, int x)
            (q.w == x ? 8u : 0u);
 }
 
-// position of x in q (0 when it is not there), and r's component there; a
-// chain of selects on one variable index would compile to nested branches
-__device__ __forceinline__ void find4(const int4 &q, const int4 &r, int x, int &i, int &rx)
-{
-    i = 0;
-    rx = r.x;
-    const bool y = q.y == x, z = q.z == x, w = q.w == x;
-    i = y ? 1 : i;
-    rx = y ? r.y : rx;
-    i = z ? 2 : i;
-    rx = z ? r.z : rx;
-    i = w ? 3 : i;
-    rx = w ? r.w : rx;
-}
-
 // the component at the one bit of m, by masks
 __device__ __forceinline__ int pick4(const int4 &q, unsigned m)
 {
     return (q.x & -(int)(m & 1u)) | (q.y & -(int)((m >> 1) & 1u)) |
            (q.z & -(int)((m >> 2) & 1u)) | (q.w & -(int)((m >> 3) & 1u));
+}
+
+// x of the lane whose number differs by a mirror: quads' pairs, quads' halves,
+// eights and sixteens, which together reach every lane of 16
+template <int CTRL>
+__device__ __forceinline__ float dpp_f(float x)
+{
+    return __int_as_float(
+        __builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float lesser(float x, float y) { return y < x ? y : x; }   // no NaN
+__device__ __forceinline__ float min16(float x)
+{
+    x = lesser(x, dpp_f<0xb1>(x));    // quad_perm 1,0,3,2
+    x = lesser(x, dpp_f<0x4e>(x));    // quad_perm 2,3,0,1
+    x = lesser(x, dpp_f<0x141>(x));   // mirrored eights
+    return lesser(x, dpp_f<0x140>(x));   // mirrored sixteens
 }
 
 // orders the compiler's LDS accesses around lanes' exchanges through LDS (a
@@ -98,22 +110,24 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_wave_barrier();
 }
 
-// find id in the table of 1 << BITS words or put `want` (its tag above a
-// pending code) there; the lowest pending code of an id stays.  Returns the
-// entry, or -1 when the table is full.
-template <int BITS>
+// first entry to look at in a table of 64 words: the top bits of a 24-bit
+// product (a full-rate multiplication; consecutive ids fall far apart)
+__device__ __forceinline__ unsigned table_first(int id)
+{
+    return (__umul24((unsigned)id, 0x9E3779u) >> 18) & 63u;
+}
+
+// find id in the table of 64 words or put `want` (its tag above a pending
+// code) there; the lowest pending code of an id stays.  Returns the entry.  A
+// round starts with at most SG tets and FG vertices and adds at most one per
+// lane of the group, so that there always is one.
 __device__ __forceinline__ int table_take(unsigned *t, int id, unsigned want)
 {
-    unsigned h = ((unsigned)id * 0x9E3779B1u) >> (32 - BITS);
-    unsigned old = 0;
-    int n = 0;
-#pragma unroll 1
-    for (; n < (1 << BITS); ++n) {
+    unsigned h = table_first(id), old = atomicCAS(&t[h], EMPTY, want);
+    while (old != EMPTY && (old >> 6) != (want >> 6)) {
+        h = (h + 1) & 63u;
         old = atomicCAS(&t[h], EMPTY, want);
-        if (old == EMPTY || (old >> 6) == (want >> 6)) break;
-        h = (h + 1) & ((1u << BITS) - 1u);
     }
-    if (n == (1 << BITS)) return -1;
     if (old != EMPTY && (old & 63u) >= PENDING) atomicMin(&t[h], want);
     return (int)h;
 }
@@ -127,17 +141,18 @@ __device__ __forceinline__ int table_take(unsigned *t, int id, unsigned want)
 template <int SG, int FG>
 struct GeomLayout {
     static constexpr int T = 0;                 // unsigned [64] tet table
-    static constexpr int V = 256;               // unsigned [32] vertex table
-    static constexpr int CAND = 384;            // int2 [QUEUE] neighbour ids to visit
+    static constexpr int V = 256;               // unsigned [64] vertex table
+    static constexpr int CAND = 512;            // int2 [QUEUE] neighbour ids to visit
     static constexpr int CC = 0;                // float [SG][3] circumcenters
-    static constexpr int TID = 12 * SG;         // int [SG] slot -> tet; then fvol
-    static constexpr int F = 16 * SG;           // unsigned [SG]
-    static constexpr int FU = 20 * SG;          // int [FG] face -> vertex
+    static constexpr int TID = CAND + 8 * QUEUE;   // int [SG] slot -> tet; then fvol
+    static constexpr int F = TID + 4 * SG;      // unsigned [SG]
+    static constexpr int FU = F + 4 * SG;       // int [FG] face -> vertex
     static constexpr int FLAG = FU + 4 * FG;    // int: a ring does not close
     static constexpr int NB = FLAG + 4;         // unsigned char [SG][3]
     static constexpr int FS = NB + 3 * SG;      // unsigned char [FG] face -> first slot
     static constexpr int BYTES = (FS + FG + 15) / 16 * 16;
-    static_assert(CAND + 8 * QUEUE <= 12 * SG, "tables and queue fit under the circumcenters");
+    static_assert(12 * SG <= TID, "the circumcenters fit over tables and queue");
+    static_assert(SG + 16 <= 64 && FG + 16 <= 64, "a round's new ids fit the tables");
 };
 
 template <int CPW, int SG, int FG, bool MULTI, bool PLANES>
@@ -152,7 +167,13 @@ __global__ __launch_bounds__(64) void k_cell_geom(CellSet<MULTI> set, PlaneBuf p
     const int lane = (int)(threadIdx.x & 63);
     const int g = lane / G, gl = lane % G;
     const unsigned long long gbits = ((1ull << G) - 1ull) << (g * G);
-    const unsigned long long below = (1ull << lane) - 1ull;
+    // a ballot's half that holds the group, the group's bits there, and those
+    // of its lower lanes
+    const bool upper = lane >= 32;
+    auto half = [upper](unsigned long long m) {
+        return upper ? (unsigned)(m >> 32) : (unsigned)m;
+    };
+    const unsigned ghalf = half(gbits), gbelow = ghalf & ((1u << (lane & 31)) - 1u);
 
     constexpr int WPT = CELL_TILE / CPW;   // waves per tile
     const int item = xcd_item((int)blockIdx.x, set.ntiles * WPT);
@@ -178,29 +199,31 @@ __global__ __launch_bounds__(64) void k_cell_geom(CellSet<MULTI> set, PlaneBuf p
     int st = !have ? G_NONE : (vt < 0 ? G_HULL : G_RUN);
 
     // ---- 1. star ------------------------------------------------------------
-    for (int i = gl; i < 96; i += G) T[i] = EMPTY;   // both tables
+    for (int i = gl; i < 128; i += G) T[i] = EMPTY;   // both tables
     if (gl == 0) *reinterpret_cast<int *>(R + L::FLAG) = 0;
     wave_sync();
     int rootn = -1;   // lanes 0..2: the first tet's neighbour across link vertex gl
     if (st == G_RUN) {
         const int4 rv = in.tets[2 * (long long)vt], rn = in.tets[2 * (long long)vt + 1];
         const unsigned mv = eq4(rv, v);
-        bool ok = __popc(mv) == 1;
+        bool ok = __popc(mv) == 1, inner = true;
         if (ok && gl < 3) {
             const unsigned mi = 1u << (gl + (gl >= __builtin_ctz(mv) ? 1 : 0));
             const int u = pick4(rv, mi);
             rootn = pick4(rn, mi);
             const unsigned want = ((unsigned)u << 6) | (unsigned)gl;
-            const int e = table_take<5>(V, u, want);
+            inner = rootn >= 0;
+            const int e = table_take(V, u, want);
             ok = V[e] == want;   // a vertex twice in the tet: not a tet
             fu[gl] = u;
             fs[gl] = 0;
         }
         if (ok && gl == 0) {
-            T[((unsigned)vt * 0x9E3779B1u) >> 26] = (unsigned)vt << 6;
+            T[table_first(vt)] = (unsigned)vt << 6;
             tid[0] = vt;
             fw[0] = 0u | (1u << 8) | (2u << 16) | (3u << 24);
         }
+        if (__ballot(!inner) & gbits) st = G_HULL;
         if (__ballot(!ok) & gbits) st = G_DEFER;
     }
     wave_sync();
@@ -215,7 +238,7 @@ __global__ __launch_bounds__(64) void k_cell_geom(CellSet<MULTI> set, PlaneBuf p
         if (mine) {
             if (q >= 3) {
                 s = (q - 1) >> 1;
-                ni = cand[(q - 1) % (2 * QUEUE)];
+                ni = cand[q - 1 - (q > 2 * QUEUE ? 2 * QUEUE : 0)];
             }
             const unsigned w = fw[s];
             if (q >= 3) {
@@ -224,31 +247,26 @@ __global__ __launch_bounds__(64) void k_cell_geom(CellSet<MULTI> set, PlaneBuf p
             }
             // loaded before the table knows whether the tet is new, so that
             // the load is in flight while it decides
-            if (ni >= 0) {
-                rv = in.tets[2 * (long long)ni];
-                rn = in.tets[2 * (long long)ni + 1];
-            }
+            const int4 *tp = in.tets + 2u * (unsigned)ni;
+            rv = tp[0];
+            rn = tp[1];
             // the link vertices shared across the face: the other two
-            fa = (int)((j == 0 ? w >> 8 : w) & 255u);
-            fb = (int)((j == 2 ? w >> 8 : w >> 16) & 255u);
+            fa = (int)((w >> (j == 0 ? 8 : 0)) & 255u);
+            fb = (int)((w >> (j == 2 ? 8 : 16)) & 255u);
             ua = fu[fa];
             ub = fu[fb];
             ptid = tid[s];
         }
-        if (__ballot(mine && ni < 0) & gbits) {   // a hull link: the cell is infinite
-            st = G_HULL;
-            mine = false;
-        }
         const unsigned code = PENDING + (unsigned)gl;
         int e = 0;
-        if (mine) e = table_take<6>(T, ni, ((unsigned)ni << 6) | code);
-        bool bad = mine && e < 0;
+        if (mine) e = table_take(T, ni, ((unsigned)ni << 6) | code);
+        bool bad = false, hull = false;
         wave_sync();
-        const unsigned te = T[e < 0 ? 0 : e];
-        const bool lead = mine && !bad && (te & 63u) == code;
-        const unsigned long long Lb = __ballot(lead) & gbits;
-        const int slot = S + __popcll(Lb & below);
-        S += __popcll(Lb);
+        const unsigned te = T[e];
+        const bool lead = mine && (te & 63u) == code;
+        const unsigned Lb = half(__ballot(lead));
+        const int slot = S + __popc(Lb & gbelow);
+        S += __popc(Lb & ghalf);
         if (S > SG || 2 * S - hc > 2 * QUEUE) st = G_DEFER;
         const bool take = lead && st == G_RUN;
         int jp = 0, ev = 0, up = 0;
@@ -258,33 +276,39 @@ __global__ __launch_bounds__(64) void k_cell_geom(CellSet<MULTI> set, PlaneBuf p
             // shared ones; where it holds the three, and its neighbours there
             up = (int)((unsigned)rv.x + (unsigned)rv.y + (unsigned)rv.z + (unsigned)rv.w -
                        (unsigned)v - (unsigned)ua - (unsigned)ub);
-            int ia, ib, ip, na, nbb, np;
-            find4(rv, rn, ua, ia, na);
-            find4(rv, rn, ub, ib, nbb);
-            find4(rv, rn, up, ip, np);
-            const bool ab = ia < ib, ap = ia < ip, bp = ib < ip;
-            // not a tet on that face, or one that does not link back
-            bad = ia == ib || ia == ip || ib == ip || np != ptid;
-            jp = (ap ? 1 : 0) + (bp ? 1 : 0);
-            const int ja = (ab ? 0 : 1) + (ap ? 0 : 1), jb = (ab ? 1 : 0) + (bp ? 0 : 1);
+            // its link vertices l and the neighbours m across them, in order
+            const bool v0 = rv.x == v, v1 = v0 || rv.y == v, v2 = v1 || rv.z == v;
+            const int l0 = v0 ? rv.y : rv.x, l1 = v1 ? rv.z : rv.y, l2 = v2 ? rv.w : rv.z;
+            const int m0 = v0 ? rn.y : rn.x, m1 = v1 ? rn.z : rn.y, m2 = v2 ? rn.w : rn.z;
+            const bool p0 = l0 == up, p2 = l2 == up;   // the apex: first, last, or second
+            jp = p0 ? 0 : (p2 ? 2 : 1);
+            const int first = p0 ? l1 : l0, second = p2 ? l1 : l2;
+            const int np = p0 ? m0 : (p2 ? m2 : m1);
+            const int na = p0 ? m1 : m0, nbb = p2 ? m1 : m2;
+            const bool fwd = first == ua;
+            // not a tet on that face, or one that does not link back (with
+            // the cell's vertex and the shared two in it, the apex is the
+            // fourth by its sum)
+            bad = !(v2 || rv.w == v) || first != (fwd ? ua : ub) || second != (fwd ? ub : ua) ||
+                  up == ua || up == ub || np != ptid;
             T[e] = (te & ~63u) | (unsigned)slot;
             tid[slot] = ni;
-            const int at = 2 * slot % (2 * QUEUE);
-            cand[at] = ab ? na : nbb;
-            cand[at + 1] = ab ? nbb : na;
-            wnew = ((unsigned)fa << (8 * ja)) | ((unsigned)fb << (8 * jb)) |
-                   ((unsigned)jp << 24);
+            const int at = 2 * (slot - (slot >= QUEUE ? QUEUE : 0));
+            cand[at] = na;
+            cand[at + 1] = nbb;
+            wnew = ((unsigned)(fwd ? fa : fb) << (p0 ? 8 : 0)) |
+                   ((unsigned)(fwd ? fb : fa) << (p2 ? 8 : 16)) | ((unsigned)jp << 24);
+            hull = (na | nbb) < 0;   // a hull link: the cell is infinite
             nb[3 * slot + jp] = (unsigned char)s;
-            ev = table_take<5>(V, up, ((unsigned)up << 6) | code);
-            bad = bad || ev < 0;
+            ev = table_take(V, up, ((unsigned)up << 6) | code);
         }
         wave_sync();
         // new apexes: face numbers in slot (lane) order
         const unsigned ve = V[take && !bad ? ev : 0];
         const bool leadv = take && !bad && (ve & 63u) == code;
-        const unsigned long long Lv = __ballot(leadv) & gbits;
-        const int fnew = F + __popcll(Lv & below);
-        F += __popcll(Lv);
+        const unsigned Lv = half(__ballot(leadv));
+        const int fnew = F + __popc(Lv & gbelow);
+        F += __popc(Lv & ghalf);
         if (F > FG) st = G_DEFER;
         if (leadv && st == G_RUN) {
             V[ev] = (ve & ~63u) | (unsigned)fnew;
@@ -302,8 +326,11 @@ __global__ __launch_bounds__(64) void k_cell_geom(CellSet<MULTI> set, PlaneBuf p
             nb[3 * s + j] = (unsigned char)sl;
             bad = bad || tid[sl] != ni;    // another tet with the same tag
         }
-        if (__ballot(bad) & gbits) st = G_DEFER;
-        hc += min(G, ncand - hc);
+        if (__ballot(bad || hull)) {
+            if (__ballot(hull) & gbits) st = G_HULL;
+            if (__ballot(bad) & gbits) st = G_DEFER;
+        }
+        hc = min(hc + G, ncand);
         wave_sync();
     }
 
@@ -328,15 +355,13 @@ __global__ __launch_bounds__(64) void k_cell_geom(CellSet<MULTI> set, PlaneBuf p
         }
     }
     if (PLANES) {
-#pragma unroll
-        for (int off = G / 2; off >= 1; off >>= 1) {   // stays inside the group
-            mnx = fminf(mnx, __shfl_xor(mnx, off));
-            mny = fminf(mny, __shfl_xor(mny, off));
-            mnz = fminf(mnz, __shfl_xor(mnz, off));
-            mxx = fmaxf(mxx, __shfl_xor(mxx, off));
-            mxy = fmaxf(mxy, __shfl_xor(mxy, off));
-            mxz = fmaxf(mxz, __shfl_xor(mxz, off));
-        }
+        static_assert(G == 16, "a group is a row of lanes");
+        mnx = min16(mnx);
+        mny = min16(mny);
+        mnz = min16(mnz);
+        mxx = -min16(-mxx);
+        mxy = -min16(-mxy);
+        mxz = -min16(-mxz);
     }
     wave_sync();
     if (PLANES && st == G_RUN) {
@@ -388,7 +413,8 @@ __global__ __launch_bounds__(64) void k_cell_geom(CellSet<MULTI> set, PlaneBuf p
             for (;;) {
                 // circulate_next (src/tet.cpp:185-215): the next vertex is the
                 // link vertex that is not u or behind
-                const int nv = (int)__builtin_amdgcn_sad_u8(w & 0xffffffu, 0u, 0u) - f - behind;
+                const int nv = (int)__builtin_amdgcn_udot4(w, 0x010101u, (unsigned)(-f - behind),
+                                                           false);
                 const int nt = qn[3 * t + wi];
                 if (nt == us) break;
                 w = qf[nt];
