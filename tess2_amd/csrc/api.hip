@@ -1288,10 +1288,9 @@ static int enqueue_kernels(tess2_ctx *c, const RunArgs &a)
                     launch_fill_u32((unsigned *)d.npts, (size_t)d.norig, 0u, s);
                 }
             }
-            launch_hash_build(d.pts, d.np, d.hash, d.hstart, d.hsums, d.hbk, d.hsorted,
-                              multi ? d.hkey : nullptr, s);
-            launch_exact_status(in, gp, d.status_ex, a.precision, d.ctrs,
-                                reinterpret_cast<unsigned char *>(d.exflags), s);
+            launch_exact_setup(in, gp, d.np, d.hash, d.hstart, d.hsums, d.hbk, d.hsorted,
+                               multi ? d.hkey : nullptr, d.status_ex, a.precision, d.ctrs,
+                               reinterpret_cast<unsigned char *>(d.exflags), s);
         }
         if (ev) HIPCHK(c, hipEventRecord(c->ev_k0, s));
         for (int k = 0; k < nb; ++k) {

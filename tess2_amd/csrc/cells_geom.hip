@@ -27,9 +27,9 @@
 // hold a slot (or face number), or 48 + lane while a round decides who takes
 // it; atomicMin leaves the lowest.  Each user then compares the slot's full id, so
 // two ids that share 26 bits only defer the cell.
-// What bounds it: vector instructions, about 450 a cell, three fifths of them in
-// the star's rounds (2.1M cells of a GRF box with planes: 1.86 ms, 24 GB of
-// tets at 32 B out of the caches; volumes of 216k cells 188 us, of 64k 64).
+// What bounds it: vector instructions, about 400 a cell, more than half of them in
+// the star's rounds (2.1M cells of a GRF box with planes: 1.86 ms; volumes of
+// 216k cells 188 us, of 64k 64).
 // Each table probe, index and mask in a round is therefore the cheapest form
 // that holds: tables of 64 words that cannot fill up (with 32 words for the
 // vertices and a probe count 2.04 ms, 219 and 74 us), 24-bit hash products,

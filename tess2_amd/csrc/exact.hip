@@ -40,10 +40,11 @@ __device__ __forceinline__ int bucket_of(float4 p, const HashP &h)
 
 // bucket of every particle and its rank there (in no set order: the searches
 // decide ties by id)
-__global__ void k_hash_count(const float4 *__restrict__ pts, int np, HashP h,
-                             unsigned *__restrict__ cnt, int2 *__restrict__ bk)
+__device__ __forceinline__ void hash_count(int wg, const float4 *__restrict__ pts, int np,
+                                           const HashP &h, unsigned *__restrict__ cnt,
+                                           int2 *__restrict__ bk)
 {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    const int p = wg * 256 + threadIdx.x;
     if (p >= np) return;
     const int b = bucket_of(pts[p], h);
     bk[p] = make_int2(b, (int)atomicAdd(&cnt[b], 1u));
@@ -51,31 +52,18 @@ __global__ void k_hash_count(const float4 *__restrict__ pts, int np, HashP h,
 
 // the fourth word is the particle's id: its index, or with several blocks
 // its home key (rank << 23 | cell), which also breaks distance ties
-__global__ void k_hash_scatter(const float4 *__restrict__ pts, int np,
-                               const int2 *__restrict__ bk, const unsigned *__restrict__ start,
-                               float4 *__restrict__ sorted, const int *__restrict__ key)
+__device__ __forceinline__ void hash_scatter(int wg, const float4 *__restrict__ pts, int np,
+                                             const int2 *__restrict__ bk,
+                                             const unsigned *__restrict__ start,
+                                             float4 *__restrict__ sorted,
+                                             const int *__restrict__ key)
 {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    const int p = wg * 256 + threadIdx.x;
     if (p >= np) return;
     const int2 b = bk[p];
     const float4 q = pts[p];
     sorted[start[b.x] + (unsigned)b.y] =
         make_float4(q.x, q.y, q.z, __int_as_float(key ? key[p] : p));
-}
-
-// start: one word more than there are buckets (the extra one turns into the
-// total)
-void launch_hash_build(const float4 *pts, int np, const HashP &h, unsigned *start,
-                       unsigned *sums, int2 *bk, float4 *sorted, const int *key, hipStream_t s)
-{
-    const int nbk = h.dims[0] * h.dims[1] * h.dims[2];
-    if (np > 0)
-        hipLaunchKernelGGL(k_hash_count, dim3((np + 255) / 256), dim3(256), 0, s, pts, np, h,
-                           start, bk);
-    launch_scan_u32(start, (unsigned)nbk + 1u, sums, s);
-    if (np > 0)
-        hipLaunchKernelGGL(k_hash_scatter, dim3((np + 255) / 256), dim3(256), 0, s, pts, np, bk,
-                           (const unsigned *)start, sorted, key);
 }
 
 // ---------------------------------------------------------------------------
@@ -502,8 +490,9 @@ __device__ __forceinline__ int comp4(const int4 &q, int i)
     return i == 0 ? q.x : (i == 1 ? q.y : (i == 2 ? q.z : q.w));
 }
 
-__global__ void k_exact_flags(BlockIn in, GridP gp, int prec, unsigned char *__restrict__ flags,
-                              unsigned *ctrs)
+__device__ __forceinline__ void exact_flags(int wg, int nwg, const BlockIn &in, const GridP &gp,
+                                            int prec, unsigned char *__restrict__ flags,
+                                            unsigned *ctrs)
 {
     const int nc = in.ncells;
     unsigned char *inc = flags, *out = flags + nc, *def = flags + 2 * (size_t)nc;
@@ -518,8 +507,7 @@ __global__ void k_exact_flags(BlockIn in, GridP gp, int prec, unsigned char *__r
     if (threadIdx.x == 0) s_fb = 0;
     __syncthreads();
     unsigned nfb = 0;   // FP64 re-checks of this lane
-    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < in.ntets;
-         t += gridDim.x * blockDim.x) {
+    for (int t = wg * 256 + threadIdx.x; t < in.ntets; t += nwg * 256) {
         const int4 vv = in.tets[2 * t];
         if (vv.x >= nc && vv.y >= nc && vv.z >= nc && vv.w >= nc) continue;   // ghosts only
         const int4 nb = in.tets[2 * t + 1];
@@ -583,10 +571,11 @@ __global__ void k_exact_flags(BlockIn in, GridP gp, int prec, unsigned char *__r
     if (threadIdx.x == 0 && s_fb) atomicAdd(&ctrs[C_FALLBACK], s_fb);
 }
 
-__global__ void k_exact_classify(const int *__restrict__ v2t, int nc,
-                                 const unsigned char *__restrict__ flags, int *status)
+__device__ __forceinline__ void exact_classify(int wg, const int *__restrict__ v2t, int nc,
+                                               const unsigned char *__restrict__ flags,
+                                               int *status)
 {
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
+    const int v = wg * 256 + threadIdx.x;
     if (v >= nc) return;
     int st;
     if (v2t[v] < 0 || flags[v]) st = EX_INCOMPLETE;
@@ -596,16 +585,52 @@ __global__ void k_exact_classify(const int *__restrict__ v2t, int nc,
     status[v] = st;
 }
 
-void launch_exact_status(const BlockIn &in, const GridP &gp, int *status, int prec, unsigned *ctrs,
-                         unsigned char *flags, hipStream_t s)
+// What the owner search needs, in two launches with the scan of the bucket
+// counts between: the bucket hash (the first bh workgroups) and the deposit
+// status of each cell.  The two are independent, and for small blocks each
+// step is a launch of 3 to 4 us (4,000 cells on 49^3, whole run: 153 us
+// apart, 143 together).
+__global__ __launch_bounds__(256) void k_exact_count(BlockIn in, GridP gp, int prec,
+                                                     unsigned char *__restrict__ flags,
+                                                     unsigned *ctrs, int np, HashP h,
+                                                     unsigned *__restrict__ cnt,
+                                                     int2 *__restrict__ bk, int bh)
 {
-    if (in.ncells <= 0) return;
-    if (in.ntets > 0) {
-        const int blocks = std::min(4096, (in.ntets + 255) / 256);
-        hipLaunchKernelGGL(k_exact_flags, dim3(blocks), dim3(256), 0, s, in, gp, prec, flags, ctrs);
-    }
-    hipLaunchKernelGGL(k_exact_classify, dim3((in.ncells + 255) / 256), dim3(256), 0, s, in.v2t,
-                       in.ncells, (const unsigned char *)flags, status);
+    if ((int)blockIdx.x < bh) hash_count((int)blockIdx.x, in.pts, np, h, cnt, bk);
+    else exact_flags((int)blockIdx.x - bh, (int)gridDim.x - bh, in, gp, prec, flags, ctrs);
+}
+
+__global__ __launch_bounds__(256) void k_exact_place(BlockIn in,
+                                                     const unsigned char *__restrict__ flags,
+                                                     int *status, int np,
+                                                     const int2 *__restrict__ bk,
+                                                     const unsigned *__restrict__ start,
+                                                     float4 *__restrict__ sorted,
+                                                     const int *__restrict__ key, int bh)
+{
+    if ((int)blockIdx.x < bh) hash_scatter((int)blockIdx.x, in.pts, np, bk, start, sorted, key);
+    else exact_classify((int)blockIdx.x - bh, in.v2t, in.ncells, flags, status);
+}
+
+// start: one word more than there are buckets (the extra one turns into the
+// total)
+void launch_exact_setup(const BlockIn &in, const GridP &gp, int np, const HashP &h,
+                        unsigned *start, unsigned *sums, int2 *bk, float4 *sorted, const int *key,
+                        int *status, int prec, unsigned *ctrs, unsigned char *flags,
+                        hipStream_t s)
+{
+    const int nbk = h.dims[0] * h.dims[1] * h.dims[2];
+    const int bh = (np + 255) / 256;
+    const int bt = in.ncells > 0 ? std::min(4096, (in.ntets + 255) / 256) : 0;
+    const int bc = (in.ncells + 255) / 256;
+    if (bh + bt > 0)
+        hipLaunchKernelGGL(k_exact_count, dim3(bh + bt), dim3(256), 0, s, in, gp, prec, flags,
+                           ctrs, np, h, start, bk, bh);
+    launch_scan_u32(start, (unsigned)nbk + 1u, sums, s);
+    if (bh + bc > 0)
+        hipLaunchKernelGGL(k_exact_place, dim3(bh + bc), dim3(256), 0, s, in,
+                           (const unsigned char *)flags, status, np, (const int2 *)bk,
+                           (const unsigned *)start, sorted, key, bh);
 }
 
 // ---------------------------------------------------------------------------

@@ -245,9 +245,13 @@ hipError_t copy_to_device(void *dst, const void *src, size_t bytes, hipStream_t 
 // circumcenters; cc.w = error bound of the float solve (inf when undefined)
 void launch_circumcenters(const float4 *pts, const int4 *tets, int ntets, float4 *cc,
                           hipStream_t s);
-// start, npts and flags below are zero on entry
-void launch_hash_build(const float4 *pts, int np, const HashP &h, unsigned *start,
-                       unsigned *sums, int2 *bk, float4 *sorted, const int *key, hipStream_t s);
+// bucket hash of the np particles and the cells' deposit status; start, flags
+// (3 * ncells bytes: incomplete, outside, defined) and the counts below are
+// zero on entry
+void launch_exact_setup(const BlockIn &in, const GridP &gp, int np, const HashP &h,
+                        unsigned *start, unsigned *sums, int2 *bk, float4 *sorted, const int *key,
+                        int *status, int prec, unsigned *ctrs, unsigned char *flags,
+                        hipStream_t s);
 // npts_tab / stex_tab (by rank) when several blocks share the assignment,
 // else nullptr; defq: queue of defq_cap grid points for the FP64 re-search
 // of the mixed precision (0: searched inline)
@@ -255,9 +259,6 @@ void launch_owner(const GridP &gp, const HashP &h, const unsigned *start, const 
                   int *owner, int prec, unsigned *ctrs, const int *status, int *npts,
                   int ncells, int *const *npts_tab, const int *const *stex_tab, unsigned *defq,
                   unsigned defq_cap, hipStream_t s);
-// flags: 3 * ncells bytes (incomplete, outside, defined)
-void launch_exact_status(const BlockIn &in, const GridP &gp, int *status, int prec,
-                         unsigned *ctrs, unsigned char *flags, hipStream_t s);
 // parts: 1 = densities of the owned points, 2 = CIC of cells that own none;
 // every block's part 1 must precede any block's part 2
 void launch_exact_tail(const BlockIn &in, const GridP &gp, const int *owner,
