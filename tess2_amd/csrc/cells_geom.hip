@@ -27,8 +27,9 @@
 // hold a slot (or face number), or 48 + lane while a round decides who takes
 // it; atomicMin leaves the lowest.  Each user then compares the slot's full id, so
 // two ids that share 26 bits only defer the cell.
-// What bounds it: vector instructions, about 400 a cell, more than half of them in
-// the star's rounds (2.1M cells of a GRF box with planes: 1.86 ms; volumes of
+// What bounds it: vector instructions, 604 a cell, more than half of them in
+// the star's rounds (2.1M cells of a GRF box with planes: 1.80 to 1.86 ms, one
+// instruction per SIMD in 3.5 cycles; volumes of
 // 216k cells 188 us, of 64k 64).
 // Each table probe, index and mask in a round is therefore the cheapest form
 // that holds: tables of 64 words that cannot fill up (with 32 words for the

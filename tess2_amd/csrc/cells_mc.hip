@@ -1,4 +1,6 @@
-// cells_mc.hip -- the single-block cell kernel with several cells per wave.
+// cells_mc.hip -- the cell kernel with two cells per wave: single blocks of
+// up to 16384 cells (above, the geometry and scan kernels of cells_geom.hip
+// and cells_scan.hip), eps < 0, or on request.
 //
 // One 64-lane wavefront takes CPW consecutive cells (in the block's Morton
 // order), G = 64 / CPW lanes per cell, for the geometry phase, where one

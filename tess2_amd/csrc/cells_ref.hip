@@ -1,4 +1,6 @@
-// cells_ref.hip -- gfx950 kernels of the reference-exact density path.
+// cells_ref.hip -- gfx950 kernels of the reference-exact density path, one
+// cell per wave: volumes of up to 4096 cells, the large-capacity pass of every
+// other cell kernel, the CIC estimator; whole runs on request.
 //
 // One 64-lane wavefront handles one Voronoi cell (one original particle):
 //   1. star: level-synchronous BFS over the tets around the site, starting at

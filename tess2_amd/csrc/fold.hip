@@ -7,9 +7,8 @@
 // (src/dense.cpp:290).  The cell kernels record the first and second
 // contribution of a point next to the point and append later ones to a
 // shared list; this pass replays the additions of every point that got more
-// than one in ascending key order (key = cell id, or the received-point key
-// above 2^31):
-// (points with exactly two are added by the pass that ends the run):
+// than two in ascending key order (key = cell id, or the received-point key
+// above 2^31; the pass that ends the run adds the points with two):
 //   1. gather: each larger point (through its representative list entry,
 //      the third contribution) reserves a contiguous segment, sized by its
 //      contribution count, is filed in one of three classes by that count,
