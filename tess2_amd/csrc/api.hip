@@ -205,9 +205,11 @@ static int cell_kernel_for(const tess2_ctx *c, int ncells, unsigned long long ng
 // 64 per workgroup) rather than a one-pass cell kernel: always for several
 // blocks (8 Plummer blocks, 57k cells on 128^3: 1.74 -> 0.74 ms; 11k cells on
 // 9 x 10 x 11: 0.96 -> 0.31), for one block from 16384 cells on.  Below that
-// their waves are too few to hide their longer chains: 4000 cells on 31^3
-// 0.153 against 0.123 ms, 16000 on 25^3 0.181 against 0.218, on 50^3 0.186
-// against 0.176, on 100^3 0.397 against 0.486; 262k on 128^3 0.61 against 0.95.
+// their waves are too few to hide their longer chains (run without volumes, in
+// us): 4000 cells on 23^3 115 against 108, on 32^3 120 against 103, on 48^3 172
+// against 136; 10000 on 31^3 120 and 121, on 65^3 198 against 162; 16000 on
+// 25^3 145 against 196, on 50^3 146 and 150, on 76^3 213 against 202, on 101^3
+// 308 against 600; 262k on 128^3 610 against 950.
 static bool split_cells(const tess2_ctx *c, float eps, int nb, int ncells)
 {
     return c->cell_kernel < 0 && eps >= 0.0f && (nb > 1 || ncells >= 16384);
