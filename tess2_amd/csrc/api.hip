@@ -785,6 +785,7 @@ static int stage_block(tess2_ctx *c, const tess2_block_t &hb, DevBlock &d, bool 
         d.hash.lo[i] = lo[i];
         d.hash.dims[i] = (int)((hi[i] - lo[i]) / cell) + 1;
     }
+    d.hash.slack = bucket_slack(std::max({d.hash.dims[0], d.hash.dims[1], d.hash.dims[2]}));
     const size_t nbk = (size_t)d.hash.dims[0] * d.hash.dims[1] * d.hash.dims[2];
     if ((r = dalloc(c, &d.hstart, nbk + 1)) ||
         (r = dalloc(c, &d.hsums, scan_sums_words(nbk + 1))) ||

@@ -1,0 +1,45 @@
+// buckets.hpp -- the bucket hash's geometry: the bucket of a position, and how
+// near the positions of a bucket can be (includable without the HIP headers).
+#pragma once
+
+#include <cmath>
+
+namespace t2 {
+
+// uniform bucket hash of the particles: bucket (i,j,k) holds the particles
+// with floor((x - lo) * inv) == (i,j,k), clamped to the grid of dims buckets
+struct HashP {
+    float lo[3];
+    float inv;      // 1 / cell
+    float cell;
+    int dims[3];
+    float slack;    // cells a position can lie outside its bucket (bucket_slack)
+};
+
+__host__ __device__ __forceinline__ int bucket_index(float q, float lo, float inv, int dim)
+{
+    const int i = (int)floorf((q - lo) * inv);
+    return i < 0 ? 0 : (i >= dim ? dim - 1 : i);
+}
+
+// The float arithmetic of bucket_index and bucket_gap is off by a few ulp of
+// the bucket number: a position lies up to that much outside its bucket.
+__host__ __device__ __forceinline__ float bucket_slack(int most_buckets)
+{
+    return 0.001f + 4.8e-7f * (float)most_buckets;
+}
+
+// Distance on one axis from [a, b] (relative to the hash's origin) to the
+// positions of bucket i: no position of the bucket is nearer by more than a
+// few ulp of the distance.  Relative to the origin, since a difference of
+// absolute edges is off by an ulp of the coordinate, more than the slack where the
+// box lies far from zero (6e-5 at 1000; the slack of 200,000 particles in a
+// unit box is 1.7e-5).
+__host__ __device__ __forceinline__ float bucket_gap(float a, float b, int i, const HashP &h)
+{
+    const float left = (float)i * h.cell, right = (float)(i + 1) * h.cell;
+    const float d = fmaxf(0.0f, fmaxf(left - b, a - right)) - h.slack * h.cell;
+    return fmaxf(0.0f, d);
+}
+
+}  // namespace t2

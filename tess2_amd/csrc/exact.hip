@@ -27,15 +27,10 @@ enum { EX_DEPOSIT = 0, EX_INCOMPLETE = 2, EX_OUTSIDE = 3, EX_DEGENERATE = 4 };
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ int bucket_of(float4 p, const HashP &h)
 {
-    int c[3];
-    const float q[3] = {p.x, p.y, p.z};
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        int ci = (int)floorf((q[i] - h.lo[i]) * h.inv);
-        ci = ci < 0 ? 0 : (ci >= h.dims[i] ? h.dims[i] - 1 : ci);
-        c[i] = ci;
-    }
-    return (c[2] * h.dims[1] + c[1]) * h.dims[0] + c[0];
+    const int x = bucket_index(p.x, h.lo[0], h.inv, h.dims[0]);
+    const int y = bucket_index(p.y, h.lo[1], h.inv, h.dims[1]);
+    const int z = bucket_index(p.z, h.lo[2], h.inv, h.dims[2]);
+    return (z * h.dims[1] + y) * h.dims[0] + x;
 }
 
 // bucket of every particle and its rank there (in no set order: the searches
@@ -110,10 +105,7 @@ __device__ __forceinline__ void home_bucket(float gx, float gy, float gz, const 
 {
     const float q[3] = {gx, gy, gz};
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        int ci = (int)floorf((q[i] - h.lo[i]) * h.inv);
-        c[i] = ci < 0 ? 0 : (ci >= h.dims[i] ? h.dims[i] - 1 : ci);
-    }
+    for (int i = 0; i < 3; ++i) c[i] = bucket_index(q[i], h.lo[i], h.inv, h.dims[i]);
 }
 
 // search in double; returns the owner id
@@ -150,10 +142,9 @@ __device__ int nearest_f64(float gx, float gy, float gz, const HashP &h,
                 }
             }
         }
-        // every bucket beyond shell r is at least r*h away
-        // (r - 0.001) cells: the bucket of a point near a bucket face can be
-        // off by ~1e-4 of a cell through the float bucket arithmetic
-        const double lb = ((double)r - 0.001) * (double)h.cell;
+        // every bucket beyond shell r is at least r cells away, less what the
+        // float bucket arithmetic can be off
+        const double lb = fmax(0.0, (double)r - (double)h.slack) * (double)h.cell;
         if (bid != 0x7fffffff && r > 0 && lb * lb > best * (1.0 + 1e-9) + 1e-300) break;
     }
     return bid;
@@ -209,13 +200,15 @@ __device__ __forceinline__ void tile_search(const Tile &t, const HashP &h,
         c0[a] = __builtin_amdgcn_readfirstlane(c0[a]);
         c1[a] = __builtin_amdgcn_readfirstlane(c1[a]);
     }
-    // distance of the box to bucket i's slab on axis a, short of it by the
-    // ~1e-4 of a cell that the float bucket arithmetic can be off
-    const float slack = 0.001f * h.cell;
-    auto gap = [&](int i, int a) {
-        const float b = h.lo[a] + (float)i * h.cell;
-        return fmaxf(0.0f, fmaxf(b - t.hi[a], t.lo[a] - (b + h.cell)) - slack);
-    };
+    // the box relative to the hash's origin, and its distance to bucket i on
+    // axis a
+    float lo[3], hi[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        lo[a] = uniform_f(t.lo[a] - h.lo[a]);
+        hi[a] = uniform_f(t.hi[a] - h.lo[a]);
+    }
+    auto gap = [&](int i, int a) { return bucket_gap(lo[a], hi[a], i, h); };
     auto run = [&](unsigned s0, unsigned s1) {
         unsigned s = s0;
         for (; s + 4 <= s1; s += 4) {
@@ -276,9 +269,10 @@ __device__ __forceinline__ void tile_search(const Tile &t, const HashP &h,
                 if (e0 < e1) run(e0, e1);
             }
         }
-        m2 = (double)reach();
+        // the squared gaps are floats: a few ulp more
+        m2 = (double)reach() * (1.0 + 2e-6);
         // every bucket beyond shell r is at least r cells from the box
-        const double lb = ((double)r - 0.001) * (double)h.cell;
+        const double lb = fmax(0.0, (double)r - (double)h.slack) * (double)h.cell;
         if (r > 0 && lb * lb > m2) break;
     }
 }

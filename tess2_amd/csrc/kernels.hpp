@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <cstdint>
 
+#include "buckets.hpp"
+
 namespace t2 {
 
 // Grid and block parameters of one dense run on one block (host-computed
@@ -79,15 +81,6 @@ struct CellOut {
     BlockStats *st;    // this block's record (st->ctrs == ctrs)
     unsigned long long ngrid;
     int ncells;
-};
-
-// uniform bucket hash of the particles: bucket (i,j,k) holds the particles
-// with floor((x - lo) * inv) == (i,j,k), clamped to the grid of dims buckets
-struct HashP {
-    float lo[3];
-    float inv;      // 1 / cell
-    float cell;
-    int dims[3];
 };
 
 // Per-block grids and outputs of all blocks of a run, in staging order (the
