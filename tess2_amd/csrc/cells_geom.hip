@@ -103,14 +103,6 @@ __device__ __forceinline__ float min16(float x)
     return lesser(x, dpp_f<0x140>(x));   // mirrored sixteens
 }
 
-// orders the compiler's LDS accesses around lanes' exchanges through LDS (a
-// wave's LDS instructions execute in order)
-__device__ __forceinline__ void wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 // first entry to look at in a table of 64 words: the top bits of a 24-bit
 // product (a full-rate multiplication; consecutive ids fall far apart)
 __device__ __forceinline__ unsigned table_first(int id)

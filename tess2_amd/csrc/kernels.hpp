@@ -215,6 +215,15 @@ __device__ __forceinline__ int hash_find(int *hk, int key)
     return -1;
 }
 
+// orders a wave's LDS accesses where its lanes exchange values through LDS (its
+// LDS instructions execute in order; the fence keeps the compiler from
+// reusing or moving a load across, which the barrier alone does not)
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Workgroup -> work item with XCD affinity: the dispatcher hands consecutive
 // workgroups to the 8 XCDs in turn, so item k = (b % 8) * chunk + b / 8 gives
 // each XCD (and its L2) one contiguous range of items.  Returns -1 for the

@@ -297,9 +297,9 @@ __global__ __launch_bounds__(256) void k_sort_scatter(const unsigned *__restrict
                 id_out[slot] = v[r];
             }
         }
-        __builtin_amdgcn_wave_barrier();   // every lane has read its counter
+        wave_sync();   // every lane has read its counter
         if (on && (same & below) == 0ull) s_c[w][d] += (unsigned)__popcll(same);
-        __builtin_amdgcn_wave_barrier();
+        wave_sync();
     }
 }
 
