@@ -342,6 +342,9 @@ template <bool MULTI>
 __global__ __launch_bounds__(64) void k_cell_scan_big(CellSet<MULTI> set, PlaneBuf pb)
 {
     constexpr int RMAX = 64;
+    static_assert(alignof(LineShared) >= alignof(int4) &&
+                      sizeof(LineShared::row) >= RMAX * sizeof(int4),
+                  "the runs overlay the lines");
     __shared__ LineShared sl;
     __shared__ float4 s_fa[PLANE_STRIDE];
     __shared__ float2 s_fb[PLANE_STRIDE];

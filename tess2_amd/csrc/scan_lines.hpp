@@ -141,7 +141,8 @@ __device__ __forceinline__ float cic_corner(const float4 site, float scalar, con
 // one wave's cell: lines, runs, and the points of a turn
 struct LineShared {
     static constexpr int ROWS = 1024, POINTS = 2048;
-    unsigned row[ROWS], run[ROWS];
+    alignas(16) unsigned row[ROWS];   // also taken as int4 runs by scan_deposit
+    unsigned run[ROWS];
     unsigned short list[POINTS];
 };
 
