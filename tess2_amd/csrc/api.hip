@@ -722,11 +722,15 @@ static int stage_block(tess2_ctx *c, const tess2_block_t &hb, DevBlock &d, bool 
             e = hipMemcpyAsync(c->h_info, c->d_info, sizeof(StageInfo) * nrec,
                                hipMemcpyDeviceToHost, s);
     }
-    // the caller's arrays are read until here
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    // the caller's arrays are read until here, by the copies before one that
+    // failed too
+    const hipError_t es = hipStreamSynchronize(s);
+    if (e == hipSuccess) e = es;
     dfree(c, xyz);
-    if (e != hipSuccess)
+    if (e != hipSuccess) {
+        (void)hipGetLastError();   // reported here, not by the next call
         return fail(c, TESS2_E_HIP, "block %d: upload: %s", d.gid, hipGetErrorString(e));
+    }
     bool bad = false, odd = false;
     float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
     for (int k = 0; k < nrec; ++k) {
@@ -1900,11 +1904,15 @@ extern "C" int tess2_ghost_sends(tess2_ctx *c, const tess2_block_t *block, int n
             e = hipMemcpyAsync(sends, dsend, sizeof(unsigned long long) * d.norig,
                                hipMemcpyDeviceToHost, s);
     }
-    if (!r && e == hipSuccess) e = hipStreamSynchronize(s);
+    const hipError_t es = hipStreamSynchronize(s);   // also of the boxes, after an error
+    if (e == hipSuccess) e = es;
     dfree(c, dbox);
     dfree(c, dsend);
     if (r) return r;
-    HIPCHK(c, e);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return fail(c, TESS2_E_HIP, "ghost test: %s", hipGetErrorString(e));
+    }
     return 0;
 }
 

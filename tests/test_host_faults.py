@@ -1,0 +1,84 @@
+"""The library's host paths on a HIP runtime without a GPU (fake_hip.py): what
+a failed copy, allocation or thread leaves behind, what a run keeps from the run
+before, and which kernels a choice reaches."""
+import shutil
+
+import numpy as np
+import pytest
+
+from tess2_amd import _native as N
+from tess2_amd import build as B
+from tess2_amd import host as D
+from tess2_amd import ingest
+from tests import fake_hip as F
+
+E_HIP, E_NOMEM = -2, -4
+MIB = 1 << 20
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    try:
+        B.hipcc()
+    except RuntimeError:
+        pytest.skip("hipcc missing")
+    if shutil.which("g++") is None:
+        pytest.skip("g++ missing")
+    return F.load(F.build(str(tmp_path_factory.mktemp("fake"))))
+
+
+@pytest.fixture
+def fake(lib, monkeypatch):
+    monkeypatch.setattr(N, "_lib", lib)
+    # a context collected later would be closed by another library
+    monkeypatch.setattr(N.Context, "__del__", lambda self: None)
+    lib.fake_reset()
+    yield lib
+    lib.fake_reset()
+
+
+def _block(n, seed=1, gid=0):
+    """n particles without ghosts or neighbours, enough for the host code."""
+    rng = np.random.default_rng(seed)
+    p = rng.random((n, 3), dtype=np.float32)
+    t = np.full((n, 8), -1, np.int32)
+    t[:, :4] = np.arange(4)
+    hb = ingest.HostBlock(p, t, np.zeros(n, np.int32), n, np.zeros(3, np.float32),
+                          np.ones(3, np.float32))
+    hb.gid = gid
+    return hb
+
+
+def _stage(ctx, blocks):
+    cs = (N.Block * len(blocks))()
+    keep = []
+    for i, hb in enumerate(blocks):
+        cs[i], k = N.make_block(hb)
+        keep.append(k)
+    return N.lib().tess2_stage(ctx.h, cs, len(blocks)), keep
+
+
+# ---- failed copies ----------------------------------------------------------
+@pytest.mark.parametrize("nth", [1, 2, 3])
+def test_failed_upload_leaves_no_copy_of_the_callers_arrays(fake, nth):
+    """The caller may free its arrays when an error is returned."""
+    ctx = N.Context(0)
+    fake.fake_fail_copy(nth)
+    r, _ = _stage(ctx, [_block(1000)])
+    assert r == E_HIP
+    assert fake.fake_pending() == 0
+    fake.fake_fail_copy(-1)
+    assert _stage(ctx, [_block(1000)])[0] == 0
+
+
+def test_failed_ghost_test_leaves_no_copy_of_the_boxes(fake):
+    hb = _block(1000)
+    boxes = np.zeros((3, 6), np.float32)
+    ctx = N.Context(0)
+    D.ghost_sends(hb, boxes, ctx=ctx)
+    n = fake.fake_copies()
+    fake.fake_fail_copy(n - 1)          # the last copy of a call: the result
+    with pytest.raises(N.Tess2Error):
+        D.ghost_sends(hb, boxes, ctx=ctx)
+    assert fake.fake_pending() == 0
+    D.ghost_sends(hb, boxes, ctx=ctx)
