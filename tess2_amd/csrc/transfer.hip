@@ -12,8 +12,8 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
 
 namespace t2 {
@@ -138,7 +138,7 @@ hipError_t copy(void *host, void *dev, size_t bytes, bool up, hipStream_t s)
     try {
         for (; started < j.workers; ++started)
             th[started] = std::thread([&j, started] { work(j, started); });
-    } catch (const std::system_error &) {   // no more threads: their pieces follow below
+    } catch (const std::exception &) {   // no thread or memory: their pieces follow below
     }
     work(j, 0);
     for (int w = 1; w < started; ++w) th[w].join();

@@ -82,3 +82,20 @@ def test_failed_ghost_test_leaves_no_copy_of_the_boxes(fake):
         D.ghost_sends(hb, boxes, ctx=ctx)
     assert fake.fake_pending() == 0
     D.ghost_sends(hb, boxes, ctx=ctx)
+
+
+def test_no_memory_for_copy_threads(fake):
+    """A large copy goes on with the threads that started."""
+    run = D.StagedRun([_block(500)])
+    g = (256, 256, 128)
+    run.run(g)
+    run.sync()
+    out = np.ones(g[0] * g[1] * g[2], np.float32)
+    assert N.lib().tess2_fetch(run.ctx.h, 0, out.ctypes.data, None, None) == 0
+    out[:] = 1.0
+    for n in range(4):      # the threads' own states
+        fake.fake_fail_new(n)
+        r = N.lib().tess2_fetch(run.ctx.h, 0, out.ctypes.data, None, None)
+        fake.fake_fail_new(-1)
+        assert r == 0 and not out.any()
+        out[:] = 1.0
