@@ -111,9 +111,20 @@ hipError_t plain(void *host, void *dev, size_t bytes, bool up, hipStream_t s)
     return e == hipSuccess && !up ? hipStreamSynchronize(s) : e;
 }
 
+// memory that the device does not reach by itself (pinned, managed and device
+// memory take one plain copy)
+bool pageable(const void *p)
+{
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+    (void)hipGetLastError();
+    return true;
+}
+
 hipError_t copy(void *host, void *dev, size_t bytes, bool up, hipStream_t s)
 {
-    if (bytes < (up ? LEAST_UP : LEAST_DOWN)) return plain(host, dev, bytes, up, s);
+    if (bytes < (up ? LEAST_UP : LEAST_DOWN) || !pageable(host))
+        return plain(host, dev, bytes, up, s);
     Slots &q = slots();
     std::unique_lock<std::mutex> lk(q.mu, std::try_to_lock);
     if (!lk.owns_lock()) return plain(host, dev, bytes, up, s);

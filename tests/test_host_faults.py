@@ -1,6 +1,7 @@
 """The library's host paths on a HIP runtime without a GPU (fake_hip.py): what
 a failed copy, allocation or thread leaves behind, what a run keeps from the run
 before, and which kernels a choice reaches."""
+import ctypes as C
 import shutil
 
 import numpy as np
@@ -99,3 +100,27 @@ def test_no_memory_for_copy_threads(fake):
         fake.fake_fail_new(-1)
         assert r == 0 and not out.any()
         out[:] = 1.0
+
+
+# ---- pinned arrays ----------------------------------------------------------
+def test_pinned_arrays_are_copied_directly(fake):
+    """An array the device reaches by itself needs no slots in between."""
+    n = (20 << 20) // 32                       # tets above the least upload in slots
+    hb = _block(n)
+    t = fake.fake_pinned(hb.tets.nbytes)
+    C.memmove(t, hb.tets.ctypes.data, hb.tets.nbytes)
+    b, keep = N.make_block(hb)
+    b.tets = t
+    ctx = N.Context(0)
+    assert N.lib().tess2_stage(ctx.h, C.byref(b), 1) == 0
+    direct = fake.fake_copies()
+    assert direct == 4                         # three arrays up, the check's record down
+
+    run = D.StagedRun([_block(500)])
+    g = (256, 256, 128)
+    run.run(g)
+    run.sync()
+    d = fake.fake_pinned(4 * g[0] * g[1] * g[2])
+    before = fake.fake_copies()
+    assert N.lib().tess2_fetch(run.ctx.h, 0, d, None, None) == 0
+    assert fake.fake_copies() == before + 1
