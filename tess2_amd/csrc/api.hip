@@ -800,6 +800,39 @@ static int stage_block(tess2_ctx *c, const tess2_block_t &hb, DevBlock &d, bool 
     return 0;
 }
 
+// descriptors, statistics and work lists of the staged blocks
+static int stage_descriptors(tess2_ctx *c)
+{
+    int r = 0;
+    const size_t nblocks = c->blocks.size();
+    if ((r = dalloc(c, &c->d_ins, nblocks)) || (r = dalloc(c, &c->d_gps, nblocks)) ||
+        (r = dalloc(c, &c->d_outs, nblocks)) || (r = dalloc(c, &c->d_router, 1)) ||
+        (r = dalloc(c, &c->d_queue, 16)) || (r = dalloc(c, &c->d_stats, nblocks)) ||
+        (r = dalloc(c, &c->d_gpart, nblocks * RUN_PARTS)))
+        return r;
+    // counters and statistics of all blocks: one device array, one pinned
+    // host copy (so that the copy can sit in a captured graph)
+    if ((int)nblocks > c->h_stats_cap) {
+        if (c->h_stats) (void)hipHostFree(c->h_stats);
+        c->h_stats = nullptr;
+        c->h_stats_cap = 0;
+        if (hipHostMalloc((void **)&c->h_stats, sizeof(BlockStats) * nblocks,
+                          hipHostMallocDefault) != hipSuccess)
+            return fail(c, TESS2_E_NOMEM, "pinned host buffer");
+        c->h_stats_cap = (int)nblocks;
+    }
+    memset(c->h_stats, 0, sizeof(BlockStats) * nblocks);
+    for (size_t k = 0; k < nblocks; ++k) {
+        DevBlock &d = c->blocks[k];
+        d.st = c->d_stats + k;
+        d.ctrs = d.st->ctrs;
+        d.hm = c->h_stats + k;
+    }
+    // work lists and home keys of multi-block runs
+    if (nblocks > 1 && !(r = build_chunks(c))) r = build_home_keys(c);
+    return r;
+}
+
 // layout: the caller's next run reads the tets (else the order is made by the
 // first run that does, prepare_run)
 static int stage_blocks(tess2_ctx *c, const tess2_block_t *blocks, int nblocks, bool layout)
@@ -865,34 +898,8 @@ static int stage_blocks(tess2_ctx *c, const tess2_block_t *blocks, int nblocks, 
     if (r) return r;
     drop_old();
     c->blocks.swap(fresh);
-    if (nblocks > 0) {
-        if ((r = dalloc(c, &c->d_ins, (size_t)nblocks)) || (r = dalloc(c, &c->d_gps, (size_t)nblocks)) ||
-            (r = dalloc(c, &c->d_outs, (size_t)nblocks)) || (r = dalloc(c, &c->d_router, 1)) ||
-            (r = dalloc(c, &c->d_queue, 16)) || (r = dalloc(c, &c->d_stats, (size_t)nblocks)) ||
-            (r = dalloc(c, &c->d_gpart, (size_t)nblocks * RUN_PARTS)))
-            return r;
-        // counters and statistics of all blocks: one device array, one pinned
-        // host copy (so that the copy can sit in a captured graph)
-        if (nblocks > c->h_stats_cap) {
-            if (c->h_stats) (void)hipHostFree(c->h_stats);
-            c->h_stats = nullptr;
-            c->h_stats_cap = 0;
-            if (hipHostMalloc((void **)&c->h_stats, sizeof(BlockStats) * nblocks,
-                              hipHostMallocDefault) != hipSuccess)
-                return fail(c, TESS2_E_NOMEM, "pinned host buffer");
-            c->h_stats_cap = nblocks;
-        }
-        memset(c->h_stats, 0, sizeof(BlockStats) * nblocks);
-        for (int k = 0; k < nblocks; ++k) {
-            DevBlock &d = c->blocks[k];
-            d.st = c->d_stats + k;
-            d.ctrs = d.st->ctrs;
-            d.hm = c->h_stats + k;
-        }
-        // work lists and home keys of multi-block runs
-        if (nblocks > 1 && ((r = build_chunks(c)) || (r = build_home_keys(c)))) return r;
-    }
-    return 0;
+    if (nblocks > 0 && (r = stage_descriptors(c))) drop_old();   // no run without them
+    return r;
 }
 
 extern "C" int tess2_stage(tess2_ctx *c, const tess2_block_t *blocks, int nblocks)
@@ -915,10 +922,13 @@ static int alloc_lists(tess2_ctx *c, DevBlock &d, unsigned cap)
     const size_t c3 = 3 * (size_t)cap;
     const unsigned c1 = (unsigned)(c3 / (FOLD_SMALL_MAX + 1) + 1),
                    c2 = (unsigned)(c3 / (FOLD_MID_MAX + 1) + 1);
+    d.ovf_cap = d.fold_cap[0] = d.fold_cap[1] = d.fold_cap[2] = 0;
     if ((r = dalloc(c, &d.ovf, (c3 + 1) / 2)) || (r = dalloc(c, &d.seg, c3)) ||
         (r = dalloc(c, &d.fold[0], cap)) || (r = dalloc(c, &d.fold[1], c1)) ||
-        (r = dalloc(c, &d.fold[2], c2)))
+        (r = dalloc(c, &d.fold[2], c2))) {
+        dfree(c, d.ovf);   // the next run starts over
         return r;
+    }
     d.ovf_cap = cap;
     d.fold_cap[0] = cap;
     d.fold_cap[1] = c1;
@@ -932,6 +942,7 @@ static int ensure_grid(tess2_ctx *c, DevBlock &d, size_t n, bool cic)
     d.ngrid = n;
     if (n > d.grid_cap) {
         int r = 0;
+        d.grid_cap = 0;   // a capacity only holds while its buffers do
         if ((r = dalloc(c, &d.density, n)) || (r = dalloc(c, &d.count, n)) ||
             (r = dalloc(c, &d.first, n)) || (r = dalloc(c, &d.second, n)) ||
             (r = dalloc(c, &d.head, n)))
@@ -1041,10 +1052,12 @@ static int build_route_table(tess2_ctx *c, Router &hr)
     }
     int r = 0;
     if (map.size() > c->rmap_cap) {
+        c->rmap_cap = 0;
         if ((r = dalloc(c, &c->d_rmap, map.size()))) return r;
         c->rmap_cap = map.size();
     }
     if (cand.size() > c->rcand_cap) {
+        c->rcand_cap = 0;
         if ((r = dalloc(c, &c->d_rcand, cand.size()))) return r;
         c->rcand_cap = cand.size();
     }
@@ -1074,6 +1087,10 @@ static int prepare_run(tess2_ctx *c, const RunArgs &a)
                 if (r) return r;
             }
     const int nb = (int)c->blocks.size();
+    if (nb > 1 && (!c->d_chunks || !c->d_tiles || !c->d_items)) {   // an option found no memory
+        const int r = build_chunks(c);
+        if (r) return r;
+    }
     const bool exact = a.alg == TESS2_DENSE_TESS && a.assignment == TESS2_ASSIGN_EXACT_VORONOI;
     if (exact && nb > 1 && !c->homes_ok)
         return fail(c, TESS2_E_ARG, "the exact assignment over several blocks: %s",
@@ -1120,9 +1137,9 @@ static int prepare_run(tess2_ctx *c, const RunArgs &a)
         int r = ensure_grid(c, d, n, a.alg == TESS2_DENSE_CIC);
         if (r) return r;
         if (exact && d.owner_cap < n) {
+            d.owner_cap = 0;
             r = dalloc(c, &d.owner, n);
             if (r) return r;
-            d.owner_cap = n;
             // a quarter of the grid (beyond it the search runs inline); the
             // queue holds 32-bit grid indices
             dfree(c, d.defq);
@@ -1133,6 +1150,7 @@ static int prepare_run(tess2_ctx *c, const RunArgs &a)
                 if (r) return r;
                 d.defq_cap = (unsigned)cap;
             }
+            d.owner_cap = n;
         }
         c->h_ins[k] = make_in(d);
         c->h_gps[k] = gp;
@@ -1485,6 +1503,7 @@ extern "C" int tess2_sync(tess2_ctx *c, tess2_stats_t *st)
                             "block %d: a cell exceeds the per-cell capacities", d.gid);
             if (d.hm->ctrs[C_ERR] & 1u) {
                 const unsigned want = std::max(2 * d.slow_cap, d.hm->ctrs[C_SLOW] + 1024u);
+                d.slow_cap = 0;
                 int r = dalloc(c, &d.slow, want);
                 if (r) return r;
                 d.slow_cap = want;

@@ -28,6 +28,7 @@ std::vector<Pending> pending;             // pageable sources not waited for
 
 // counters, by name in fake_count
 long n_malloc, n_copy, n_graph, n_sync, n_slot_copy;
+long n_bad;                               // launches with a buffer missing or too small
 // launches: number and cost (ms) by kind
 std::map<int, long> n_launch;
 std::map<int, double> cost;
@@ -59,6 +60,15 @@ void launch(int kind)
     (capturing ? graph_ms : now) += cost.count(kind) ? cost[kind] : 0.001;
 }
 
+// whether p has room for so many bytes; counted when not
+void need(const void *p, size_t bytes)
+{
+    std::lock_guard<std::mutex> lk(mu);
+    auto it = device.upper_bound((char *)p);
+    if (it != device.begin() && (--it, (char *)p + bytes <= it->first + it->second)) return;
+    ++n_bad;
+}
+
 enum { K_OTHER = 0, K_GEOM = 1, K_SCAN = 2, K_REF_BATCHED = 3, K_MC_BATCHED = 4, K_MC_ITEMS = 5,
        K_REF = 6, K_MC = 7 };
 
@@ -74,7 +84,7 @@ void fake_reset()
     fail_new = -1;
     last_error = hipSuccess;
     pending.clear();
-    n_malloc = n_copy = n_graph = n_sync = n_slot_copy = 0;
+    n_malloc = n_copy = n_graph = n_sync = n_slot_copy = n_bad = 0;
     n_launch.clear();
     cost.clear();
 }
@@ -88,6 +98,7 @@ long fake_copies() { return n_copy; }
 long fake_pinned_copies() { return n_slot_copy; }
 long fake_graphs() { return n_graph; }
 long fake_mallocs() { return n_malloc; }
+long fake_bad_launches() { return n_bad; }
 void *fake_pinned(size_t bytes)
 {
     void *p = nullptr;
@@ -258,9 +269,14 @@ void launch_circumcenters(const float4 *, const int4 *, int, float4 *, hipStream
 void launch_exact_setup(const BlockIn &, const GridP &, int, const HashP &, unsigned *, unsigned *,
                         int2 *, float4 *, const int *, int *, int, unsigned *, unsigned char *,
                         hipStream_t) { launch(K_OTHER); }
-void launch_owner(const GridP &, const HashP &, const unsigned *, const float4 *, int *, int,
-                  unsigned *, const int *, int *, int, int *const *, const int *const *, unsigned *,
-                  unsigned, hipStream_t) { launch(K_OTHER); }
+void launch_owner(const GridP &gp, const HashP &, const unsigned *, const float4 *, int *owner, int,
+                  unsigned *, const int *, int *, int, int *const *, const int *const *,
+                  unsigned *defq, unsigned defq_cap, hipStream_t)
+{
+    launch(K_OTHER);
+    need(owner, 4 * (size_t)gp.bnum_idx[0] * gp.bnum_idx[1] * gp.bnum_idx[2]);
+    if (defq_cap) need(defq, 4 * (size_t)defq_cap);
+}
 void launch_exact_tail(const BlockIn &, const GridP &, const int *, const int *, const CellOut &,
                        int, int *const *, const int *const *, const Router *, int, int,
                        hipStream_t) { launch(K_OTHER); }
@@ -269,8 +285,25 @@ void launch_ghost_sends(const float4 *, const int4 *, int, int, const float *, c
                         const float *, int, int, unsigned long long *, hipStream_t) { launch(K_OTHER); }
 void launch_device_block(const float *, int, const int4 *, int, const int *, float4 *, float4 *,
                          unsigned *, unsigned *, unsigned, hipStream_t) { launch(K_OTHER); }
-void launch_run_prep(const BlockIn *, const CellOut *, int, int, unsigned long long,
-                     const ZeroList &, hipStream_t) { launch(K_OTHER); }
+void launch_run_prep(const BlockIn *, const CellOut *outs, int nb, int, unsigned long long,
+                     const ZeroList &z, hipStream_t)
+{
+    launch(K_OTHER);
+    for (int b = 0; b < nb; ++b) {
+        const CellOut &o = outs[b];
+        need(o.density, 4 * o.ngrid);
+        need(o.count, 4 * o.ngrid);
+        need(o.first, 8 * o.ngrid);
+        need(o.second, 8 * o.ngrid);
+        need(o.head, 4 * o.ngrid);
+        need(o.slow, 4 * (size_t)o.slow_cap);
+        need(o.ovf, 24 * (size_t)o.ovf_cap);
+        need(o.seg, 24 * (size_t)o.ovf_cap);
+        for (int k = 0; k < 3; ++k) need(o.fold[k], 16 * (size_t)o.fold_cap[k]);
+    }
+    for (int k = 0; k < 4; ++k)
+        if (z.n[k]) need(z.p[k], 4 * z.n[k]);
+}
 void launch_cells_ref(const BlockIn &, const GridP &, const CellOut &, int, hipStream_t)
 {
     launch(K_REF);

@@ -23,6 +23,7 @@ CONTROL = {
     "fake_pinned_copies": (C.c_long, []),
     "fake_graphs": (C.c_long, []),
     "fake_mallocs": (C.c_long, []),
+    "fake_bad_launches": (C.c_long, []),         # with a buffer missing or too small
     "fake_pinned": (C.c_void_p, [C.c_size_t]),
 }
 (K_OTHER, K_GEOM, K_SCAN, K_REF_BATCHED, K_MC_BATCHED, K_MC_ITEMS, K_REF, K_MC) = range(8)

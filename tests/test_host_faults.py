@@ -124,3 +124,51 @@ def test_pinned_arrays_are_copied_directly(fake):
     before = fake.fake_copies()
     assert N.lib().tess2_fetch(run.ctx.h, 0, d, None, None) == 0
     assert fake.fake_copies() == before + 1
+
+
+# ---- failed allocations -----------------------------------------------------
+@pytest.mark.parametrize("mib", [0, 10, 40, 75, 140, 200, 210])
+def test_run_after_a_run_without_memory(fake, mib):
+    """A run on a larger grid finds no memory part of the way; the smaller grid
+    then runs on buffers that are all there."""
+    run = D.StagedRun([_block(2000)])
+    kw = dict(assignment=D.EXACT_VORONOI, want_volumes=False)
+    run.run((33, 33, 33), **kw)
+    run.sync()
+    fake.fake_limit(mib * MIB)
+    with pytest.raises(N.Tess2Error, match="out of device memory"):
+        run.run((200, 200, 200), **kw)
+    fake.fake_limit(2 ** 64 - 1)
+    run.run((33, 33, 33), **kw)
+    run.sync()
+    run.run((20, 20, 20))
+    run.sync()
+    assert fake.fake_bad_launches() == 0
+
+
+def test_run_after_a_staging_without_memory(fake):
+    """Whatever allocation of a staging fails, the next run has all its buffers
+    (the blocks staged before) or is refused."""
+    blocks = [_block(300, 1, 0), _block(200, 2, 1)]
+    ctx = N.Context(0)
+    g = N.i3((9, 9, 9))
+
+    def run():
+        r = N.lib().tess2_run(ctx.h, 0, 0, N.f3(None), N.f3(None), 0, N.f3((0, 0, 1)), 1.0, 1e-4,
+                              g, 0, 0, 0)
+        return r or N.lib().tess2_sync(ctx.h, None)
+
+    refused = staged = 0
+    for kib in range(0, 1500, 8):
+        fake.fake_limit(kib << 10)
+        r, _ = _stage(ctx, blocks)
+        fake.fake_limit(2 ** 64 - 1)
+        assert r in (0, E_NOMEM)
+        staged += r == 0
+        if run():
+            assert b"no staged blocks" in N.lib().tess2_last_error(ctx.h)
+            refused += 1
+        assert fake.fake_bad_launches() == 0
+        N.lib().tess2_destroy(ctx.h)        # the next without buffers of this one
+        ctx = N.Context(0)
+    assert refused and staged
