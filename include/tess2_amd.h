@@ -270,7 +270,7 @@ enum {
     TESS2_OPT_CHUNK_SMALL = 2,    /* cells per work item, blocks with < 20000 cells */
     TESS2_OPT_CHUNK_MEDIUM = 3,   /* cells per work item, blocks with < 100000 cells */
     TESS2_OPT_CHUNK_LARGE = 4,    /* cells per work item, larger blocks */
-    TESS2_OPT_CELL_KERNEL = 5     /* cell kernel: -1 (default) chosen per run (several blocks,
+    TESS2_OPT_CELL_KERNEL = 5,    /* cell kernel: -1 (default) chosen per run (several blocks,
                                    * or 16384 cells and more: a geometry kernel and a scan
                                    * kernel over all cells; else 1, or 2 when cell boxes are
                                    * not small, 6 or more grid points per cell); 0 one cell
@@ -285,10 +285,16 @@ enum {
                                    * two cells per wave as 2 (one block runs 2);
                                    * with the option at -1, tess2_autotune also times
                                    * 3, 1 and 4 and keeps the fastest */
+    TESS2_OPT_PLANE_TILES = 6     /* tiles of 64 cells whose face planes are in memory at a
+                                   * time between the geometry and the scan kernel (42 KB a
+                                   * tile), 1..32768 (default 32768); a run of more tiles
+                                   * takes them in turns.  Without memory for its planes a
+                                   * run halves the number, and at last takes the one-pass
+                                   * kernels */
 };
 
 /* Set / read one option.  Chunk sizes 1..4096, waves per CU 1..64, cell
- * kernel -1..4. */
+ * kernel -1..4, plane tiles 1..32768. */
 int tess2_set_option(tess2_ctx *ctx, int option, int value);
 int tess2_get_option(tess2_ctx *ctx, int option, int *value);
 

@@ -55,6 +55,13 @@ static unsigned char *scratch_ptr(int device)
 
 namespace {
 
+// tiles per launch of the geometry and scan kernels at most: 2M cells, 664
+// bytes of planes each (fewer tiles cost their tails: 2.1M cells in 4 turns
+// 3.04 ms, in one 2.88).  Without memory for those of a run, half as many at a
+// time, down to PLANE_LEAST (44 MB); then the one-pass kernels, which take
+// twice the time and hold no planes.
+constexpr int PLANE_TILES = 1 << 15, PLANE_LEAST = 1 << 10;
+
 struct DevBlock {
     int gid = 0, norig = 0, np = 0, nt = 0;
     float bmin[3] = {0, 0, 0}, bmax[3] = {0, 0, 0};
@@ -144,7 +151,10 @@ struct tess2_ctx {
     CellTile *d_tiles = nullptr;         // 64 cells of one block each (several blocks)
     int ntiles = 0;
     PlaneBuf planes{};                   // cell planes of one launch, plane_tiles tiles
-    int plane_tiles = 0;
+    int plane_tiles = 0, plane_turns = 0;
+    int plane_opt = PLANE_TILES;         // tiles a launch at most (tess2_set_option), and
+    int plane_most = PLANE_TILES;        // as far as there was memory since the last staging
+    bool split = false;                  // the run takes the geometry and scan kernels
     std::vector<BlockIn> h_ins;
     std::vector<GridP> h_gps;
     std::vector<CellOut> h_outs;
@@ -214,10 +224,6 @@ static bool split_cells(const tess2_ctx *c, float eps, int nb, int ncells)
 {
     return c->cell_kernel < 0 && eps >= 0.0f && (nb > 1 || ncells >= 16384);
 }
-
-// tiles per launch of those kernels: 2M cells, 664 bytes of planes each
-// (fewer tiles cost their tails: 2.1M cells in 4 turns 3.04 ms, in one 2.88)
-static constexpr int PLANE_TILES = 1 << 15;
 
 static void drop_graph(tess2_ctx *c)
 {
@@ -352,6 +358,16 @@ static void free_block(tess2_ctx *c, DevBlock &b)
     b = DevBlock();
 }
 
+static void free_planes(tess2_ctx *c)
+{
+    dfree(c, c->planes.hdr);
+    dfree(c, c->planes.fa);
+    dfree(c, c->planes.fb);
+    dfree(c, c->planes.big);
+    dfree(c, c->planes.nbig);
+    c->plane_tiles = c->plane_turns = 0;
+}
+
 static void free_multi(tess2_ctx *c)
 {
     dfree(c, c->d_ins);
@@ -364,12 +380,9 @@ static void free_multi(tess2_ctx *c)
     dfree(c, c->d_items);
     dfree(c, c->d_queue);
     dfree(c, c->d_tiles);
-    dfree(c, c->planes.hdr);
-    dfree(c, c->planes.fa);
-    dfree(c, c->planes.fb);
-    dfree(c, c->planes.big);
-    dfree(c, c->planes.nbig);
-    c->ntiles = c->plane_tiles = 0;
+    free_planes(c);
+    c->plane_most = c->plane_opt;
+    c->ntiles = 0;
     dfree(c, c->d_stats);
     dfree(c, c->d_gpart);
     dfree(c, c->d_npts_tab);
@@ -1073,6 +1086,38 @@ static int build_route_table(tess2_ctx *c, Router &hr)
     return 0;
 }
 
+// tiles of all staged cells
+static int run_tiles(const tess2_ctx *c)
+{
+    return c->blocks.size() > 1 ? c->ntiles : (c->blocks[0].norig + CELL_TILE - 1) / CELL_TILE;
+}
+
+// Planes for the nt tiles of a run in equal turns of at most plane_most;
+// false when there is no memory for them.
+static bool ensure_planes(tess2_ctx *c, int nt)
+{
+    PlaneBuf &p = c->planes;
+    while (c->plane_most > 0) {
+        const int turns = std::max(1, (nt + c->plane_most - 1) / c->plane_most);
+        const int most = std::max(1, (nt + turns - 1) / turns);
+        if (most <= c->plane_tiles && turns <= c->plane_turns) return true;
+        const size_t n = (size_t)most * CELL_TILE;
+        c->plane_tiles = c->plane_turns = 0;
+        if (!dalloc(c, &p.hdr, 2 * n) && !dalloc(c, &p.fa, n * PLANE_STRIDE) &&
+            !dalloc(c, &p.fb, n * PLANE_STRIDE) && !dalloc(c, &p.big, n) &&
+            !dalloc(c, &p.nbig, (size_t)turns)) {
+            c->plane_tiles = most;
+            c->plane_turns = turns;
+            return true;
+        }
+        free_planes(c);
+        drop_spare(c);
+        const int half = (most + 1) / 2;
+        c->plane_most = half >= PLANE_LEAST ? half : 0;
+    }
+    return false;
+}
+
 // enqueue the whole path for every staged block
 // host-side set-up of a run: grid parameters, buffers, device descriptors
 static int prepare_run(tess2_ctx *c, const RunArgs &a)
@@ -1156,23 +1201,8 @@ static int prepare_run(tess2_ctx *c, const RunArgs &a)
         c->h_gps[k] = gp;
         c->h_outs[k] = make_out(d, a.want_vol != 0);
     }
-    if (a.alg == TESS2_DENSE_TESS && !exact && split_cells(c, a.eps, nb, c->blocks[0].norig)) {
-        int nt = c->ntiles;
-        if (nb == 1) nt = (c->blocks[0].norig + CELL_TILE - 1) / CELL_TILE;
-        const int chunks = (nt + PLANE_TILES - 1) / PLANE_TILES;
-        const int most = std::min(nt, PLANE_TILES);
-        if (most > c->plane_tiles) {
-            const size_t n = (size_t)most * CELL_TILE;
-            PlaneBuf &p = c->planes;
-            int r = 0;
-            c->plane_tiles = 0;
-            if ((r = dalloc(c, &p.hdr, 2 * n)) || (r = dalloc(c, &p.fa, n * PLANE_STRIDE)) ||
-                (r = dalloc(c, &p.fb, n * PLANE_STRIDE)) || (r = dalloc(c, &p.big, n)) ||
-                (r = dalloc(c, &p.nbig, (size_t)chunks)))
-                return r;
-            c->plane_tiles = most;
-        }
-    }
+    c->split = a.alg == TESS2_DENSE_TESS && !exact &&
+               split_cells(c, a.eps, nb, c->blocks[0].norig) && ensure_planes(c, run_tiles(c));
     if (c->desc_gen == c->gen && same_args(a, c->desc_args)) return 0;   // unchanged
     if (nb > 1) {
         // XCD ranges of the item list by estimated cost: a cell, plus its
@@ -1216,16 +1246,15 @@ static int prepare_run(tess2_ctx *c, const RunArgs &a)
     return 0;
 }
 
-// geometry, then scan and deposit, of all cells of a scan run, at most
-// PLANE_TILES tiles at a time (planes.nbig is zero on entry)
+// geometry, then scan and deposit, of all cells of a scan run, plane_tiles
+// tiles at a time (planes.nbig is zero on entry)
 template <bool MULTI>
 static void enqueue_split(tess2_ctx *c, CellSet<MULTI> set, int ntiles, hipStream_t s)
 {
-    const int chunks = (ntiles + PLANE_TILES - 1) / PLANE_TILES;
     PlaneBuf pb = c->planes;
-    for (int k = 0; k < chunks; ++k, ++pb.nbig) {
-        set.tile0 = k * PLANE_TILES;
-        set.ntiles = std::min(PLANE_TILES, ntiles - set.tile0);
+    for (int t0 = 0; t0 < ntiles; t0 += c->plane_tiles, ++pb.nbig) {
+        set.tile0 = t0;
+        set.ntiles = std::min(c->plane_tiles, ntiles - t0);
         launch_cell_geom(set, pb, 1, s);
         launch_cell_scan(set, pb, s);
     }
@@ -1257,9 +1286,7 @@ static int enqueue_kernels(tess2_ctx *c, const RunArgs &a)
 
     // phase A: clear per-block outputs and counters, circumcenters, and the
     // arrays that phase B adds to
-    const bool split = a.alg == TESS2_DENSE_TESS && !exact &&
-                       split_cells(c, a.eps, nb, c->blocks[0].norig);
-    const int ntiles = nb > 1 ? c->ntiles : (c->blocks[0].norig + CELL_TILE - 1) / CELL_TILE;
+    const int ntiles = run_tiles(c);
     {
         int mt = 0;
         unsigned long long mg = 0;
@@ -1270,9 +1297,9 @@ static int enqueue_kernels(tess2_ctx *c, const RunArgs &a)
         ZeroList z{};
         z.p[0] = reinterpret_cast<unsigned *>(c->d_stats);
         z.n[0] = sizeof(BlockStats) / 4 * (unsigned long long)nb;
-        if (split) {
+        if (c->split) {
             z.p[1] = c->planes.nbig;
-            z.n[1] = (unsigned long long)((ntiles + PLANE_TILES - 1) / PLANE_TILES);
+            z.n[1] = (unsigned long long)c->plane_turns;
         }
         if (exact && nb == 1) {
             const DevBlock &d = c->blocks[0];
@@ -1340,7 +1367,7 @@ static int enqueue_kernels(tess2_ctx *c, const RunArgs &a)
             launch_cic(c->h_ins[k], c->h_gps[k], c->h_outs[k], nb > 1 ? c->d_router : nullptr, k,
                        s);
         if (ev) HIPCHK(c, hipEventRecord(c->ev_k1, s));
-    } else if (split) {
+    } else if (c->split) {
         if (ev) HIPCHK(c, hipEventRecord(c->ev_k0, s));
         if (nb == 1)
             enqueue_split(c, CellSet<false>{c->h_ins[0], c->h_outs[0], c->d_gps, 0, 0},
@@ -1589,6 +1616,14 @@ extern "C" int tess2_set_option(tess2_ctx *c, int option, int value)
         if (value != c->cell_kernel) c->gen++;   // a recorded graph is recorded again
         c->cell_kernel = value;
         return 0;
+    case TESS2_OPT_PLANE_TILES:
+        if (value < 1 || value > PLANE_TILES)
+            return fail(c, TESS2_E_ARG, "plane tiles: 1..%d", PLANE_TILES);
+        if (value == c->plane_opt) return 0;
+        c->plane_opt = c->plane_most = value;
+        c->gen++;
+        free_planes(c);
+        return 0;
     case TESS2_OPT_CHUNK_SMALL: chunk = &c->chunk_small; break;
     case TESS2_OPT_CHUNK_MEDIUM: chunk = &c->chunk_medium; break;
     case TESS2_OPT_CHUNK_LARGE: chunk = &c->chunk_large; break;
@@ -1610,6 +1645,7 @@ extern "C" int tess2_get_option(tess2_ctx *c, int option, int *value)
     case TESS2_OPT_CHUNK_MEDIUM: *value = c->chunk_medium; return 0;
     case TESS2_OPT_CHUNK_LARGE: *value = c->chunk_large; return 0;
     case TESS2_OPT_CELL_KERNEL: *value = c->cell_kernel; return 0;
+    case TESS2_OPT_PLANE_TILES: *value = c->plane_opt; return 0;
     default: return fail(c, TESS2_E_ARG, "unknown option %d", option);
     }
 }

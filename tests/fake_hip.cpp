@@ -312,8 +312,25 @@ void launch_cells_ref_slow(const BlockIn &, const GridP &, const CellOut &, int,
 {
     launch(K_OTHER);
 }
-void launch_cell_geom(const CellSet<false> &, const PlaneBuf &, int, hipStream_t) { launch(K_GEOM); }
-void launch_cell_geom(const CellSet<true> &, const PlaneBuf &, int, hipStream_t) { launch(K_GEOM); }
+static void geom(int ntiles, const PlaneBuf &pb, int want_density)
+{
+    launch(K_GEOM);
+    if (!want_density) return;
+    const size_t n = (size_t)ntiles * CELL_TILE;
+    need(pb.hdr, 32 * n);
+    need(pb.fa, 16 * n * PLANE_STRIDE);
+    need(pb.fb, 8 * n * PLANE_STRIDE);
+    need(pb.big, 8 * n);
+    need(pb.nbig, 4);
+}
+void launch_cell_geom(const CellSet<false> &set, const PlaneBuf &pb, int want_density, hipStream_t)
+{
+    geom(set.ntiles, pb, want_density);
+}
+void launch_cell_geom(const CellSet<true> &set, const PlaneBuf &pb, int want_density, hipStream_t)
+{
+    geom(set.ntiles, pb, want_density);
+}
 void launch_cell_scan(const CellSet<false> &, const PlaneBuf &, hipStream_t) { launch(K_SCAN); }
 void launch_cell_scan(const CellSet<true> &, const PlaneBuf &, hipStream_t) { launch(K_SCAN); }
 int launch_cells_mc(const BlockIn &, const GridP *, const CellOut &, int, int, hipStream_t)

@@ -172,3 +172,51 @@ def test_run_after_a_staging_without_memory(fake):
         N.lib().tess2_destroy(ctx.h)        # the next without buffers of this one
         ctx = N.Context(0)
     assert refused and staged
+
+
+def _runs(run, g=(9, 9, 9)):
+    run.run(g, want_volumes=False)
+    run.sync()
+
+
+def test_planes_without_memory(fake):
+    """The planes between the geometry and the scan kernel (4097 tiles of 42 KB)
+    are held in fewer tiles at a time where memory is short, and a run that finds
+    none takes the one-pass kernel, as it did without planes."""
+    n = 64 * 4096 + 1
+    hb = _block(n)
+    turns = {}
+    for mib in (400, 100, 60, 30, 0):
+        run = D.StagedRun([hb])
+        run.set_option("cell_kernel", 1)        # all other buffers
+        _runs(run)
+        run.set_option("cell_kernel", -1)
+        fake.fake_limit(mib * MIB)
+        before = [fake.fake_launches(k) for k in (F.K_GEOM, F.K_SCAN, F.K_MC)]
+        _runs(run)
+        _runs(run)
+        fake.fake_limit(2 ** 64 - 1)
+        turns[mib] = [fake.fake_launches(k) - b
+                      for k, b in zip((F.K_GEOM, F.K_SCAN, F.K_MC), before)]
+        assert fake.fake_bad_launches() == 0
+        # the next staging has its planes again
+        assert _stage(run.ctx, [hb])[0] == 0
+        before = fake.fake_launches(F.K_GEOM)
+        _runs(run)
+        assert fake.fake_launches(F.K_GEOM) == before + 1
+        run.ctx.close()
+    assert turns == {400: [2, 2, 0], 100: [4, 4, 0], 60: [8, 8, 0], 30: [0, 0, 2], 0: [0, 0, 2]}
+
+
+def test_plane_turns_are_equal(fake):
+    run = D.StagedRun([_block(64 * 1000 + 5)])      # 1001 tiles
+    for most, turns in ((32768, 1), (1001, 1), (1000, 2), (400, 3), (1, 1001)):
+        run.set_option("plane_tiles", most)
+        assert run.get_option("plane_tiles") == most
+        before = fake.fake_launches(F.K_GEOM)
+        _runs(run)
+        assert fake.fake_launches(F.K_GEOM) - before == turns
+        assert fake.fake_bad_launches() == 0
+    for bad in (0, 32769):
+        with pytest.raises(N.Tess2Error):
+            run.set_option("plane_tiles", bad)
