@@ -940,6 +940,9 @@ static int alloc_lists(tess2_ctx *c, DevBlock &d, unsigned cap)
         (r = dalloc(c, &d.fold[0], cap)) || (r = dalloc(c, &d.fold[1], c1)) ||
         (r = dalloc(c, &d.fold[2], c2))) {
         dfree(c, d.ovf);   // the next run starts over
+        dfree(c, d.seg);
+        for (int k = 0; k < 3; ++k) dfree(c, d.fold[k]);
+        drop_spare(c);
         return r;
     }
     d.ovf_cap = cap;
@@ -968,9 +971,12 @@ static int ensure_grid(tess2_ctx *c, DevBlock &d, size_t n, bool cic)
         // the particles nearly all share a point: room for them (up to 16M
         // entries) spares the overflow and the second run (125k particles on
         // a 301^2 plane: about 190 us of a 2.0 ms call)
-        size_t cap = std::max<size_t>(1u << 16, n / 8);
+        const size_t least = std::max<size_t>(1u << 16, n / 8);
+        size_t cap = least;
         if (cic) cap = std::max(cap, std::min<size_t>(8 * (size_t)d.norig, 1u << 24));
         int r = alloc_lists(c, d, (unsigned)std::min<size_t>(cap, 1u << 30));
+        if (r == TESS2_E_NOMEM && cap > least)   // grows when a run overflows it
+            r = alloc_lists(c, d, (unsigned)std::min<size_t>(least, 1u << 30));
         if (r) return r;
     }
     return 0;

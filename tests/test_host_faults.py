@@ -220,3 +220,17 @@ def test_plane_turns_are_equal(fake):
     for bad in (0, 32769):
         with pytest.raises(N.Tess2Error):
             run.set_option("plane_tiles", bad)
+
+
+def test_cic_list_without_memory(fake):
+    """A CIC run's list holds eight contributions a cell where there is memory,
+    and starts as small as a scan's where there is not."""
+    hb = _block(400000)
+    for mib in (4000, 60):
+        run = D.StagedRun([hb])
+        fake.fake_limit(mib * MIB)
+        run.run((9, 9, 9), alg=D.DENSE_CIC)
+        run.sync()
+        fake.fake_limit(2 ** 64 - 1)
+        assert fake.fake_bad_launches() == 0
+        run.ctx.close()
