@@ -288,12 +288,12 @@ static void dfree(tess2_ctx *c, T *&p)
     c->spare.erase(c->spare.begin(), c->spare.begin() + (long)k);
 }
 
+// a buffer of one call, which no run and no captured graph refers to
 template <class T>
-static int dalloc(tess2_ctx *c, T **p, size_t n)
+static int dalloc_call(tess2_ctx *c, T **p, size_t n)
 {
     dfree(c, *p);
     if (n == 0) n = 1;
-    c->gen++;   // any captured graph refers to the old buffers
     // sizes in steps of an eighth of their power of two, so that calls of
     // similar size find each other's buffers
     size_t bytes = std::max<size_t>(n * sizeof(T), 256), step = 32;
@@ -324,6 +324,14 @@ static int dalloc(tess2_ctx *c, T **p, size_t n)
     }
     c->live[*p] = bytes;
     return 0;
+}
+
+// a buffer of the staged blocks or of their runs
+template <class T>
+static int dalloc(tess2_ctx *c, T **p, size_t n)
+{
+    c->gen++;   // any captured graph refers to the old buffers
+    return dalloc_call(c, p, n);
 }
 
 static void free_block(tess2_ctx *c, DevBlock &b)
@@ -1768,7 +1776,7 @@ extern "C" int tess2_fetch(tess2_ctx *c, int b, float *density, float *volumes,
     if (circumcenters && d.nt) {
         // packed on the device, in the caller's numbering
         float *tmp = nullptr;
-        const int r = dalloc(c, &tmp, 3 * (size_t)d.nt);
+        const int r = dalloc_call(c, &tmp, 3 * (size_t)d.nt);
         if (r) return r;
         launch_unpack_cc(d.cc, d.laid ? d.tet_new : nullptr, d.nt, tmp, c->stream);
         const hipError_t e = copy_to_host(circumcenters, tmp, 12 * (size_t)d.nt, c->stream);

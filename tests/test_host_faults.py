@@ -234,3 +234,25 @@ def test_cic_list_without_memory(fake):
         fake.fake_limit(2 ** 64 - 1)
         assert fake.fake_bad_launches() == 0
         run.ctx.close()
+
+
+# ---- what a run keeps -------------------------------------------------------
+@pytest.mark.parametrize("graph", [0, 1])
+@pytest.mark.parametrize("nb", [1, 2])
+def test_fetching_leaves_the_next_run_its_descriptors(fake, graph, nb):
+    """A steady state of run and fetch uploads nothing and records no graph
+    again, whatever is fetched."""
+    run = D.StagedRun([_block(500, k, k) for k in range(nb)])
+    run.set_option("graph", graph)
+    _runs(run)
+    _runs(run)
+    before = fake.fake_copies()
+    _runs(run)
+    steady, graphs = fake.fake_copies() - before, fake.fake_graphs()
+    for _ in range(3):
+        run.fetch(0, circumcenters=True)
+        run.cells(0)
+        before = fake.fake_copies()
+        _runs(run)
+        assert fake.fake_copies() - before == steady
+    assert fake.fake_graphs() == graphs
