@@ -302,7 +302,9 @@ int tess2_get_option(tess2_ctx *ctx, int option, int *value);
  * multi-block persistent cell kernel (chunk sizes x persistent waves per CU),
  * and, when TESS2_OPT_CELL_KERNEL is -1, the geometry and scan kernels and the
  * two-cell kernels (cell kernels 1 and 4), `reps` runs each, keep the fastest,
- * and leave it set.  Results of the staged blocks are those of the last timed
+ * and leave it set.  A cell kernel chosen here (tess2_get_option returns it)
+ * holds for several blocks, until the option is set or they are tuned again; a
+ * single block keeps the automatic choice.  Results of the staged blocks are those of the last timed
  * run (identical for every candidate).
  * best_ms (may be NULL) receives the fastest median run time. */
 int tess2_autotune(tess2_ctx *ctx, int reps, float *best_ms);

@@ -165,6 +165,7 @@ struct tess2_ctx {
     // cell per wave, 1 / 2 = two cells per wave in the geometry phase
     // (launch_cells_mc), 2 with the multi-word verdict masks
     int cell_kernel = -1;
+    bool ck_tuned = false;               // cell_kernel is tess2_autotune's choice
     // graph replay of the steady-state sequence (tess2_set_option)
     bool graph_on = false;
     hipGraphExec_t gexec = nullptr;
@@ -197,17 +198,24 @@ static bool same_args(const RunArgs &x, const RunArgs &y)
     return memcmp(&x, &y, sizeof(RunArgs)) == 0;
 }
 
-// The one-pass single-block cell kernel of a run: the option when set, else
+// The cell kernel option as it holds for a run over nb blocks (or volumes of
+// one): tess2_autotune chooses among the kernels for several.
+static int asked_kernel(const tess2_ctx *c, int nb)
+{
+    return nb == 1 && c->ck_tuned ? -1 : c->cell_kernel;
+}
+
+// The one-pass single-block cell kernel of a run: the one asked for, else
 // two cells per wave, with the multi-word verdict masks when cell boxes are
 // not small (6 or more grid points per cell: 4000 cells on 31^3 0.164 ->
 // 0.123 ms, on 15^3 0.147 and 0.148).
-static int cell_kernel_for(const tess2_ctx *c, int ncells, unsigned long long ngrid)
+static int cell_kernel_for(int asked, int ncells, unsigned long long ngrid)
 {
     // the multi-block choices; one block: one cell per wave, or two with
     // the multi-word masks
-    if (c->cell_kernel == 3) return 0;
-    if (c->cell_kernel == 4) return 2;
-    if (c->cell_kernel >= 0) return c->cell_kernel;
+    if (asked == 3) return 0;
+    if (asked == 4) return 2;
+    if (asked >= 0) return asked;
     return ngrid >= 6ull * (unsigned long long)std::max(ncells, 1) ? 2 : 1;
 }
 
@@ -220,9 +228,9 @@ static int cell_kernel_for(const tess2_ctx *c, int ncells, unsigned long long ng
 // against 136; 10000 on 31^3 120 and 121, on 65^3 198 against 162; 16000 on
 // 25^3 145 against 196, on 50^3 146 and 150, on 76^3 213 against 202, on 101^3
 // 308 against 600; 262k on 128^3 610 against 950.
-static bool split_cells(const tess2_ctx *c, float eps, int nb, int ncells)
+static bool split_cells(int asked, float eps, int nb, int ncells)
 {
-    return c->cell_kernel < 0 && eps >= 0.0f && (nb > 1 || ncells >= 16384);
+    return asked < 0 && eps >= 0.0f && (nb > 1 || ncells >= 16384);
 }
 
 static void drop_graph(tess2_ctx *c)
@@ -1216,7 +1224,7 @@ static int prepare_run(tess2_ctx *c, const RunArgs &a)
         c->h_outs[k] = make_out(d, a.want_vol != 0);
     }
     c->split = a.alg == TESS2_DENSE_TESS && !exact &&
-               split_cells(c, a.eps, nb, c->blocks[0].norig) && ensure_planes(c, run_tiles(c));
+               split_cells(asked_kernel(c, nb), a.eps, nb, c->blocks[0].norig) && ensure_planes(c, run_tiles(c));
     if (c->desc_gen == c->gen && same_args(a, c->desc_args)) return 0;   // unchanged
     if (nb > 1) {
         // XCD ranges of the item list by estimated cost: a cell, plus its
@@ -1275,12 +1283,12 @@ static void enqueue_split(tess2_ctx *c, CellSet<MULTI> set, int ntiles, hipStrea
 }
 
 // volume() of one block's cells (o.vol), the deferred ones too
-static void launch_volumes(const tess2_ctx *c, const BlockIn &in, const CellOut &o, hipStream_t s)
+static void launch_volumes(int asked, const BlockIn &in, const CellOut &o, hipStream_t s)
 {
     const GridP gp{};   // no density: the grid is not read
     // 4096 cells or fewer: a wave per cell, which ends soonest
-    const int ck = c->cell_kernel < 0 && in.ncells <= 4096 ? 0 : cell_kernel_for(c, in.ncells, 0);
-    if (split_cells(c, 0.0f, 1, in.ncells))
+    const int ck = asked < 0 && in.ncells <= 4096 ? 0 : cell_kernel_for(asked, in.ncells, 0);
+    if (split_cells(asked, 0.0f, 1, in.ncells))
         launch_cell_geom(CellSet<false>{in, o, nullptr, 0, (in.ncells + CELL_TILE - 1) / CELL_TILE},
                          PlaneBuf{}, 0, s);
     else if (ck == 0)
@@ -1335,7 +1343,8 @@ static int enqueue_kernels(tess2_ctx *c, const RunArgs &a)
         const bool multi = nb > 1;
         int *const *ntab = multi ? c->d_npts_tab : nullptr;
         const int *const *stab = multi ? c->d_stex_tab : nullptr;
-        if (a.want_vol && multi && c->cell_kernel < 0) {   // every block's volumes in one launch
+        const int asked = asked_kernel(c, nb);
+        if (a.want_vol && multi && asked < 0) {   // every block's volumes in one launch
             launch_cell_geom(CellSet<true>{c->d_ins, c->d_outs, c->d_gps, c->d_router, c->d_tiles,
                                            0, c->ntiles}, PlaneBuf{}, 0, s);
             launch_cells_ref_slow_batched(c->d_ins, c->d_router, 0, s);
@@ -1345,7 +1354,7 @@ static int enqueue_kernels(tess2_ctx *c, const RunArgs &a)
             const BlockIn &in = c->h_ins[k];
             const GridP &gp = c->h_gps[k];
             // volume() as the reference computes it
-            if (a.want_vol && !(multi && c->cell_kernel < 0)) launch_volumes(c, in, c->h_outs[k], s);
+            if (a.want_vol && !(multi && asked < 0)) launch_volumes(asked, in, c->h_outs[k], s);
             if (multi) {   // one block's are zero from the start
                 launch_fill_u32(d.hstart, (size_t)d.hash.dims[0] * d.hash.dims[1] *
                                 d.hash.dims[2] + 1, 0u, s);
@@ -1394,7 +1403,8 @@ static int enqueue_kernels(tess2_ctx *c, const RunArgs &a)
         else launch_cells_ref_slow_batched(c->d_ins, c->d_router, 1, s);
     } else if (nb == 1) {
         if (ev) HIPCHK(c, hipEventRecord(c->ev_k0, s));
-        const int ck = cell_kernel_for(c, c->blocks[0].norig, c->blocks[0].ngrid);
+        const int ck = cell_kernel_for(asked_kernel(c, 1), c->blocks[0].norig,
+                                       c->blocks[0].ngrid);
         if (ck == 0)
             launch_cells_ref(c->h_ins[0], c->h_gps[0], c->h_outs[0], 1, s);
         else if (launch_cells_mc(c->h_ins[0], c->d_gps, c->h_outs[0], 1, ck, s))
@@ -1627,8 +1637,10 @@ extern "C" int tess2_set_option(tess2_ctx *c, int option, int value)
         return c->blocks.size() > 1 ? build_chunks(c) : 0;
     case TESS2_OPT_CELL_KERNEL:
         if (value < -1 || value > 4) return fail(c, TESS2_E_ARG, "cell kernel: -1..4");
-        if (value != c->cell_kernel) c->gen++;   // a recorded graph is recorded again
+        // a recorded graph is recorded again
+        if (value != c->cell_kernel || c->ck_tuned) c->gen++;
         c->cell_kernel = value;
+        c->ck_tuned = false;
         return 0;
     case TESS2_OPT_PLANE_TILES:
         if (value < 1 || value > PLANE_TILES)
@@ -1687,7 +1699,10 @@ extern "C" int tess2_autotune(tess2_ctx *c, int reps, float *best_ms)
     if (reps < 1 || reps > 100) return fail(c, TESS2_E_ARG, "reps: 1..100");
     HIPCHK(c, hipSetDevice(c->device));
     float best = 0.0f;
-    int r = time_runs(c, 1, &best);   // warm-up (and capture, in graph mode)
+    int r = 0;
+    // an earlier choice is made again
+    if (c->ck_tuned && (r = tess2_set_option(c, TESS2_OPT_CELL_KERNEL, -1))) return r;
+    r = time_runs(c, 1, &best);   // warm-up (and capture, in graph mode)
     if (r) return r;
     r = time_runs(c, reps, &best);
     if (r) return r;
@@ -1698,11 +1713,18 @@ extern "C" int tess2_autotune(tess2_ctx *c, int reps, float *best_ms)
         // geometry and scan kernels timed above
         static const int chunks[][3] = {{8, 16, 32}, {16, 32, 64}, {32, 64, 128}, {64, 128, 256}};
         static const int waves[] = {8, 16, 24, 32};
-        const bool any = c->cell_kernel == -1;
+        // (CIC, and the exact assignment without volumes, take no cell kernel)
+        const bool any = c->cell_kernel == -1 && c->last.alg == TESS2_DENSE_TESS &&
+                         (c->last.assignment == TESS2_ASSIGN_REFERENCE_SCAN || c->last.want_vol);
         int bk = c->cell_kernel;
         int bc[3] = {c->chunk_small, c->chunk_medium, c->chunk_large}, bw = c->waves_per_cu;
         float bsplit = any ? INFINITY : best;
-        if (any && (r = tess2_set_option(c, TESS2_OPT_CELL_KERNEL, 3))) return r;
+        auto choose = [&](int k) {
+            const int e = tess2_set_option(c, TESS2_OPT_CELL_KERNEL, k);
+            c->ck_tuned = k >= 0;
+            return e;
+        };
+        if (any && (r = choose(3))) return r;
         for (const auto &ch : chunks)
             for (int w : waves) {
                 if ((r = tess2_set_option(c, TESS2_OPT_CHUNK_SMALL, ch[0])) ||
@@ -1732,15 +1754,14 @@ extern "C" int tess2_autotune(tess2_ctx *c, int reps, float *best_ms)
         if (any) {
             for (int k : {1, 4}) {
                 float t = 0.0f;
-                if ((r = tess2_set_option(c, TESS2_OPT_CELL_KERNEL, k)) ||
-                    (r = time_runs(c, 1, &t)) || (r = time_runs(c, reps, &t)))
+                if ((r = choose(k)) || (r = time_runs(c, 1, &t)) || (r = time_runs(c, reps, &t)))
                     return r;
                 if (t < best) {
                     best = t;
                     bk = k;
                 }
             }
-            if ((r = tess2_set_option(c, TESS2_OPT_CELL_KERNEL, bk))) return r;
+            if ((r = choose(bk))) return r;
         }
         float t = 0.0f;
         if ((r = time_runs(c, 1, &t))) return r;   // leave the results of the chosen split
@@ -1848,7 +1869,7 @@ extern "C" int tess2_volumes(tess2_ctx *c, const tess2_block_t *block, float *ou
     BlockIn in = make_in(d);
     CellOut o = make_out(d, true);
     GridP gp{};
-    launch_volumes(c, in, o, s);
+    launch_volumes(asked_kernel(c, 1), in, o, s);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipMemcpyAsync(d.hm->ctrs, d.ctrs, sizeof(unsigned) * C_NCTR, hipMemcpyDeviceToHost,
                              s));
@@ -1930,7 +1951,7 @@ extern "C" int tess2_volumes_noalloc(tess2_ctx *c, const float *particles, int n
     o.slow = reinterpret_cast<int *>(base + o_sl);
     o.slow_cap = (unsigned)norig;
     o.ncells = norig;
-    launch_volumes(c, in, o, s);
+    launch_volumes(asked_kernel(c, 1), in, o, s);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipMemcpyAsync(c->h_noalloc, ctrs, sizeof(unsigned) * (C_NCTR + 1),
                              hipMemcpyDeviceToHost, s));

@@ -33,6 +33,8 @@ long n_bad;                               // launches with a buffer missing or t
 std::map<int, long> n_launch;
 std::map<int, double> cost;
 double now = 0.0;                         // the stream's clock
+double drift = 1.0;                       // each launch costs so much of the one before
+double speed = 1.0;
 bool capturing = false;
 double graph_ms = 0.0;
 
@@ -57,7 +59,8 @@ void launch(int kind)
 {
     std::lock_guard<std::mutex> lk(mu);
     ++n_launch[kind];
-    (capturing ? graph_ms : now) += cost.count(kind) ? cost[kind] : 0.001;
+    (capturing ? graph_ms : now) += (cost.count(kind) ? cost[kind] : 0.001) * speed;
+    speed *= drift;
 }
 
 // whether p has room for so many bytes; counted when not
@@ -87,11 +90,13 @@ void fake_reset()
     n_malloc = n_copy = n_graph = n_sync = n_slot_copy = n_bad = 0;
     n_launch.clear();
     cost.clear();
+    drift = speed = 1.0;
 }
 void fake_limit(size_t bytes) { limit = bytes == ~size_t(0) ? bytes : used + bytes; }
 void fake_fail_copy(long n) { fail_copy = n; }
 void fake_fail_new(long n) { fail_new = n; }
 void fake_cost(int kind, double ms) { cost[kind] = ms; }
+void fake_drift(double f) { drift = f; }
 long fake_pending() { return (long)pending.size(); }
 long fake_launches(int kind) { return n_launch[kind]; }
 long fake_copies() { return n_copy; }
@@ -280,7 +285,12 @@ void launch_owner(const GridP &gp, const HashP &, const unsigned *, const float4
 void launch_exact_tail(const BlockIn &, const GridP &, const int *, const int *, const CellOut &,
                        int, int *const *, const int *const *, const Router *, int, int,
                        hipStream_t) { launch(K_OTHER); }
-void launch_fill_u32(unsigned *, size_t, unsigned, hipStream_t) { launch(K_OTHER); }
+void launch_fill_u32(unsigned *p, size_t n, unsigned v, hipStream_t)
+{
+    launch(K_OTHER);
+    need(p, 4 * n);
+    std::fill(p, p + n, v);
+}
 void launch_ghost_sends(const float4 *, const int4 *, int, int, const float *, const float *,
                         const float *, int, int, unsigned long long *, hipStream_t) { launch(K_OTHER); }
 void launch_device_block(const float *, int, const int4 *, int, const int *, float4 *, float4 *,
@@ -302,7 +312,10 @@ void launch_run_prep(const BlockIn *, const CellOut *outs, int nb, int, unsigned
         for (int k = 0; k < 3; ++k) need(o.fold[k], 16 * (size_t)o.fold_cap[k]);
     }
     for (int k = 0; k < 4; ++k)
-        if (z.n[k]) need(z.p[k], 4 * z.n[k]);
+        if (z.n[k]) {
+            need(z.p[k], 4 * z.n[k]);
+            std::fill(z.p[k], z.p[k] + z.n[k], 0u);
+        }
 }
 void launch_cells_ref(const BlockIn &, const GridP &, const CellOut &, int, hipStream_t)
 {

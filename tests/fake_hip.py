@@ -17,6 +17,7 @@ CONTROL = {
     "fake_fail_copy": (None, [C.c_long]),        # copies until one fails
     "fake_fail_new": (None, [C.c_long]),         # allocations until operator new throws
     "fake_cost": (None, [C.c_int, C.c_double]),  # ms per launch of a kind
+    "fake_drift": (None, [C.c_double]),          # cost of a launch in terms of the one before
     "fake_pending": (C.c_long, []),              # uploads from pageable memory not waited for
     "fake_launches": (C.c_long, [C.c_int]),
     "fake_copies": (C.c_long, []),

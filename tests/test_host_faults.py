@@ -256,3 +256,72 @@ def test_fetching_leaves_the_next_run_its_descriptors(fake, graph, nb):
         _runs(run)
         assert fake.fake_copies() - before == steady
     assert fake.fake_graphs() == graphs
+
+
+# ---- the tuned cell kernel --------------------------------------------------
+KERNELS = {3: F.K_REF_BATCHED, 1: F.K_MC_BATCHED, 4: F.K_MC_ITEMS, -1: F.K_GEOM}
+
+
+def _used(fake, run, **kw):
+    before = {k: fake.fake_launches(k) for k in range(8)}
+    run.run((9, 9, 9), **kw)
+    run.sync()
+    return {k for k in range(1, 8) if fake.fake_launches(k) > before[k]}
+
+
+@pytest.mark.parametrize("best", [3, 1, 4, -1])
+def test_tuned_kernel_is_for_several_blocks(fake, best):
+    """What tess2_autotune chooses for several blocks is neither the choice for
+    a single block staged later nor the end of the choice."""
+    for k in KERNELS.values():
+        fake.fake_cost(k, 1.0)
+    fake.fake_cost(KERNELS[best], 0.01)
+    run = D.StagedRun([_block(300, 1, 0), _block(200, 2, 1)])
+    _runs(run)
+    run.autotune(reps=1)
+    assert run.get_option("cell_kernel") == best
+    assert KERNELS[best] in _used(fake, run, want_volumes=False)
+    # one block: the geometry and scan kernels, and the automatic volumes
+    big, few = _block(20000), _block(300)
+    assert _stage(run.ctx, [big])[0] == 0
+    run.blocks = [big]
+    assert _used(fake, run, want_volumes=False) == {F.K_GEOM, F.K_SCAN}
+    D.volumes(few, ctx=run.ctx)
+    assert _stage(run.ctx, [few])[0] == 0
+    run.blocks = [few]
+    assert _used(fake, run, want_volumes=False) == {F.K_MC}
+    # another set of blocks is tuned over all kernels again
+    blocks = [_block(100, 1, 0), _block(900, 2, 1)]
+    assert _stage(run.ctx, blocks)[0] == 0
+    run.blocks = blocks
+    _runs(run)
+    for now, k in KERNELS.items():
+        fake.fake_cost(k, 0.01 if now == 4 else 1.0)
+    run.autotune(reps=1)
+    assert run.get_option("cell_kernel") == 4
+
+
+def test_asked_kernel_stays(fake):
+    run = D.StagedRun([_block(300, 1, 0), _block(200, 2, 1)])
+    run.set_option("cell_kernel", 1)
+    _runs(run)
+    run.autotune(reps=1)
+    assert run.get_option("cell_kernel") == 1
+    few = _block(20000)
+    assert _stage(run.ctx, [few])[0] == 0
+    run.blocks = [few]
+    assert _used(fake, run, want_volumes=False) == {F.K_MC}
+
+
+def test_runs_without_cell_kernels_choose_none(fake):
+    """The time of a CIC run says nothing about the cell kernels."""
+    run = D.StagedRun([_block(300, 1, 0), _block(200, 2, 1)])
+    fake.fake_cost(F.K_OTHER, 1.0)
+    fake.fake_drift(0.999)              # every candidate looks faster than the one before
+    for kw in (dict(alg=D.DENSE_CIC), dict(assignment=D.EXACT_VORONOI, want_volumes=False)):
+        run.run((9, 9, 9), **kw)
+        run.sync()
+        before = sum(fake.fake_launches(k) for k in range(1, 8))
+        run.autotune(reps=1)
+        assert run.get_option("cell_kernel") == -1
+        assert sum(fake.fake_launches(k) for k in range(1, 8)) == before
