@@ -14,6 +14,7 @@
 #include "kernels.hpp"
 #include "geom.hpp"
 #include "deposit.hpp"
+#include "owner_tiles.hpp"
 
 #include <algorithm>
 
@@ -151,15 +152,17 @@ __device__ int nearest_f64(float gx, float gy, float gz, const HashP &h,
 }
 
 // ---------------------------------------------------------------------------
-// The nearest sites of the 64 points of a tile at once: the wave takes the
-// buckets around the tile's box shell by shell, and every lane meets every
-// particle of a bucket.  The particles are wave-uniform (scalar loads, no
-// per-lane runs), a row of buckets farther from the box than the largest best
-// distance of the lanes is skipped, and nothing diverges.  A lane by itself
-// sees 27 buckets where the tile sees up to 64, but its wave runs the longest
-// of 64 different row sequences, and in a cluster's core it cannot skip the
-// full buckets around its own: 262k particles on 192^3 0.48 -> 0.29 ms, 8 Plummer
-// blocks on 128^3 6.4 -> 1.06, 262k on 63^3 (a tile spans three buckets)
+// The nearest sites of the P points of a tile at once: the wave takes the
+// buckets around the tile's box shell by shell.  With P = 64 every lane meets
+// every particle of a bucket; with 8 points or one (grids coarser than the
+// particles, owner_tile) the 64 / P lanes of a point take a run's particles in
+// turn and compare what they found at the end.  With P = 64 the particles are
+// wave-uniform (scalar loads, no per-lane runs), a row of buckets farther from
+// the box than the largest best distance of the lanes is skipped, and nothing
+// diverges.  A lane by itself sees 27 buckets where the tile sees up to 64, but
+// its wave runs the longest of 64 different row sequences, and in a cluster's
+// core it cannot skip the full buckets around its own: 262k particles on 192^3
+// 0.48 -> 0.29 ms, 8 Plummer blocks on 128^3 6.4 -> 1.06, 262k on 63^3
 // 0.108 -> 0.067.  Vector issue bounds it: 13 instructions per particle met.
 // ---------------------------------------------------------------------------
 struct Tile {
@@ -185,7 +188,7 @@ template <class T> __device__ __forceinline__ T wave_max(T x)
 // point, all lanes together, until no unvisited one can be: reach() is the
 // wave's largest squared distance still to beat (infinite before the first
 // particle), widened by the caller's rounding margin.
-template <class Visit, class Reach>
+template <int P, class Visit, class Reach>
 __device__ __forceinline__ void tile_search(const Tile &t, const HashP &h,
                                             const unsigned *__restrict__ start,
                                             const float4 *__restrict__ hp, Visit visit,
@@ -209,16 +212,17 @@ __device__ __forceinline__ void tile_search(const Tile &t, const HashP &h,
         hi[a] = uniform_f(t.hi[a] - h.lo[a]);
     }
     auto gap = [&](int i, int a) { return bucket_gap(lo[a], hi[a], i, h); };
+    constexpr unsigned L = 64 / P;   // lanes per point: each meets its share of a run
     auto run = [&](unsigned s0, unsigned s1) {
-        unsigned s = s0;
-        for (; s + 4 <= s1; s += 4) {
-            const float4 p0 = hp[s], p1 = hp[s + 1], p2 = hp[s + 2], p3 = hp[s + 3];
+        unsigned s = s0 + (L > 1 ? (unsigned)lane / P : 0u);
+        for (; s + 3 * L < s1; s += 4 * L) {
+            const float4 p0 = hp[s], p1 = hp[s + L], p2 = hp[s + 2 * L], p3 = hp[s + 3 * L];
             visit(p0);
             visit(p1);
             visit(p2);
             visit(p3);
         }
-        for (; s < s1; ++s) visit(hp[s]);
+        for (; s < s1; s += L) visit(hp[s]);
     };
     const int rmax = h.dims[0] + h.dims[1] + h.dims[2];
     double m2 = INFINITY;
@@ -277,7 +281,9 @@ __device__ __forceinline__ void tile_search(const Tile &t, const HashP &h,
     }
 }
 
-// on: this lane has a point (the others see the same particles and are ignored)
+// on: this lane has a point (the others see the same particles and are
+// ignored); the 64 / P lanes of a point end with the same answer
+template <int P>
 __device__ __forceinline__ int tile_nearest_f32(float gx, float gy, float gz, bool on,
                                                 const Tile &t, const HashP &h,
                                                 const unsigned *__restrict__ start,
@@ -285,7 +291,7 @@ __device__ __forceinline__ int tile_nearest_f32(float gx, float gy, float gz, bo
 {
     float best = INFINITY, second = INFINITY;
     int bid = -1;
-    tile_search(
+    tile_search<P>(
         t, h, start, hp,
         [&](const float4 p) {
             const float ex = gx - p.x, ey = gy - p.y, ez = gz - p.z;
@@ -294,7 +300,18 @@ __device__ __forceinline__ int tile_nearest_f32(float gx, float gy, float gz, bo
             bid = d < best ? __float_as_int(p.w) : bid;
             best = fminf(best, d);
         },
-        [&] { return wave_max(on ? best * 1.0001f + 1e-30f : 0.0f); });
+        [&] {
+            float b = best;
+            for (int off = P; off < 64; off <<= 1) b = fminf(b, __shfl_xor(b, off));
+            return wave_max(on ? b * 1.0001f + 1e-30f : 0.0f);
+        });
+    for (int off = P; off < 64; off <<= 1) {
+        const float ob = __shfl_xor(best, off), os = __shfl_xor(second, off);
+        const int oid = __shfl_xor(bid, off);
+        second = fminf(fminf(second, os), fmaxf(best, ob));
+        bid = ob < best ? oid : bid;   // of two equal ones neither stands
+        best = fminf(best, ob);
+    }
     // decided only if the runner-up is clearly farther (32 ulp window) and
     // nothing underflowed, or the point coincides with a site: exact in float
     const float tau = 32.0f * 5.9604645e-8f;
@@ -303,6 +320,7 @@ __device__ __forceinline__ int tile_nearest_f32(float gx, float gy, float gz, bo
     return -1;
 }
 
+template <int P>
 __device__ __forceinline__ int tile_nearest_f64(float gx, float gy, float gz, bool on,
                                                 const Tile &t, const HashP &h,
                                                 const unsigned *__restrict__ start,
@@ -310,30 +328,38 @@ __device__ __forceinline__ int tile_nearest_f64(float gx, float gy, float gz, bo
 {
     double best = 1e300;
     int bid = 0x7fffffff;
-    tile_search(
+    auto meet = [&](double d, int id) {
+        const bool b = better64(d, id, best, bid);
+        best = b ? d : best;
+        bid = b ? id : bid;
+    };
+    tile_search<P>(
         t, h, start, hp,
         [&](const float4 p) {
             const double ex = (double)gx - (double)p.x;
             const double ey = (double)gy - (double)p.y;
             const double ez = (double)gz - (double)p.z;
-            const double d = ex * ex + ey * ey + ez * ez;
-            const int id = __float_as_int(p.w);
-            const bool b = better64(d, id, best, bid);
-            best = b ? d : best;
-            bid = b ? id : bid;
+            meet(ex * ex + ey * ey + ez * ez, __float_as_int(p.w));
         },
-        [&] { return wave_max(on ? best * (1.0 + 1e-9) + 1e-300 : 0.0); });
+        [&] {
+            double b = best;
+            for (int off = P; off < 64; off <<= 1) b = fmin(b, __shfl_xor(b, off));
+            return wave_max(on ? b * (1.0 + 1e-9) + 1e-300 : 0.0);
+        });
+    for (int off = P; off < 64; off <<= 1)
+        meet(__shfl_xor(best, off), __shfl_xor(bid, off));
     return bid;
 }
 
-// one thread per block grid point; a 64-lane wave covers a 4x4x4 tile
+// a wave per tile of P block grid points (owner_tile), 64 / P lanes per point.
 // With several blocks the owner is a home key (rank << 23 | cell) and the
 // counts go to the home block's cell (npts_tab / stex_tab by rank).
+template <int P>
 __global__ __launch_bounds__(256) void k_owner(GridP gp, HashP h,
                                                const unsigned *__restrict__ start,
                                                const float4 *__restrict__ hp, int *__restrict__ owner,
-                                               int prec, unsigned *ctrs, int tiles_x, int tiles_y,
-                                               int ntiles, const int *__restrict__ status,
+                                               int prec, unsigned *ctrs, OwnerTile ot, int tiles_x,
+                                               int tiles_y, int ntiles, const int *__restrict__ status,
                                                int *__restrict__ npts, int ncells,
                                                int *const *__restrict__ npts_tab,
                                                const int *const *__restrict__ stex_tab,
@@ -341,13 +367,17 @@ __global__ __launch_bounds__(256) void k_owner(GridP gp, HashP h,
 {
     const int wave = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (wave >= ntiles) return;
-    const int lane = threadIdx.x & 63;
+    const int lane = threadIdx.x & 63, pt = lane & (P - 1);
     const int tx = wave % tiles_x, ty = (wave / tiles_x) % tiles_y, tz = wave / (tiles_x * tiles_y);
-    const int lx0 = tx * 4 + (lane & 3), ly0 = ty * 4 + ((lane >> 2) & 3), lz0 = tz * 4 + (lane >> 4);
+    const int g0[3] = {tx << ot.bits[0], ty << ot.bits[1], tz << ot.bits[2]};
+    const int lx0 = g0[0] + (pt & ((1 << ot.bits[0]) - 1)),
+              ly0 = g0[1] + ((pt >> ot.bits[0]) & ((1 << ot.bits[1]) - 1)),
+              lz0 = g0[2] + (pt >> (ot.bits[0] + ot.bits[1]));
     const bool on_grid = lx0 < gp.bnum_idx[0] && ly0 < gp.bnum_idx[1] && lz0 < gp.bnum_idx[2];
+    const bool mine = on_grid && lane < P;   // the point's lane that writes and counts
     // off-grid lanes of an edge tile stand in for an on-grid point of the
     // tile but write nothing and count nothing
-    const int lx = on_grid ? lx0 : tx * 4, ly = on_grid ? ly0 : ty * 4, lz = on_grid ? lz0 : tz * 4;
+    const int lx = on_grid ? lx0 : g0[0], ly = on_grid ? ly0 : g0[1], lz = on_grid ? lz0 : g0[2];
     const long long lidx = ((long long)lz * gp.bnum_idx[1] + ly) * gp.bnum_idx[0] + lx;
     const int gx = gp.bmin_idx[0] + lx, gy = gp.bmin_idx[1] + ly, gz = gp.bmin_idx[2] + lz;
     const float px = idx2phys1(gx, gp.step[0], gp.gmin[0]);
@@ -355,23 +385,22 @@ __global__ __launch_bounds__(256) void k_owner(GridP gp, HashP h,
     const float pz = idx2phys1(gz, gp.step[2], gp.gmin[2]);
     const bool in_block = px >= gp.bmin[0] && px <= gp.bmax[0] && py >= gp.bmin[1] &&
                           py <= gp.bmax[1] && pz >= gp.bmin[2] && pz <= gp.bmax[2];
-    if (!in_block && on_grid) owner[lidx] = -1;
+    if (!in_block && mine) owner[lidx] = -1;
     int o = -1;
     bool failed = false;
     const bool on = in_block && on_grid;
     if (__ballot(on)) {
         Tile t;
-        const int g0[3] = {tx * 4, ty * 4, tz * 4};
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
             t.lo[a] = uniform_f(idx2phys1(gp.bmin_idx[a] + g0[a], gp.step[a], gp.gmin[a]));
-            t.hi[a] = uniform_f(idx2phys1(gp.bmin_idx[a] + min(g0[a] + 3, gp.bnum_idx[a] - 1),
-                                          gp.step[a], gp.gmin[a]));
+            const int last = min(g0[a] + (1 << ot.bits[a]) - 1, gp.bnum_idx[a] - 1);
+            t.hi[a] = uniform_f(idx2phys1(gp.bmin_idx[a] + last, gp.step[a], gp.gmin[a]));
         }
-        if (prec == 0) o = tile_nearest_f32(px, py, pz, on, t, h, start, hp);
-        else o = tile_nearest_f64(px, py, pz, on, t, h, start, hp);
-        if (!on) o = -1;
-        failed = on && o < 0 && prec == 0;
+        if (prec == 0) o = tile_nearest_f32<P>(px, py, pz, on, t, h, start, hp);
+        else o = tile_nearest_f64<P>(px, py, pz, on, t, h, start, hp);
+        if (!on || !mine) o = -1;
+        failed = on && mine && o < 0 && prec == 0;
     }
     // FP32 filter failures go to a queue that k_owner_deferred searches in
     // FP64 with full waves: searched here, one failing lane would hold its
@@ -390,7 +419,7 @@ __global__ __launch_bounds__(256) void k_owner(GridP gp, HashP h,
             defer = true;
         }
     }
-    if (in_block && on_grid) {
+    if (in_block && mine) {
         if (o < 0 && !defer) o = nearest_f64(px, py, pz, h, start, hp);
         owner[lidx] = o;           // -1 for a deferred point until its FP64 search
     }
@@ -399,7 +428,7 @@ __global__ __launch_bounds__(256) void k_owner(GridP gp, HashP h,
     const int hc = npts_tab ? (o & 0x7fffff) : o;
     const int *hst = npts_tab && o >= 0 ? stex_tab[o >> 23] : status;
     int *hnp = npts_tab && o >= 0 ? npts_tab[o >> 23] : npts;
-    const bool cnt = on_grid && in_block && o >= 0 && (npts_tab || o < ncells) &&
+    const bool cnt = mine && in_block && o >= 0 && (npts_tab || o < ncells) &&
                      hst[hc] == EX_DEPOSIT;
     unsigned long long pend = __ballot(cnt);
     while (pend) {
@@ -449,13 +478,17 @@ void launch_owner(const GridP &gp, const HashP &h, const unsigned *start, const 
                   int *const *npts_tab, const int *const *stex_tab, unsigned *defq,
                   unsigned defq_cap, hipStream_t s)
 {
-    const int tx = (gp.bnum_idx[0] + 3) / 4, ty = (gp.bnum_idx[1] + 3) / 4,
-              tz = (gp.bnum_idx[2] + 3) / 4;
-    const int ntiles = tx * ty * tz;
+    double step[3];
+    for (int a = 0; a < 3; ++a) step[a] = (double)gp.step[a] * (double)h.inv;
+    const OwnerTile ot = owner_tile(gp.bnum_idx, step);
+    int n[3];
+    for (int a = 0; a < 3; ++a) n[a] = ((gp.bnum_idx[a] - 1) >> ot.bits[a]) + 1;
+    const int ntiles = n[0] * n[1] * n[2];
     if (ntiles <= 0) return;
-    hipLaunchKernelGGL(k_owner, dim3((ntiles + 3) / 4), dim3(256),
-                       0, s, gp, h, start, hp, owner, prec, ctrs, tx, ty, ntiles, status, npts,
-                       ncells, npts_tab, stex_tab, defq, prec == 0 ? defq_cap : 0u);
+    hipLaunchKernelGGL(
+        (ot.points == 64 ? k_owner<64> : (ot.points == 8 ? k_owner<8> : k_owner<1>)),
+        dim3((ntiles + 3) / 4), dim3(256), 0, s, gp, h, start, hp, owner, prec, ctrs, ot, n[0], n[1],
+        ntiles, status, npts, ncells, npts_tab, stex_tab, defq, prec == 0 ? defq_cap : 0u);
     if (prec == 0 && defq_cap > 0) {
         const unsigned nblk = defq_cap / 256 + 1;
         hipLaunchKernelGGL(k_owner_deferred, dim3(nblk < 2048 ? nblk : 2048), dim3(256), 0, s,
