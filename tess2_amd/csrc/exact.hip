@@ -115,6 +115,7 @@ __device__ int nearest_f64(float gx, float gy, float gz, const HashP &h,
 {
     int c[3];
     home_bucket(gx, gy, gz, h, c);
+    const float rel[3] = {gx - h.lo[0], gy - h.lo[1], gz - h.lo[2]};
     double best = 1e300;
     int bid = 0x7fffffff;
     const int rmax = h.dims[0] + h.dims[1] + h.dims[2];
@@ -143,10 +144,15 @@ __device__ int nearest_f64(float gx, float gy, float gz, const HashP &h,
                 }
             }
         }
+        if (bid == 0x7fffffff) continue;
         // every bucket beyond shell r is at least r cells away, less what the
         // float bucket arithmetic can be off
         const double lb = fmax(0.0, (double)r - (double)h.slack) * (double)h.cell;
-        if (bid != 0x7fffffff && r > 0 && lb * lb > best * (1.0 + 1e-9) + 1e-300) break;
+        if (r > 0 && lb * lb > best * (1.0 + 1e-9) + 1e-300) break;
+        // most end above (this bound's squares are floats: a few ulp more)
+        if (r > 1 &&
+            (double)beyond_shell2(r, c, c, rel, rel, h) > best * (1.0 + 2e-6) + 1e-300)
+            break;
     }
     return bid;
 }
@@ -188,7 +194,7 @@ template <class T> __device__ __forceinline__ T wave_max(T x)
 // point, all lanes together, until no unvisited one can be: reach() is the
 // wave's largest squared distance still to beat (infinite before the first
 // particle), widened by the caller's rounding margin.
-template <int P, class Visit, class Reach>
+template <int P, bool OUT, class Visit, class Reach>
 __device__ __forceinline__ void tile_search(const Tile &t, const HashP &h,
                                             const unsigned *__restrict__ start,
                                             const float4 *__restrict__ hp, Visit visit,
@@ -275,15 +281,19 @@ __device__ __forceinline__ void tile_search(const Tile &t, const HashP &h,
         }
         // the squared gaps are floats: a few ulp more
         m2 = (double)reach() * (1.0 + 2e-6);
-        // every bucket beyond shell r is at least r cells from the box
-        const double lb = fmax(0.0, (double)r - (double)h.slack) * (double)h.cell;
-        if (r > 0 && lb * lb > m2) break;
+        if (OUT) {
+            if ((double)beyond_shell2(r, c0, c1, lo, hi, h) > m2) break;
+        } else {
+            // every bucket beyond shell r is at least r cells from the box
+            const double lb = fmax(0.0, (double)r - (double)h.slack) * (double)h.cell;
+            if (r > 0 && lb * lb > m2) break;
+        }
     }
 }
 
 // on: this lane has a point (the others see the same particles and are
 // ignored); the 64 / P lanes of a point end with the same answer
-template <int P>
+template <int P, bool OUT>
 __device__ __forceinline__ int tile_nearest_f32(float gx, float gy, float gz, bool on,
                                                 const Tile &t, const HashP &h,
                                                 const unsigned *__restrict__ start,
@@ -291,7 +301,7 @@ __device__ __forceinline__ int tile_nearest_f32(float gx, float gy, float gz, bo
 {
     float best = INFINITY, second = INFINITY;
     int bid = -1;
-    tile_search<P>(
+    tile_search<P, OUT>(
         t, h, start, hp,
         [&](const float4 p) {
             const float ex = gx - p.x, ey = gy - p.y, ez = gz - p.z;
@@ -320,7 +330,7 @@ __device__ __forceinline__ int tile_nearest_f32(float gx, float gy, float gz, bo
     return -1;
 }
 
-template <int P>
+template <int P, bool OUT>
 __device__ __forceinline__ int tile_nearest_f64(float gx, float gy, float gz, bool on,
                                                 const Tile &t, const HashP &h,
                                                 const unsigned *__restrict__ start,
@@ -333,7 +343,7 @@ __device__ __forceinline__ int tile_nearest_f64(float gx, float gy, float gz, bo
         best = b ? d : best;
         bid = b ? id : bid;
     };
-    tile_search<P>(
+    tile_search<P, OUT>(
         t, h, start, hp,
         [&](const float4 p) {
             const double ex = (double)gx - (double)p.x;
@@ -354,7 +364,7 @@ __device__ __forceinline__ int tile_nearest_f64(float gx, float gy, float gz, bo
 // a wave per tile of P block grid points (owner_tile), 64 / P lanes per point.
 // With several blocks the owner is a home key (rank << 23 | cell) and the
 // counts go to the home block's cell (npts_tab / stex_tab by rank).
-template <int P>
+template <int P, bool OUT>
 __global__ __launch_bounds__(256) void k_owner(GridP gp, HashP h,
                                                const unsigned *__restrict__ start,
                                                const float4 *__restrict__ hp, int *__restrict__ owner,
@@ -397,8 +407,8 @@ __global__ __launch_bounds__(256) void k_owner(GridP gp, HashP h,
             const int last = min(g0[a] + (1 << ot.bits[a]) - 1, gp.bnum_idx[a] - 1);
             t.hi[a] = uniform_f(idx2phys1(gp.bmin_idx[a] + last, gp.step[a], gp.gmin[a]));
         }
-        if (prec == 0) o = tile_nearest_f32<P>(px, py, pz, on, t, h, start, hp);
-        else o = tile_nearest_f64<P>(px, py, pz, on, t, h, start, hp);
+        if (prec == 0) o = tile_nearest_f32<P, OUT>(px, py, pz, on, t, h, start, hp);
+        else o = tile_nearest_f64<P, OUT>(px, py, pz, on, t, h, start, hp);
         if (!on || !mine) o = -1;
         failed = on && mine && o < 0 && prec == 0;
     }
@@ -485,10 +495,21 @@ void launch_owner(const GridP &gp, const HashP &h, const unsigned *start, const 
     for (int a = 0; a < 3; ++a) n[a] = ((gp.bnum_idx[a] - 1) >> ot.bits[a]) + 1;
     const int ntiles = n[0] * n[1] * n[2];
     if (ntiles <= 0) return;
-    hipLaunchKernelGGL(
-        (ot.points == 64 ? k_owner<64> : (ot.points == 8 ? k_owner<8> : k_owner<1>)),
-        dim3((ntiles + 3) / 4), dim3(256), 0, s, gp, h, start, hp, owner, prec, ctrs, ot, n[0], n[1],
-        ntiles, status, npts, ncells, npts_tab, stex_tab, defq, prec == 0 ? defq_cap : 0u);
+    // a grid that leaves the particles' box by more than a bucket
+    bool out = false;
+    for (int a = 0; a < 3; ++a) {
+        const float g0 = idx2phys1(gp.bmin_idx[a], gp.step[a], gp.gmin[a]);
+        const float g1 = idx2phys1(gp.bmin_idx[a] + gp.bnum_idx[a] - 1, gp.step[a], gp.gmin[a]);
+        out |= g0 < h.lo[a] - h.cell || g1 > h.lo[a] + (float)(h.dims[a] + 1) * h.cell;
+    }
+    auto *kernel = out ? (ot.points == 64 ? k_owner<64, true>
+                                          : (ot.points == 8 ? k_owner<8, true> : k_owner<1, true>))
+                       : (ot.points == 64 ? k_owner<64, false>
+                                          : (ot.points == 8 ? k_owner<8, false>
+                                                            : k_owner<1, false>));
+    hipLaunchKernelGGL(kernel, dim3((ntiles + 3) / 4), dim3(256), 0, s, gp, h, start, hp, owner,
+                       prec, ctrs, ot, n[0], n[1], ntiles, status, npts, ncells, npts_tab, stex_tab,
+                       defq, prec == 0 ? defq_cap : 0u);
     if (prec == 0 && defq_cap > 0) {
         const unsigned nblk = defq_cap / 256 + 1;
         hipLaunchKernelGGL(k_owner_deferred, dim3(nblk < 2048 ? nblk : 2048), dim3(256), 0, s,
