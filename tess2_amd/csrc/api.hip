@@ -227,7 +227,10 @@ static int cell_kernel_for(int asked, int ncells, unsigned long long ngrid)
 // us): 4000 cells on 23^3 115 against 108, on 32^3 120 against 103, on 48^3 172
 // against 136; 10000 on 31^3 120 and 121, on 65^3 198 against 162; 16000 on
 // 25^3 145 against 196, on 50^3 146 and 150, on 76^3 213 against 202, on 101^3
-// 308 against 600; 262k on 128^3 610 against 950.
+// 308 against 600; 262k on 128^3 610 against 950.  (A run of one block on fewer
+// than 64 grid points is bound by the atomics on those, which the one-pass
+// kernel has under way beside its geometry: 200,000 cells on 3^3 4605 against
+// 4418, on 4^3 2328 against 3261.)
 static bool split_cells(int asked, float eps, int nb, int ncells)
 {
     return asked < 0 && eps >= 0.0f && (nb > 1 || ncells >= 16384);
@@ -1224,7 +1227,8 @@ static int prepare_run(tess2_ctx *c, const RunArgs &a)
         c->h_outs[k] = make_out(d, a.want_vol != 0);
     }
     c->split = a.alg == TESS2_DENSE_TESS && !exact &&
-               split_cells(asked_kernel(c, nb), a.eps, nb, c->blocks[0].norig) && ensure_planes(c, run_tiles(c));
+               split_cells(asked_kernel(c, nb), a.eps, nb, c->blocks[0].norig) &&
+               (nb > 1 || c->blocks[0].ngrid >= 64) && ensure_planes(c, run_tiles(c));
     if (c->desc_gen == c->gen && same_args(a, c->desc_args)) return 0;   // unchanged
     if (nb > 1) {
         // XCD ranges of the item list by estimated cost: a cell, plus its

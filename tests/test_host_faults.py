@@ -325,3 +325,12 @@ def test_runs_without_cell_kernels_choose_none(fake):
         run.autotune(reps=1)
         assert run.get_option("cell_kernel") == -1
         assert sum(fake.fake_launches(k) for k in range(1, 8)) == before
+
+
+def test_few_grid_points_take_the_one_pass_kernel(fake):
+    one, two = D.StagedRun([_block(20000)]), D.StagedRun([_block(300, 1, 0), _block(200, 2, 1)])
+    for run, split in ((one, False), (two, True)):
+        for g in ((3, 3, 3), (4, 4, 4), (2, 2, 16)):
+            before = fake.fake_launches(F.K_SCAN)
+            _runs(run, g)
+            assert (fake.fake_launches(F.K_SCAN) > before) == (split or g != (3, 3, 3))
