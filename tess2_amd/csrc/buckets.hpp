@@ -37,9 +37,8 @@ __host__ __device__ __forceinline__ float bucket_slack(int most_buckets)
 // unit box is 1.7e-5).
 __host__ __device__ __forceinline__ float bucket_gap(float a, float b, int i, const HashP &h)
 {
-    const float left = (float)i * h.cell, right = (float)(i + 1) * h.cell;
-    const float d = fmaxf(0.0f, fmaxf(left - b, a - right)) - h.slack * h.cell;
-    return fmaxf(0.0f, d);
+    const float left = (float)i * h.cell, right = left + h.cell;
+    return fmaxf(0.0f, fmaxf(left - b, a - right) - h.slack * h.cell);
 }
 
 // Squared distance from the box [lo, hi] (relative to the origin, in buckets c0
