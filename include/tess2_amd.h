@@ -271,10 +271,10 @@ enum {
     TESS2_OPT_CHUNK_MEDIUM = 3,   /* cells per work item, blocks with < 100000 cells */
     TESS2_OPT_CHUNK_LARGE = 4,    /* cells per work item, larger blocks */
     TESS2_OPT_CELL_KERNEL = 5,    /* cell kernel: -1 (default) chosen per run (several blocks,
-                                   * or 16384 cells and more: a geometry kernel and a scan
-                                   * kernel over all cells; else 1, or 2 when cell boxes are
-                                   * not small, 6 or more grid points per cell); 0 one cell
-                                   * per wave; 1 two cells per wave in the star / face / ring
+                                   * or 16384 cells and more on 64 grid points and more: a
+                                   * geometry kernel and a scan kernel over all cells; else
+                                   * 1, or 2 when cell boxes are not small, 6 or more grid
+                                   * points per cell); 0 one cell per wave; 1 two cells per wave in the star / face / ring
                                    * phase; 2 the same with the verdict masks of boxes up
                                    * to 512 points (several blocks: 1 and 2 both run the
                                    * two-cell persistent kernel with those masks); 3 one
