@@ -274,15 +274,16 @@ enum {
                                    * or 16384 cells and more on 64 grid points and more: a
                                    * geometry kernel and a scan kernel over all cells; else
                                    * 1, or 2 when cell boxes are not small, 6 or more grid
-                                   * points per cell); 0 one cell per wave; 1 two cells per wave in the star / face / ring
-                                   * phase; 2 the same with the verdict masks of boxes up
-                                   * to 512 points (several blocks: 1 and 2 both run the
-                                   * two-cell persistent kernel with those masks); 3 one
-                                   * cell per wave with the star search's record loads
-                                   * issued before its table work (several blocks only;
-                                   * one block runs 0); 4 several blocks in one launch
-                                   * without the work queue, a workgroup per two cells,
-                                   * two cells per wave as 2 (one block runs 2);
+                                   * points per cell); 0 one cell per wave; 1 two cells
+                                   * per wave in the star / face / ring phase; 2 the same
+                                   * with the verdict masks of boxes up to 512 points
+                                   * (several blocks: 1 and 2 both run the two-cell
+                                   * persistent kernel with those masks); 3 one cell per
+                                   * wave with the star search's record loads issued before
+                                   * its table work (several blocks only; one block runs
+                                   * 0); 4 several blocks in one launch without the work
+                                   * queue, a workgroup per two cells, two cells per wave
+                                   * as 2 (one block runs 2);
                                    * with the option at -1, tess2_autotune also times
                                    * 3, 1 and 4 and keeps the fastest */
     TESS2_OPT_PLANE_TILES = 6     /* tiles of 64 cells whose face planes are in memory at a
