@@ -490,7 +490,7 @@ void launch_owner(const GridP &gp, const HashP &h, const unsigned *start, const 
 {
     double step[3];
     for (int a = 0; a < 3; ++a) step[a] = (double)gp.step[a] * (double)h.inv;
-    const OwnerTile ot = owner_tile(gp.bnum_idx, step);
+    const OwnerTile ot = owner_tile(gp.bnum_idx, step, h.dims);
     int n[3];
     for (int a = 0; a < 3; ++a) n[a] = ((gp.bnum_idx[a] - 1) >> ot.bits[a]) + 1;
     const int ntiles = n[0] * n[1] * n[2];

@@ -13,15 +13,18 @@ struct OwnerTile {
 };
 
 // particles that a wave meets, at one a bucket: the tile's box, and the
-// buckets about it that the nearest sites of its points can lie in
-inline double tile_meets(const OwnerTile &t, const double step[3])
+// buckets about it that the nearest sites of its points can lie in, at most all
+inline double tile_meets(const OwnerTile &t, const double step[3], const int buckets[3])
 {
-    double m = 1.0;
-    for (int a = 0; a < 3; ++a) m *= ((1 << t.bits[a]) - 1) * step[a] + 2.5;
-    return m;
+    double m = 1.0, all = 1.0;
+    for (int a = 0; a < 3; ++a) {
+        m *= ((1 << t.bits[a]) - 1) * step[a] + 2.5;
+        all *= buckets[a];
+    }
+    return std::min(m, all);
 }
 
-// dims: grid points; step: their distance in buckets.
+// dims: grid points; step: their distance in buckets; buckets: of the hash.
 //
 // A wave on 64 points loads every particle once for all of them, but where the
 // grid is coarser than the particles it meets all particles of its box one
@@ -34,10 +37,12 @@ inline double tile_meets(const OwnerTile &t, const double step[3])
 // 65^3 69, 111 and 441; a lane per point took 57, 93 and 111).  The edges double
 // on the axis where that keeps the box shortest (200,000 on 300 x 300 x 9: 4 x
 // 4 x 4 points 205 us, a lane per point 145, 8 x 8 x 1 points 87).
-inline OwnerTile owner_tile(const int dims[3], const double step[3])
+// Particles in a small part of the grid are few to meet (1,000 in a hundredth of
+// its edge on 257^3: 8.2 ms with 64 points, 30 with 8, 88 with one).
+inline OwnerTile owner_tile(const int dims[3], const double step[3], const int buckets[3])
 {
     static const struct { int points; double chain, met, wave, issue; } fit[3] = {
-        {64, 20.0, 0.14, 1.5e-3, 5e-5}, {8, 17.0, 0.07, 0.5e-3, 5e-5}, {1, 15.0, 0.0, 1.5e-3, 0.0}};
+        {64, 20.0, 0.14, 1.5e-3, 5e-5}, {8, 17.0, 0.07, 0.5e-3, 5e-5}, {1, 15.0, 0.0, 1.8e-3, 0.0}};
     OwnerTile best{}, t{};
     double least = 0.0;
     for (int k = 2; k >= 0; --k) {
@@ -57,13 +62,14 @@ inline OwnerTile owner_tile(const int dims[3], const double step[3])
         }
         double waves = 1.0;
         for (int a = 0; a < 3; ++a) waves *= ((dims[a] - 1) >> t.bits[a]) + 1;
-        const double m = tile_meets(t, step);
+        const double m = tile_meets(t, step, buckets);
         const double us = fit[k].chain + fit[k].met * m + waves * (fit[k].wave + fit[k].issue * m);
         // at most 400 particles in a row, as many as were measured (a clustered
-        // block holds many times the mean in some tiles); tiles are counted in
-        // an int
-        if (k == 2 || (us < least && m * fit[k].points / 64.0 <= 400.0) ||
-            waves * fit[k].points >= 2e9) {
+        // block holds many times the mean in some tiles), unless there are no
+        // more; tiles are counted in an int
+        const bool few = m * fit[k].points / 64.0 <= 400.0 ||
+                         m >= (double)buckets[0] * buckets[1] * buckets[2];
+        if (k == 2 || (us < least && few) || waves * fit[k].points >= 2e9) {
             least = us;
             best = t;
         }

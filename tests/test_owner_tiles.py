@@ -18,14 +18,14 @@ HARNESS = r"""
 using namespace t2;
 
 static int bad = 0;
-static void check(const int d[3], const double s[3])
+static void check(const int d[3], const double s[3], const int b[3])
 {
-    const OwnerTile t = owner_tile(d, s);
+    const OwnerTile t = owner_tile(d, s, b);
     const int bits = t.bits[0] + t.bits[1] + t.bits[2];
     double tiles = 1.0;
     for (int a = 0; a < 3; ++a) tiles *= ((d[a] - 1) >> t.bits[a]) + 1;
     // particles one lane meets in a row
-    const double row = tile_meets(t, s) * t.points / 64.0;
+    const double row = tile_meets(t, s, b) * t.points / 64.0;
     if ((1 << bits) != t.points || (t.points != 64 && t.points != 8 && t.points != 1) ||
         tiles > 2147483000.0 || row > 400.0) {
         ++bad;
@@ -48,17 +48,24 @@ int main()
                                          side / (z > 1 ? z - 1 : 1)};
                     // grids of points as dense as the memory of a few runs
                     if ((double)x * y * z * 64.0 < particles && x < 9 && particles > 1e8) continue;
-                    check(d, s);
+                    const int b[3] = {(int)side + 1, (int)side + 1, (int)side + 1};
+                    check(d, s, b);
                 }
     const int huge[3] = {2000, 2000, 2000};
     const double coarse[3] = {30.0, 30.0, 30.0};
-    const OwnerTile t = owner_tile(huge, coarse);     // 8e9 points
+    const int many[3] = {60000, 60000, 60000};
+    const OwnerTile t = owner_tile(huge, coarse, many);     // 8e9 points
     if (t.points != 64) ++bad;
     // a fine grid keeps 64 points a wave, in a cube
     const int fine[3] = {192, 192, 192};
     const double f[3] = {0.33, 0.33, 0.33};
-    const OwnerTile c = owner_tile(fine, f);
+    const int side[3] = {64, 64, 64};
+    const OwnerTile c = owner_tile(fine, f, side);
     if (c.points != 64 || c.bits[0] != 2 || c.bits[1] != 2 || c.bits[2] != 2) ++bad;
+    // and so does one whose particles all lie in a small part of it
+    const int wide[3] = {257, 257, 257}, ten[3] = {11, 11, 11};
+    const double w[3] = {3.9, 3.9, 3.9};
+    if (owner_tile(wide, w, ten).points != 64) ++bad;
     return bad;
 }
 """
