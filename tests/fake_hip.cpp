@@ -27,7 +27,7 @@ struct Pending { const char *host; size_t bytes; };
 std::vector<Pending> pending;             // pageable sources not waited for
 
 // counters, by name in fake_count
-long n_malloc, n_copy, n_graph, n_sync, n_slot_copy;
+long n_malloc, n_copy, n_graph, n_sync, n_slot_copy, n_async_down;
 long n_bad;                               // launches with a buffer missing or too small
 // launches: number and cost (ms) by kind
 std::map<int, long> n_launch;
@@ -87,7 +87,7 @@ void fake_reset()
     fail_new = -1;
     last_error = hipSuccess;
     pending.clear();
-    n_malloc = n_copy = n_graph = n_sync = n_slot_copy = n_bad = 0;
+    n_malloc = n_copy = n_graph = n_sync = n_slot_copy = n_async_down = n_bad = 0;
     n_launch.clear();
     cost.clear();
     drift = speed = 1.0;
@@ -103,6 +103,7 @@ long fake_copies() { return n_copy; }
 long fake_pinned_copies() { return n_slot_copy; }
 long fake_graphs() { return n_graph; }
 long fake_mallocs() { return n_malloc; }
+long fake_async_downloads() { return n_async_down; }
 long fake_bad_launches() { return n_bad; }
 void *fake_pinned(size_t bytes)
 {
@@ -178,8 +179,23 @@ hipError_t hipMemcpyAsync(void *dst, const void *src, size_t n, hipMemcpyKind ki
     const void *host = kind == hipMemcpyHostToDevice ? src : dst;
     if (in(pinned, host)) ++n_slot_copy;
     else if (kind == hipMemcpyHostToDevice) pending.push_back({(const char *)src, n});
+    else ++n_async_down;
     std::memmove(dst, src, n);
     return hipSuccess;
+}
+hipError_t hipMemcpy(void *dst, const void *src, size_t n, hipMemcpyKind kind)
+{
+    return hipMemcpyWithStream(dst, src, n, kind, nullptr);
+}
+hipError_t hipMemcpyWithStream(void *dst, const void *src, size_t n, hipMemcpyKind, hipStream_t s)
+{
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        ++n_copy;
+        if (fail_copy >= 0 && fail_copy-- == 0) return ret(hipErrorUnknown);
+        std::memmove(dst, src, n);
+    }
+    return hipStreamSynchronize(s);
 }
 hipError_t hipStreamSynchronize(hipStream_t)
 {

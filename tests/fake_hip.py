@@ -24,6 +24,7 @@ CONTROL = {
     "fake_pinned_copies": (C.c_long, []),
     "fake_graphs": (C.c_long, []),
     "fake_mallocs": (C.c_long, []),
+    "fake_async_downloads": (C.c_long, []),      # to pageable memory
     "fake_bad_launches": (C.c_long, []),         # with a buffer missing or too small
     "fake_pinned": (C.c_void_p, [C.c_size_t]),
 }

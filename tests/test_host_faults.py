@@ -334,3 +334,16 @@ def test_few_grid_points_take_the_one_pass_kernel(fake):
             before = fake.fake_launches(F.K_SCAN)
             _runs(run, g)
             assert (fake.fake_launches(F.K_SCAN) > before) == (split or g != (3, 3, 3))
+
+
+def test_small_results_come_in_one_waiting_copy(fake):
+    """An asynchronous copy of up to 16 KB to pageable memory and a wait behind
+    it take the runtime twice as long as a copy that waits."""
+    run = D.StagedRun([_block(500)])
+    _runs(run)
+    before = fake.fake_copies()
+    run.cells(0)
+    run.fetch(0, volumes=False)
+    run.fetch(0, ngrid=False, circumcenters=True)
+    assert fake.fake_copies() == before + 4
+    assert fake.fake_async_downloads() == 0
